@@ -339,6 +339,25 @@ __device__ __forceinline__ float pair_max(float x) {
   return fmaxf(a, b);
 }
 
+// Two values summed over lanes l and l ^ M (M = 16 or 32), one to each lane of the pair: a's sum to
+// the lane with bit M clear, b's to the other. One exchange and one add.
+template <int M>
+__device__ __forceinline__ float swap_sum(float a, float b) {
+  static_assert(M == 16 || M == 32, "pairs lanes 16 or 32 apart");
+  const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
+  uint32_t x, y;
+  if constexpr (M == 16) {
+    const auto p = __builtin_amdgcn_permlane16_swap(ua, ub, false, false);
+    x = p[0];
+    y = p[1];
+  } else {
+    const auto p = __builtin_amdgcn_permlane32_swap(ua, ub, false, false);
+    x = p[0];
+    y = p[1];
+  }
+  return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+}
+
 // ---- whole-wave integer scans and reductions without LDS traffic ------------------------------
 template <int CTRL, int ROWS = 0xF>
 __device__ __forceinline__ uint32_t dpp_u32(uint32_t x) {  // rows outside ROWS read 0

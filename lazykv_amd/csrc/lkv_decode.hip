@@ -896,6 +896,54 @@ __device__ __forceinline__ void attend_hybrid_piped(const DecodeArgs& a, const i
   }
 }
 
+// A wave's o totals over its RG row groups, into the wave's LDS rows [G][D]. Each step pairs lanes of
+// two row groups and halves what a lane holds: the lane keeps one half of the values, added to its
+// partner's, and the partner the other half. permlane16_swap(a, b) and permlane32_swap(a, b) hand out
+// both halves at once: the pair's even lane gets both lanes' a, its odd lane both lanes' b. G * EPL = 32
+// values take 56 adds and exchanges on 8-lane rows, where a full sum of every value in every lane took
+// about 330 instructions; the tail of a launch that attends one pair a wave is mostly this sum.
+// The pairs are those of groups_sum, in its order, so the totals are the same bits.
+template <int D, int G>
+__device__ __forceinline__ void scatter_totals(const float (&o)[G][Lanes<D>::EPL], int lane, float* rows) {
+  using L = Lanes<D>;
+  constexpr int EPL = L::EPL, RG = L::RG;
+  constexpr int N0 = G * EPL;
+  constexpr int N1 = RG == 8 ? N0 / 2 : N0;  // values left after the 8-lane rows' own step
+  constexpr int M = N0 / RG;
+  static_assert(M >= 1 && N1 >= 4, "at least one value per lane");
+  float v[N1];
+  const bool odd8 = (lane & 8) != 0;
+#pragma unroll
+  for (int i = 0; i < N1; ++i) {
+    if constexpr (RG == 8) {
+      const float a = o[i / EPL][i % EPL], b = o[(i + N1) / EPL][(i + N1) % EPL];
+      const float keep = odd8 ? b : a, give = odd8 ? a : b;
+      v[i] = keep + lkv::dpp<lkv::kDppRowRor8>(give);
+    } else {
+      v[i] = o[i / EPL][i % EPL];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < N1 / 2; ++i) v[i] = lkv::swap_sum<16>(v[i], v[i + N1 / 2]);
+#pragma unroll
+  for (int i = 0; i < N1 / 4; ++i) v[i] = lkv::swap_sum<32>(v[i], v[i + N1 / 4]);
+  // The lane's M values are o's flattened [j][e] positions x0 .. x0 + M - 1.
+  const int x0 = (RG == 8 && odd8 ? N1 : 0) + ((lane & 16) ? N1 / 2 : 0) + ((lane & 32) ? N1 / 4 : 0);
+  float* at = rows + (lane % L::LPR) * EPL;
+  constexpr int V = M < 4 ? M : 4;
+#pragma unroll
+  for (int i = 0; i < M; i += V) {
+    float* p = at + (x0 + i) / EPL * D + (x0 + i) % EPL;
+    if constexpr (V == 4) {
+      *(float4*)p = make_float4(v[i], v[i + 1], v[i + 2], v[i + 3]);
+    } else if constexpr (V == 2) {
+      *(float2*)p = make_float2(v[i], v[i + 1]);
+    } else {
+      *p = v[i];
+    }
+  }
+}
+
 // Candidates a fused-selection workgroup holds (KPT keys per thread): SEL * kSelUnit per KV head.
 // SEL 1 holds 2,048 (a 32,768-token context at 16-token blocks), SEL 2 holds 4,096, SEL 4 holds
 // 8,192; a launch takes the smallest that fits, since every key slot a thread holds costs its
@@ -922,7 +970,7 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
   const int S = a.splits_a + a.splits_b;
 
   __shared__ float s_m[NW][G], s_l[NW][G];
-  __shared__ float s_o[NW][G][D];
+  __shared__ __align__(16) float s_o[NW][G][D];
   __shared__ uint32_t s_excl[64];  // segment B: bitmap of excluded blocks in this run
   static_assert(!MF || (!I8 && MT != LKV_F32), "the matrix-core path reads model-dtype pairs");
   __shared__ float s_pb[MF ? NW : 1][MF ? kMfBroadcast<G, kMfMaxPairs> : 1];
@@ -1108,17 +1156,12 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
 #pragma unroll
   for (int j = 0; j < G; ++j) {
     const float l = lkv::groups_sum<L::RG>(st.l[j]);
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) st.o[j][e] = lkv::groups_sum<L::RG>(st.o[j][e]);
     if (lane == 0) {
       s_m[wave][j] = st.m[j];
       s_l[wave][j] = l;
     }
-    if (r == 0) {
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) s_o[wave][j][c * EPL + e] = st.o[j][e];
-    }
   }
+  scatter_totals<D, G>(st.o, lane, &s_o[wave][0][0]);
   __syncthreads();
   float* pml = a.part_ml + ((int64_t)h * S + split) * G * 2;
   float* po = a.part_o + ((int64_t)h * S + split) * G * D;
