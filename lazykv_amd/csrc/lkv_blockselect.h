@@ -3,17 +3,20 @@
 //
 // The rule is lkv_bound_topk's: the k candidates with the highest bound, ties at the threshold
 // taken towards the lower candidate index, reported in ascending index order. Each thread holds a
-// contiguous run of up to KPT candidates as order-preserving integer keys. The k-th largest key is
-// found by range-adaptive radix select: a pass histograms the live key range into at most 2048
-// bins scaled to that range and keeps the bin holding the k-th key. When that bin's keys are all
-// taken the selection is complete; when it holds at most NT keys they are ranked directly (one
-// thread each) instead of another pass. Three passes narrow any 32-bit range to one value, so the
-// loop is capped at four.
+// contiguous run of up to KPT candidates as order-preserving integer keys. The k-th best candidate
+// (key, index) is found by range-adaptive radix select: a pass histograms the live key range into at
+// most 2048 bins scaled to that range and keeps the bin holding the k-th key. When that bin's keys are
+// all taken the selection is complete; when it holds at most 64 keys every wave ranks them for itself,
+// one lane each, with the keys handed round by v_readlane. Three passes narrow any 32-bit range to one
+// value, so the loop is capped at four.
 //
-// Each phase is one LDS round trip and one barrier: a thread owns kSelBins / NT consecutive bins
-// and reads them in one vector load, and the boundary bin is found in registers. (On MI355X an LDS
-// atomic to a random bin costs about one lane per clock when lanes collide on banks, so a key
-// takes part in a pass only while it lies in the live range.)
+// What bounds it is the chain of phases, not bytes: each is one LDS round trip and one barrier, 0.2 to
+// 1.4 us in a decode launch of 512 threads. So
+//   - the first range starts at the least of the threads' own largest keys (second largest) when there
+//     are at least k (k / 2) of them: that many keys lie above it. With k of 512 threads that leaves
+//     about a third of the keys to the histogram, whose LDS atomics to random bins are its cost;
+//   - the ranking of the boundary bin gives the k-th candidate itself, (key, index), and a thread then
+//     takes every key above one threshold: no bitmap, no second barrier, two instructions a key.
 #pragma once
 
 #include "lkv_common.h"
@@ -22,6 +25,7 @@ namespace lkv {
 
 constexpr int kSelBins = 2048;
 constexpr int kSelPasses = 4;
+constexpr int kSelRank = 64;  // a boundary bin of up to this many keys is ranked, a lane each
 
 __device__ __forceinline__ uint32_t orderable_key(float f) {
   const uint32_t u = __float_as_uint(f);
@@ -31,15 +35,13 @@ __device__ __forceinline__ uint32_t orderable_key(float f) {
 template <int NT, int KPT>
 struct SelectLds {
   static constexpr int kWaves = NT / 64;
-  static constexpr int kCap = NT * KPT;          // candidates one workgroup can hold
   static constexpr int kBpt = kSelBins / NT;     // bins a thread owns
   static_assert(kBpt == 2 || kBpt == 4 || kBpt == 8, "256, 512 or 1024 threads");
   alignas(16) uint32_t hist[kSelBins];
-  uint32_t list_key[NT];
-  uint32_t list_id[NT];
-  uint32_t taken[kCap / 32];  // boundary-bin keys ranked among the best, one bit per candidate
+  uint32_t list_key[kSelRank];  // the boundary bin's keys and candidate indices, in any order
+  uint32_t list_id[kSelRank];
   uint32_t mm[2 * kWaves];
-  uint32_t scan[2][kWaves];
+  uint32_t scan[3][kWaves];
   uint32_t info[4];  // boundary bin, keys above it, keys in it, boundary-list length
 };
 
@@ -129,23 +131,34 @@ __device__ __forceinline__ SelectPick block_top_k(const float* __restrict__ boun
 #pragma unroll
     for (int u = 0; u < KPT; ++u) key[u] = u < nlive ? orderable_key(bound_h[i0 + u]) : 0u;
   }
-  uint32_t live = 0u;  // bit u: slot u holds a candidate
-#pragma unroll
-  for (int u = 0; u < KPT; ++u) live |= (u < nlive ? 1u : 0u) << u;
-  // While the loads are in flight: clear the bitmap and this thread's bins for the first pass.
-  for (int i = threadIdx.x; i < SelectLds<NT, KPT>::kCap / 32; i += NT) L.taken[i] = 0u;
+  const uint32_t live = nlive >= 32 ? 0xffffffffu : (1u << nlive) - 1u;  // bit u: slot u holds a candidate
+  // While the loads are in flight: this thread's bins for the first pass.
   clear_bins<kBpt>(L.hist + threadIdx.x * kBpt);
-  uint32_t lmin = 0xffffffffu, lmax = 0u;
+  // This thread's largest and second largest key (0 for slots without a candidate).
+  uint32_t m1 = 0u, m2 = 0u;
 #pragma unroll
   for (int u = 0; u < KPT; ++u) {
-    lmin = min(lmin, ((live >> u) & 1u) ? key[u] : 0xffffffffu);
-    lmax = max(lmax, ((live >> u) & 1u) ? key[u] : 0u);
+    const uint32_t x = u < nlive ? key[u] : 0u;
+    m2 = max(m2, min(m1, x));
+    m1 = max(m1, x);
   }
-  lmin = wave_min_u32(lmin);
-  lmax = wave_max_u32(lmax);
+  // A value that at least k keys reach: each of the nth threads with a key holds one of at least its m1,
+  // each of the nth2 threads with two keys another of at least its m2. Beyond 2 * nth2, the least key.
+  const int nth = (n + npt - 1) / npt, nth2 = nth - (n % npt == 1 ? 1 : 0);
+  uint32_t low = 0xffffffffu;
+  if (k <= nth) {  // workgroup-uniform, as below
+    if (nlive > 0) low = m1;
+  } else if (k <= 2 * nth2) {
+    if (nlive > 1) low = m2;
+  } else {
+#pragma unroll
+    for (int u = 0; u < KPT; ++u) low = min(low, u < nlive ? key[u] : 0xffffffffu);
+  }
+  low = wave_min_u32(low);
+  m1 = wave_max_u32(m1);
   if (lane == 0) {
-    L.mm[2 * wave] = lmin;
-    L.mm[2 * wave + 1] = lmax;
+    L.mm[2 * wave] = low;
+    L.mm[2 * wave + 1] = m1;
   }
   __syncthreads();
   uint32_t lo = L.mm[0], hi = L.mm[1];
@@ -155,12 +168,11 @@ __device__ __forceinline__ SelectPick block_top_k(const float* __restrict__ boun
     hi = max(hi, L.mm[2 * w + 1]);
   }
 
-  // After the loop: every key above hi is taken, and of the keys in [lo, hi] either all
-  // (whole), the marked ones (ranked), or -- when lo == hi, or the pass cap was reached -- the
-  // first `need` keys equal to lo in index order.
-  int need = k;
-  bool whole = false, ranked = false;
-  uint32_t marked = 0u;  // bit u: key[u] was ranked among the boundary bin's best
+  // The k-th best candidate: taken are the keys above tk, and those equal to it up to index tid.
+  uint32_t tk = lo;
+  int tid = -1;
+  bool found = false;
+  int need = k;  // still to take from [lo, hi]; every key above hi is taken
 #pragma unroll 1
   for (int pass = 0; pass < kSelPasses; ++pass) {
     if (lo >= hi) break;
@@ -173,7 +185,7 @@ __device__ __forceinline__ SelectPick block_top_k(const float* __restrict__ boun
     }
 #pragma unroll
     for (int u = 0; u < KPT; ++u)
-      if (((live >> u) & 1u) && key[u] >= lo && key[u] <= hi) atomicAdd(&L.hist[(key[u] - lo) >> shift], 1u);
+      if (u < nlive && key[u] >= lo && key[u] <= hi) atomicAdd(&L.hist[(key[u] - lo) >> shift], 1u);
     __syncthreads();
     uint32_t cnt[kBpt];
     read_bins<kBpt>(L.hist + threadIdx.x * kBpt, cnt);
@@ -204,66 +216,71 @@ __device__ __forceinline__ SelectPick block_top_k(const float* __restrict__ boun
     const uint32_t span = shift ? ((1u << shift) - 1u) : 0u;
     hi = min(hi, new_lo + span);
     lo = new_lo;
+    tk = lo;
     if (in_bin == (uint32_t)need) {  // the boundary bin is taken whole
-      whole = true;
+      tid = 0x7fffffff;
+      found = true;
       break;
     }
-    if (lo < hi && in_bin <= (uint32_t)NT) {
-      // Few keys in the boundary bin: rank them directly by (key desc, index asc) and mark the
-      // `need` best in the bitmap, which each thread reads back for its own run.
+    if (lo < hi && in_bin <= (uint32_t)kSelRank) {
 #pragma unroll
       for (int u = 0; u < KPT; ++u) {
-        if (((live >> u) & 1u) && key[u] >= lo && key[u] <= hi) {
+        if (u < nlive && key[u] >= lo && key[u] <= hi) {
           const uint32_t slot = atomicAdd(&L.info[3], 1u);
           L.list_key[slot] = key[u];
           L.list_id[slot] = (uint32_t)(i0 + u);
         }
       }
       __syncthreads();
-      const int m = (int)L.info[3];
-      if ((int)threadIdx.x < m) {
-        const uint32_t mk = L.list_key[threadIdx.x], mi = L.list_id[threadIdx.x];
-        int rank = 0;
-        for (int e = 0; e < m; ++e) {
-          const uint32_t ek = L.list_key[e], ei = L.list_id[e];
-          rank += (ek > mk) | ((ek == mk) & (ei < mi));
-        }
-        if (rank < need) atomicOr(&L.taken[mi >> 5], 1u << (mi & 31));
+      // Lane e ranks entry e by (key desc, index asc); the entry of rank need - 1 is the k-th best.
+      const int m = __builtin_amdgcn_readfirstlane((int)in_bin);
+      const uint32_t ek = lane < m ? L.list_key[lane] : 0u, ei = lane < m ? L.list_id[lane] : 0xffffffffu;
+      int rank = 0;
+      for (int e = 0; e < m; ++e) {
+        const uint32_t sk = (uint32_t)__builtin_amdgcn_readlane((int)ek, e), si = (uint32_t)__builtin_amdgcn_readlane((int)ei, e);
+        rank += (sk > ek) | ((sk == ek) & (si < ei));
       }
-      __syncthreads();
-      // A run [i0, i0 + npt) spans at most two bitmap words.
-      const uint32_t w0 = L.taken[i0 >> 5];
-      const uint32_t w1 = ((i0 >> 5) + 1) < SelectLds<NT, KPT>::kCap / 32 ? L.taken[(i0 >> 5) + 1] : 0u;
-      const uint64_t both = ((uint64_t)w1 << 32) | w0;
-      marked = (uint32_t)(both >> (i0 & 31)) & (npt >= 32 ? 0xffffffffu : ((1u << npt) - 1u));
-      ranked = true;
+      const uint64_t at = __ballot(lane < m && rank == need - 1);
+      const int src = at != 0 ? __ffsll((unsigned long long)at) - 1 : 0;
+      tk = (uint32_t)__builtin_amdgcn_readlane((int)ek, src);
+      tid = __builtin_amdgcn_readlane((int)ei, src);
+      found = true;
       break;
     }
   }
-
-  // Per thread, the slots taken outright and the ties (equal to lo, unmarked, in tie mode).
-  const bool tie_mode = !whole && !ranked;
-  uint32_t above_m = 0u, tie_m = 0u;
+  if (!found) {
+    // Every key left equals tk: the first `need` of them in index order are taken, so tid is the
+    // index of the need-th.
+    uint32_t tie_m = 0u;
 #pragma unroll
-  for (int u = 0; u < KPT; ++u) {
-    const uint32_t lv = (live >> u) & 1u;
-    const uint32_t out = (key[u] > hi ? 1u : 0u) | (whole && key[u] >= lo ? 1u : 0u) | (ranked ? (marked >> u) & 1u : 0u);
-    above_m |= (lv & out) << u;
-    tie_m |= (lv & (tie_mode && key[u] == lo ? 1u : 0u)) << u;
+    for (int u = 0; u < KPT; ++u) tie_m |= (u < nlive && key[u] == tk ? 1u : 0u) << u;
+    uint32_t tot;
+    const int before = (int)workgroup_exclusive_sum<NT, SCALAR_WAVE>(__popc(tie_m), L.scan[2], &tot);
+    if (before < need && need <= before + (int)__popc(tie_m)) {
+      for (int t = before + 1; t < need; ++t) tie_m &= tie_m - 1u;  // drop the ties before it
+      L.info[0] = (uint32_t)(i0 + __ffs((int)tie_m) - 1);
+    }
+    __syncthreads();
+    tid = (int)L.info[0];
   }
-  if (!tie_mode) need = 0;
-  const uint32_t gt = __popc(above_m), eq = __popc(tie_m);
-  uint32_t tot;
-  const uint32_t packed = workgroup_exclusive_sum<NT, SCALAR_WAVE>((eq << 16) | gt, L.scan[1], &tot);
-  const int eq_before = (int)(packed >> 16), gt_before = (int)(packed & 0xffffu);
-  int take_eq = need - eq_before;
-  take_eq = take_eq < 0 ? 0 : (take_eq > (int)eq ? (int)eq : take_eq);
-  // Ties are taken in index order: this thread's first take_eq ties.
-  uint32_t ties = tie_m;
-  for (int t = (int)eq; t > take_eq; --t) ties &= ~(0x80000000u >> __clz(ties));  // drop the highest
+
+  // A thread whose run ends by tid takes its keys from tk up, one whose run starts behind it those
+  // above tk; only the run that tid cuts looks at indices.
+  const bool after = i0 > tid;
+  const bool cut = !after && i0 + npt - 1 > tid;
+  const uint32_t thr = after ? tk + 1u : tk;
   SelectPick p;
-  p.take = above_m | ties;
-  p.pos = gt_before + min(eq_before, need);
+  p.take = 0u;
+#pragma unroll
+  for (int u = 0; u < KPT; ++u) p.take |= (key[u] >= thr ? 1u : 0u) << u;
+  p.take &= (after && tk == 0xffffffffu) ? 0u : live;
+  if (cut) {
+#pragma unroll
+    for (int u = 0; u < KPT; ++u)
+      if (key[u] == tk && i0 + u > tid) p.take &= ~(1u << u);
+  }
+  uint32_t tot;
+  p.pos = (int)workgroup_exclusive_sum<NT, SCALAR_WAVE>(__popc(p.take), L.scan[1], &tot);
   p.i0 = i0;
   return p;
 }

@@ -1006,15 +1006,15 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
     const int je = min(last, has_sink + a.k) - has_sink;
     int32_t* ids = (int32_t*)s_sel.hist;
     int32_t* out_h = (a.idx_out != nullptr && split == 0) ? a.idx_out + (int64_t)h * a.idx_out_stride : nullptr;
+    // Most threads' few picks lie outside this workgroup's run.
     int pos = pk.pos;
-#pragma unroll
-    for (int u = 0; u < kSelKpt<NT, SEL>; ++u) {
-      if ((pk.take >> u) & 1u) {
-        const int32_t id = pk.i0 + u + a.cand_offset;
-        if (pos >= js && pos < je) ids[pos - js] = id;
-        if (out_h != nullptr && pos < a.k) out_h[pos] = id;
-        ++pos;
-      }
+    uint32_t take = (out_h != nullptr || (pos < je && pos + __popc(pk.take) > js)) ? pk.take : 0u;
+    while (take != 0u) {
+      const int32_t id = pk.i0 + __ffs((int)take) - 1 + a.cand_offset;
+      if (pos >= js && pos < je) ids[pos - js] = id;
+      if (out_h != nullptr && pos < a.k) out_h[pos] = id;
+      ++pos;
+      take &= take - 1u;
     }
     __syncthreads();
     idx_h = ids;
@@ -1627,16 +1627,10 @@ __global__ __launch_bounds__(kResThreads) void residency_kernel(const int32_t* _
     const lkv::SelectPick pk = lkv::block_top_k<kResThreads, kResSelKpt, true>(rs.bounds + (int64_t)h * rs.bound_stride, rs.aligned != 0, rs.n_cand, k, s_sel);
     int32_t* ids_h = rs.ids + (int64_t)h * rs.ids_stride;
     int pos = pk.pos;
-#pragma unroll
-    for (int u = 0; u < kResSelKpt; ++u) {
-      if ((pk.take >> u) & 1u) {
-        const int32_t id = pk.i0 + u + rs.cand_offset;
-        if (pos < k) {
-          s_ids[pos] = id;
-          ids_h[pos] = id;
-        }
-        ++pos;
-      }
+    for (uint32_t take = pk.take; take != 0u && pos < k; take &= take - 1u, ++pos) {
+      const int32_t id = pk.i0 + __ffs((int)take) - 1 + rs.cand_offset;
+      s_ids[pos] = id;
+      ids_h[pos] = id;
     }
     __syncthreads();
   }

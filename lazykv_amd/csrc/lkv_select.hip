@@ -568,13 +568,7 @@ __global__ __launch_bounds__(kSelBlockThreads) void select_block_kernel(const fl
   const lkv::SelectPick pk = lkv::block_top_k<kSelBlockThreads, kSelBlockKpt, true>(bounds + (int64_t)h * bstride, true, n_cand, k, L);
   int32_t* out_h = out_idx + (int64_t)h * idx_stride;
   int pos = pk.pos;
-#pragma unroll
-  for (int u = 0; u < kSelBlockKpt; ++u) {
-    if ((pk.take >> u) & 1u) {
-      if (pos < k) out_h[pos] = pk.i0 + u + cand_offset;
-      ++pos;
-    }
-  }
+  for (uint32_t take = pk.take; take != 0u && pos < k; take &= take - 1u, ++pos) out_h[pos] = pk.i0 + __ffs((int)take) - 1 + cand_offset;
 }
 
 // Rows the in-workgroup top-K may read as 16-byte vectors: aligned, and padded to 4 floats.
