@@ -261,12 +261,12 @@ def _pmc_file() -> dict:
 def step_kernels(fused: bool, in_decode: bool, n_cand: int) -> str:
     """One layer's launches, as rocprof names them, by the library's dispatch rules: the matrix-core
     bound for a model-dtype query with aligned rows; the top K inside the decode launch when the
-    fused call selects there, else select_block_kernel up to 8,192 candidates, select_kernel up to
-    12,288 and select_stream_kernel beyond."""
+    fused call selects there, else select_block_kernel up to 12,288 candidates and
+    select_stream_kernel beyond."""
     call = "one lkv_select_decode call: " if fused else "lkv_bound_topk + lkv_sparse_decode: "
     if fused and in_decode:
         return call + "bound_kernel_mf, sparse_decode_kernel choosing the top K itself, decode_merge_wave_kernel"
-    sel = "select_block_kernel" if n_cand <= 8192 else ("select_kernel" if n_cand <= 12288 else "select_stream_kernel")
+    sel = "select_block_kernel" if n_cand <= 12288 else "select_stream_kernel"
     return call + f"bound_kernel_mf, {sel}, sparse_decode_kernel, decode_merge_wave_kernel"
 
 

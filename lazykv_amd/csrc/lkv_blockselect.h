@@ -27,10 +27,8 @@ constexpr int kSelBins = 2048;
 constexpr int kSelPasses = 4;
 constexpr int kSelRank = 64;  // a boundary bin of up to this many keys is ranked, a lane each
 
-__device__ __forceinline__ uint32_t orderable_key(float f) {
-  const uint32_t u = __float_as_uint(f);
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
+__device__ __forceinline__ uint32_t orderable_bits(uint32_t u) { return (u & 0x80000000u) ? ~u : (u | 0x80000000u); }
+__device__ __forceinline__ uint32_t orderable_key(float f) { return orderable_bits(__float_as_uint(f)); }
 
 template <int NT, int KPT>
 struct SelectLds {
@@ -102,6 +100,23 @@ __device__ __forceinline__ void clear_bins(uint32_t* p) {
 #pragma unroll
     for (int i = 0; i < B; i += 4) *(uint4*)(p + i) = make_uint4(0u, 0u, 0u, 0u);
   }
+}
+
+// The need-th best of the m <= kSelRank listed candidates by (key desc, index asc), found by every wave
+// for itself: lane e ranks entry e, the entries handed round by v_readlane.
+__device__ __forceinline__ void rank_boundary(const uint32_t* list_key, const uint32_t* list_id, int m_, int need, int lane, uint32_t* tk,
+                                              int* tid) {
+  const int m = __builtin_amdgcn_readfirstlane(m_);
+  const uint32_t ek = lane < m ? list_key[lane] : 0u, ei = lane < m ? list_id[lane] : 0xffffffffu;
+  int rank = 0;
+  for (int e = 0; e < m; ++e) {
+    const uint32_t sk = (uint32_t)__builtin_amdgcn_readlane((int)ek, e), si = (uint32_t)__builtin_amdgcn_readlane((int)ei, e);
+    rank += (sk > ek) | ((sk == ek) & (si < ei));
+  }
+  const uint64_t at = __ballot(lane < m && rank == need - 1);
+  const int src = at != 0 ? __ffsll((unsigned long long)at) - 1 : 0;
+  *tk = (uint32_t)__builtin_amdgcn_readlane((int)ek, src);
+  *tid = __builtin_amdgcn_readlane((int)ei, src);
 }
 
 // Select k of the n bounds at `bound_h` (n <= NT * KPT; the row is readable in whole 16-byte
@@ -232,18 +247,7 @@ __device__ __forceinline__ SelectPick block_top_k(const float* __restrict__ boun
         }
       }
       __syncthreads();
-      // Lane e ranks entry e by (key desc, index asc); the entry of rank need - 1 is the k-th best.
-      const int m = __builtin_amdgcn_readfirstlane((int)in_bin);
-      const uint32_t ek = lane < m ? L.list_key[lane] : 0u, ei = lane < m ? L.list_id[lane] : 0xffffffffu;
-      int rank = 0;
-      for (int e = 0; e < m; ++e) {
-        const uint32_t sk = (uint32_t)__builtin_amdgcn_readlane((int)ek, e), si = (uint32_t)__builtin_amdgcn_readlane((int)ei, e);
-        rank += (sk > ek) | ((sk == ek) & (si < ei));
-      }
-      const uint64_t at = __ballot(lane < m && rank == need - 1);
-      const int src = at != 0 ? __ffsll((unsigned long long)at) - 1 : 0;
-      tk = (uint32_t)__builtin_amdgcn_readlane((int)ek, src);
-      tid = __builtin_amdgcn_readlane((int)ei, src);
+      rank_boundary(L.list_key, L.list_id, (int)in_bin, need, lane, &tk, &tid);
       found = true;
       break;
     }

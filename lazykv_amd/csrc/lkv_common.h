@@ -377,6 +377,26 @@ __device__ __forceinline__ void lane_pair_u32(uint32_t x, uint32_t& a, uint32_t&
   }
 }
 
+// The value of lane l ^ M: DPP within a 16-lane row (xor 4 as xor 7 and xor 3), a lane swap across rows.
+template <int M>
+__device__ __forceinline__ uint32_t lane_xor_u32(uint32_t x) {
+  static_assert(M == 1 || M == 2 || M == 4 || M == 8 || M == 16 || M == 32, "one bit of the lane id");
+  if constexpr (M == 1) {
+    return dpp_u32<kDppQuadSwap1>(x);
+  } else if constexpr (M == 2) {
+    return dpp_u32<kDppQuadSwap2>(x);
+  } else if constexpr (M == 4) {
+    constexpr int kDppQuadReverse = 0x1B;  // quad_perm [3,2,1,0]
+    return dpp_u32<kDppQuadReverse>(dpp_u32<kDppHalfMirror>(x));
+  } else if constexpr (M == 8) {
+    return dpp_u32<kDppRowRor8>(x);
+  } else {
+    uint32_t a, b;
+    lane_pair_u32<M>(x, a, b);
+    return (threadIdx.x & M) ? a : b;
+  }
+}
+
 // Inclusive prefix sum over the 64 lanes (ascending lane id): row_shr 1, 2, 4, 8 within each
 // 16-lane row, then row_bcast:15 adds row 0's total to row 1 and row 2's to row 3, and
 // row_bcast:31 adds the total of rows 0-1 to rows 2 and 3.

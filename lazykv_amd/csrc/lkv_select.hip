@@ -12,17 +12,13 @@
 // its channels of the G query heads in registers. The row sum is a 4-step DPP reduction; the max
 // over the group is taken in registers. The float32 bounds go to a scratch row per head.
 //
-// select_kernel: one 1024-thread workgroup per KV head; each thread holds a contiguous run of up to
-// 12 candidates as order-preserving integer keys in registers. The K-th largest is found by
-// range-adaptive radix select: each pass
+// Selection: one 1024-thread workgroup per KV head, by range-adaptive radix select: each pass
 // histograms the keys of the current range into at most 2048 bins scaled to that range (so the
 // first pass spreads the clustered bounds instead of piling them into a few exponent bins) and
-// keeps the bin holding the K-th key; once that bin holds at most 1024 keys they are ranked
-// directly, one thread each, instead of further passes over every key. An ordered compaction
-// then writes the ids in ascending order, or a bitonic sort puts them in descending bound order
-// with ties broken towards the lower id. Scoring and selection are separate launches so that no
-// workgroup has to publish its bounds across XCDs inside one launch (a device-scope release
-// writes back the L2); the kernel boundary does that once.
+// keeps the bin holding the K-th key; once that bin holds few keys they are ranked directly.
+// Scoring and selection are separate launches so that no workgroup has to publish its bounds across
+// XCDs inside one launch (a device-scope release writes back the L2); the kernel boundary does that
+// once.
 #include "lkv_blockselect.h"
 #include "lkv_common.h"
 
@@ -40,21 +36,7 @@ constexpr int kIter = LKV_BOUND_ITER;                     // 4-block rows per wa
 constexpr int kBlocksPerWG = kBoundWaves * 4 * kIter;     // candidate blocks per workgroup
 constexpr int kSelThreads = 1024;
 constexpr int kSelWaves = kSelThreads / 64;
-constexpr int kBins = 2048;
-constexpr int kPerThread = 12;                            // candidate keys held per thread
-static_assert(kPerThread <= 32, "a thread's candidate slots are tracked in 32-bit masks");
-constexpr int kMaxCand = kSelThreads * kPerThread;        // 12288 candidates per KV head
 constexpr int kMaxSortedK = 2048;
-// Passes of the radix select. Each pass narrows the live key range to one bin of at most 2048:
-// a 32-bit range (width < 2^32) becomes < 2^21 wide, then < 2^10, then a single key value, and the
-// fourth pass finds lo == hi and stops. The loops are capped at this count, so a kernel whose
-// invariants were broken still ends (with the threshold it has) instead of spinning.
-constexpr int kRadixPasses = 4;
-
-__device__ __forceinline__ uint32_t orderable(float f) {
-  uint32_t u = __float_as_uint(f);
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
 
 template <int D, int MT, int G>
 __global__ __launch_bounds__(kBoundThreads) void bound_kernel(const void* __restrict__ q, int q_dtype,
@@ -282,497 +264,392 @@ __global__ __launch_bounds__(kBoundMfThreads) void bound_kernel_mf(const uint16_
   }
 }
 
-// Exclusive prefix sum over the workgroup's threads (ascending thread id). `slots` holds one word
-// per wave and is read after a barrier; the caller separates reuses of `slots` by a barrier.
-__device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* slots, uint32_t* total) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const uint32_t x = lkv::wave_inclusive_sum(v);
-  if (lane == 63) slots[wave] = x;
-  __syncthreads();
-  uint32_t before = 0, all = 0;
-#pragma unroll
-  for (int w = 0; w < kSelWaves; ++w) {
-    uint32_t s = slots[w];
-    if (w < wave) before += s;
-    all += s;
-  }
-  *total = all;
-  return before + x - v;
-}
-
-constexpr int kStage = 4096;  // ids staged in LDS per coalesced write-out round
-
-__global__ __launch_bounds__(kSelThreads) void select_kernel(const float* __restrict__ bounds, int64_t bstride,
-                                                             int n_cand, int k, int cand_offset, int sorted,
-                                                             int32_t* __restrict__ out_idx, int64_t idx_stride) {
-  // LDS, one region per use so that phases need no barrier before reusing memory:
-  //   hist      -- radix histogram (kBins)
-  //   list      -- the boundary bin's keys and ids (2 * kSelThreads)
-  //   taken     -- bitmap of the boundary-bin keys that rank among the best (one bit per candidate)
-  //   stage     -- the selected ids in output order, written out coalesced (kStage), or the
-  //                64-bit sort slots of the sorted mode (2 * kp2 <= 2 * kMaxSortedK words)
-  //   mm / scan_* / info -- per-wave partials and broadcast words
-  static_assert(2 * kMaxSortedK <= kStage, "sort slots must fit the staging region");
-  __shared__ uint32_t hist[kBins + 64];  // + one spare bin per lane for keys outside the range
-  __shared__ uint32_t list[2 * kSelThreads];
-  __shared__ uint32_t taken[(kMaxCand + 31) / 32];
-  __shared__ __align__(16) uint32_t stage[kStage + 64];  // + one spare slot per lane
-  __shared__ uint32_t mm[2 * kSelWaves];
-  __shared__ uint32_t scan_pass[kSelWaves], scan_out[kSelWaves];
-  __shared__ uint32_t info[4];  // boundary bin, keys above it, keys in it, boundary-list length
-  const int h = blockIdx.x;
-  const int n = n_cand;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  // Keys per thread, a multiple of 4 so a thread's run is whole 16-byte vectors when rows are
-  // padded (bstride % 4 == 0).
-  const int npt = ((n + kSelThreads - 1) / kSelThreads + 3) & ~3;
-  const int i0 = threadIdx.x * npt;
-  const float* bound_h = bounds + (int64_t)h * bstride;
-
-  // Each thread holds the keys of indices [i0, i0 + npt) in registers; all loads in one round.
-  uint32_t key[kPerThread];
-  if ((bstride & 3) == 0) {
-#pragma unroll
-    for (int u = 0; u < kPerThread; u += 4) {
-      float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (u < npt && i0 + u < n) f = *(const float4*)(bound_h + i0 + u);  // padded row: in bounds
-      key[u] = orderable(f.x);
-      key[u + 1] = orderable(f.y);
-      key[u + 2] = orderable(f.z);
-      key[u + 3] = orderable(f.w);
-    }
-  } else {
-#pragma unroll
-    for (int u = 0; u < kPerThread; ++u) key[u] = (u < npt && i0 + u < n) ? orderable(bound_h[i0 + u]) : 0u;
-  }
-  // While the loads are in flight: clear the bitmap (read only after two later barriers) and the
-  // first pass's histogram (published by the min/max barrier below).
-  for (int i = threadIdx.x; i < (kMaxCand + 31) / 32; i += kSelThreads) taken[i] = 0u;
-  for (int i = threadIdx.x; i < kBins; i += kSelThreads) hist[i] = 0u;
-  // Slots u < nlive hold candidates (a count, not a per-slot flag array: an array of divergent
-  // booleans lives in scalar register pairs and spills).
-  const int nlive = max(0, min(npt, n - i0));
-  uint32_t lmin = 0xffffffffu, lmax = 0u;
-#pragma unroll
-  for (int u = 0; u < kPerThread; ++u) {
-    lmin = min(lmin, u < nlive ? key[u] : 0xffffffffu);
-    lmax = max(lmax, u < nlive ? key[u] : 0u);
-  }
-  // Workgroup min and max in one reduction.
-  lmin = lkv::wave_min_u32(lmin);
-  lmax = lkv::wave_max_u32(lmax);
-  if (lane == 0) {
-    mm[2 * wave] = lmin;
-    mm[2 * wave + 1] = lmax;
-  }
-  __syncthreads();
-  uint32_t lo = mm[0], hi = mm[1];
-#pragma unroll
-  for (int w = 1; w < kSelWaves; ++w) {
-    lo = min(lo, mm[2 * w]);
-    hi = max(hi, mm[2 * w + 1]);
-  }
-
-  // ---- range-adaptive radix select of the k-th largest key --------------------------------------
-  int need = k;  // keys still to take from [lo, hi]; every key above hi is taken
-  uint32_t T;    // after the loop: take every key > T, `need` keys == T, and the marked keys
-  uint32_t marked = 0u;  // bit u: key[u] lies in the final bin and ranks among the `need` best
-  bool first_pass = true;
-  T = lo;  // kept only if the pass cap is reached, which the narrowing above rules out
-#pragma unroll 1
-  for (int pass = 0; pass < kRadixPasses; ++pass) {
-    if (lo >= hi) {
-      T = lo;
-      break;
-    }
-    const uint32_t width = hi - lo;
-    const int bits = 32 - __clz(width);  // width < 2^bits
-    const int shift = bits > 11 ? bits - 11 : 0;
-    const int nb = (int)(width >> shift) + 1;  // at most 2048 bins
-    if (!first_pass) {
-      for (int i = threadIdx.x; i < nb; i += kSelThreads) hist[i] = 0;
-      __syncthreads();
-    }
-    first_pass = false;
-    // Branch-free: a key outside the range (or an empty slot) counts in this lane's spare bin.
-#pragma unroll
-    for (int u = 0; u < kPerThread; ++u) {
-      const bool in = u < nlive && key[u] >= lo && key[u] <= hi;
-      atomicAdd(&hist[in ? (key[u] - lo) >> shift : kBins + lane], 1u);
-    }
-    __syncthreads();
-    // Thread t owns bins [t*per, (t+1)*per); the bins above it hold `above` keys.
-    const int per = (nb + kSelThreads - 1) / kSelThreads;
-    uint32_t local = 0;
-    for (int j = 0; j < per; ++j) {
-      const int bin = threadIdx.x * per + j;
-      if (bin < nb) local += hist[bin];
-    }
-    uint32_t total;
-    const uint32_t below = block_exclusive_scan(local, scan_pass, &total);
-    const uint32_t above = total - below - local;
-    if (above < (uint32_t)need && (uint32_t)need <= above + local) {
-      uint32_t acc = above;
-      for (int j = per - 1; j >= 0; --j) {
-        const int bin = threadIdx.x * per + j;
-        const uint32_t cnt = bin < nb ? hist[bin] : 0u;
-        if ((uint32_t)need <= acc + cnt) {
-          info[0] = (uint32_t)bin;
-          info[1] = acc;
-          info[2] = cnt;
-          info[3] = 0u;
-          break;
-        }
-        acc += cnt;
-      }
-    }
-    __syncthreads();
-    const uint32_t bin = info[0];
-    need -= (int)info[1];
-    const uint32_t in_bin = info[2];
-    const uint32_t new_lo = lo + (bin << shift);
-    const uint32_t span = shift ? ((1u << shift) - 1u) : 0u;
-    hi = min(hi, new_lo + span);
-    lo = new_lo;
-    if (lo < hi && in_bin <= (uint32_t)kSelThreads) {
-      // Few keys left in the bin: rank them directly instead of more passes. They are listed (in
-      // any order) and ranked by (key desc, id asc); the `need` best are marked in a bitmap that
-      // each thread reads back for its own run of candidates.
-      uint32_t* list_key = list;
-      uint32_t* list_id = list + kSelThreads;
-#pragma unroll
-      for (int u = 0; u < kPerThread; ++u) {
-        if (u < nlive && key[u] >= lo && key[u] <= hi) {
-          const uint32_t slot = atomicAdd(&info[3], 1u);
-          list_key[slot] = key[u];
-          list_id[slot] = (uint32_t)(i0 + u);
-        }
-      }
-      __syncthreads();
-      const int m = (int)info[3];
-      if ((int)threadIdx.x < m) {
-        const uint32_t mk = list_key[threadIdx.x], mi = list_id[threadIdx.x];
-        int rank = 0;
-        for (int e = 0; e < m; ++e) {
-          const uint32_t ek = list_key[e], ei = list_id[e];
-          rank += (ek > mk) | ((ek == mk) & (ei < mi));
-        }
-        if (rank < need) atomicOr(&taken[mi >> 5], 1u << (mi & 31));
-      }
-      __syncthreads();
-      // A thread's run [i0, i0 + npt) spans at most two bitmap words.
-      const uint32_t w0 = taken[i0 >> 5];
-      const uint32_t w1 = ((i0 >> 5) + 1) < (kMaxCand + 31) / 32 ? taken[(i0 >> 5) + 1] : 0u;
-      const uint64_t bitsw = ((uint64_t)w1 << 32) | w0;
-      marked = (uint32_t)(bitsw >> (i0 & 31)) & ((npt >= 32) ? 0xffffffffu : ((1u << npt) - 1u));
-      T = hi;  // keys above are taken; keys in [lo, hi] are taken when marked
-      need = 0;
-      break;
-    }
-    __syncthreads();  // info and hist are rewritten by the next pass
-  }
-
-  // ---- ordered compaction: ascending block id ----------------------------------------------------
-  // One scan of (ties, taken-above) counts; ties are taken in index order, so the ties before a
-  // thread that are taken number min(ties before, need).
-  // Per thread, two bit masks over its slots: keys taken outright (above T, or marked) and ties
-  // (== T, unmarked). Built branch-free, kept in vector registers.
-  uint32_t above_m = 0u, tie_m = 0u;
-#pragma unroll
-  for (int u = 0; u < kPerThread; ++u) {
-    const uint32_t mk = (marked >> u) & 1u;
-    const uint32_t lv = u < nlive ? 1u : 0u;
-    above_m |= (lv & ((key[u] > T ? 1u : 0u) | mk)) << u;
-    tie_m |= (lv & (key[u] == T ? 1u : 0u) & (mk ^ 1u)) << u;
-  }
-  const uint32_t gt = __popc(above_m), eq = __popc(tie_m);
-  uint32_t tot;
-  const uint32_t packed = block_exclusive_scan((eq << 16) | gt, scan_out, &tot);
-  const int eq_before = (int)(packed >> 16), gt_before = (int)(packed & 0xffffu);
-  int take_eq = need - eq_before;
-  take_eq = take_eq < 0 ? 0 : (take_eq > (int)eq ? (int)eq : take_eq);
-  const uint32_t pos0 = (uint32_t)gt_before + (uint32_t)min(eq_before, need);
-  // Ties are taken in index order: this thread's first take_eq ties.
-  uint32_t ties_taken = tie_m;
-  for (int t = (int)eq; t > take_eq; --t) ties_taken &= ~(0x80000000u >> __clz(ties_taken));  // drop the highest
-  const uint32_t tk = above_m | ties_taken;  // the slots this thread contributes, in index order
-  int32_t* out_h = out_idx + (int64_t)h * idx_stride;
-  if (!sorted) {
-    // Each thread writes its ids straight to their output positions: a run of consecutive
-    // positions in index order, so the output is ascending (no staging round through LDS and its
-    // barrier).
-    uint32_t pos = pos0;
-#pragma unroll
-    for (int u = 0; u < kPerThread; ++u) {
-      const uint32_t bit = (tk >> u) & 1u;
-      if (bit && pos < (uint32_t)k) out_h[pos] = (int32_t)(i0 + u) + cand_offset;
-      pos += bit;
-    }
-    return;
-  }
-
-  // ---- sorted mode: bitonic sort, descending (key, then lower id first) --------------------------
-  uint64_t* sortbuf = reinterpret_cast<uint64_t*>(stage);
-  {
-    uint32_t pos = pos0;
-#pragma unroll
-    for (int u = 0; u < kPerThread; ++u) {
-      if ((tk >> u) & 1u) {
-        if (pos < (uint32_t)k) sortbuf[pos] = ((uint64_t)key[u] << 32) | (uint64_t)(0xffffffffu - (uint32_t)(i0 + u));
-        ++pos;
-      }
-    }
-  }
-  int kp2 = 1;
-  while (kp2 < k) kp2 <<= 1;
-  for (int i = k + threadIdx.x; i < kp2; i += kSelThreads) sortbuf[i] = 0;
-  __syncthreads();
-  for (int size = 2; size <= kp2; size <<= 1) {
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int t = threadIdx.x; t < kp2 / 2; t += kSelThreads) {
-        const int a = 2 * t - (t & (stride - 1));
-        const int b = a + stride;
-        const bool desc = (a & size) == 0;
-        const uint64_t x = sortbuf[a], y = sortbuf[b];
-        if ((x < y) == desc) {
-          sortbuf[a] = y;
-          sortbuf[b] = x;
-        }
-      }
-      __syncthreads();
-    }
-  }
-  for (int i = threadIdx.x; i < k; i += kSelThreads) {
-    const uint32_t id = 0xffffffffu - (uint32_t)(sortbuf[i] & 0xffffffffu);
-    out_h[i] = (int32_t)id + cand_offset;
-  }
-}
-
-// ---- the unsorted selection as one in-workgroup top-K ----------------------------------------------
-// The same rule and ids as select_kernel's unsorted mode, by the routine the decode and residency
-// launches run inside themselves (lkv_blockselect.h: 2,048 bins a pass read as vectors, a direct
-// rank of a small boundary bin, an exit when that bin is taken whole), with 1,024 threads of 8 keys
-// (8,192 candidates per head; every key slot a thread holds costs instructions in each phase, and
-// against 512 threads of 16 the 128K-token zero-copy step measured 615.23 -> 614.47 us per layer),
-// the wave index scalar in the scans (as lane masks, the scans' wave tests spilled scalar
-// registers), over rows that are 16-byte aligned and padded to 4 floats (the workspace's). Each
-// thread writes its ids straight to their ascending output positions.
-constexpr int kSelBlockThreads = 1024;
-constexpr int kSelBlockKpt = 8;
-constexpr int kSelBlockCap = kSelBlockThreads * kSelBlockKpt;  // 8,192 candidates per head
-__global__ __launch_bounds__(kSelBlockThreads) void select_block_kernel(const float* __restrict__ bounds, int64_t bstride,
-                                                                        int n_cand, int k, int cand_offset,
-                                                                        int32_t* __restrict__ out_idx, int64_t idx_stride) {
-  __shared__ lkv::SelectLds<kSelBlockThreads, kSelBlockKpt> L;
-  const int h = blockIdx.x;
-  const lkv::SelectPick pk = lkv::block_top_k<kSelBlockThreads, kSelBlockKpt, true>(bounds + (int64_t)h * bstride, true, n_cand, k, L);
-  int32_t* out_h = out_idx + (int64_t)h * idx_stride;
-  int pos = pk.pos;
-  for (uint32_t take = pk.take; take != 0u && pos < k; take &= take - 1u, ++pos) out_h[pos] = pk.i0 + __ffs((int)take) - 1 + cand_offset;
-}
-
 // Rows the in-workgroup top-K may read as 16-byte vectors: aligned, and padded to 4 floats.
 static bool rows_vector_readable(const float* bounds, int64_t bstride, int n_cand) {
   return ((uintptr_t)bounds & 15u) == 0 && bstride % 4 == 0 && bstride >= (int64_t)lkv_align_up((size_t)n_cand, 4);
 }
 
-// ---- select for long contexts: keys streamed from memory on every pass --------------------------
-// The same selection as select_kernel -- range-adaptive radix select of the K-th largest key, direct
-// ranking of the boundary bin, ties to the lower id, ascending or sorted output -- for heads with
-// more candidates than the registers hold (kMaxCand). Thread t owns the contiguous run
-// [t * npt, (t + 1) * npt) and re-reads its bounds (L2-resident after the first pass) on each pass.
+// ---- the general selection: any candidate count, any row alignment, either order ------------------
+// One 1024-thread workgroup per KV head. Each wave owns a contiguous run of candidates and reads it 256
+// at a time, 16 bytes a lane, four reads in flight, on every pass; the row comes from the L2 after the
+// first. (Reading a run per thread, a float at a time, the 65,535-candidate selection of a million-token
+// context took 155 us, nearly all of it in seven passes of strided 4-byte reads.) The k-th best
+// candidate (key, index) is found as block_top_k does (lkv_blockselect.h): a first range that starts at
+// the least of the lanes' own largest keys, histograms of the live range, and a boundary bin of at most
+// 64 keys ranked by every wave. One more pass writes the picks in index order; in sorted mode they are
+// gathered in LDS and sorted, each thread holding one or two in registers: only partners in other waves
+// go through LDS, 10 of the 55 steps for 1,024 picks, and the others are lane exchanges. With the bound launch, 1,024 of 65,535 in descending order: 176.0 -> 51.1 us (head_dim 64), 2,047
+// of 262,144: 654 -> 151; what is left is one CU's vector work per head, three passes over its row.
 constexpr int kMaxStreamCand = 1 << 18;  // 262,144 candidates per head: 4M tokens at 16-token blocks
 
-__global__ __launch_bounds__(kSelThreads) void select_stream_kernel(const float* __restrict__ bounds, int64_t bstride,
-                                                                    int n_cand, int k, int cand_offset, int sorted,
-                                                                    int32_t* __restrict__ out_idx, int64_t idx_stride) {
-  __shared__ uint32_t hist[kBins];
-  __shared__ uint32_t list[2 * kSelThreads];
-  __shared__ uint32_t taken[kMaxStreamCand / 32];
-  __shared__ __align__(16) uint32_t stage[kStage];
-  __shared__ uint32_t mm[2 * kSelWaves];
-  __shared__ uint32_t scan_pass[kSelWaves], scan_out[kSelWaves];
-  __shared__ uint32_t info[4];
-  const int h = blockIdx.x;
-  const int n = n_cand;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int npt = (n + kSelThreads - 1) / kSelThreads;
-  const int i0 = threadIdx.x * npt;
-  const int i1 = min(n, i0 + npt);
-  const float* bound_h = bounds + (int64_t)h * bstride;
-  for (int i = threadIdx.x; i < (n + 31) / 32; i += kSelThreads) taken[i] = 0u;
-  uint32_t lmin = 0xffffffffu, lmax = 0u;
-  for (int i = i0; i < i1; ++i) {
-    const uint32_t key = orderable(bound_h[i]);
-    lmin = min(lmin, key);
-    lmax = max(lmax, key);
+// f(i, keys of candidates i .. i + 3, how many of them exist) over [begin, end), 256 candidates a call.
+template <bool VEC, typename F>
+__device__ __forceinline__ void for_each_quad(const float* __restrict__ row, int begin, int end, int lane, F&& f) {
+  int base = begin;
+  if constexpr (VEC) {
+#pragma unroll 1
+    for (; base + 1024 <= end; base += 1024) {  // whole batches: no bounds to look at
+      uint4 x[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = *(const uint4*)(row + base + 256 * u + 4 * lane);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t key[4] = {lkv::orderable_bits(x[u].x), lkv::orderable_bits(x[u].y), lkv::orderable_bits(x[u].z), lkv::orderable_bits(x[u].w)};
+        f(base + 256 * u + 4 * lane, key, 4);
+      }
+    }
   }
-  lmin = lkv::wave_min_u32(lmin);
-  lmax = lkv::wave_max_u32(lmax);
+#pragma unroll 1
+  for (; base < end; base += 256) {  // wave-uniform: every lane of the wave calls f
+    const int i = base + 4 * lane;
+    uint32_t key[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) key[e] = i + e < end ? lkv::orderable_key(row[i + e]) : 0u;
+    f(i, key, max(0, min(4, end - i)));
+  }
+}
+
+// Element of a descending bitonic merge: keeps the larger of its own and its partner's value where
+// `larger`, else the smaller.
+__device__ __forceinline__ uint64_t keep_one(uint64_t mine, uint64_t theirs, bool larger) {
+  return ((mine > theirs) == larger) ? mine : theirs;
+}
+
+template <int M>
+__device__ __forceinline__ uint64_t lane_xor_u64(uint64_t x) {
+  return ((uint64_t)lkv::lane_xor_u32<M>((uint32_t)(x >> 32)) << 32) | lkv::lane_xor_u32<M>((uint32_t)x);
+}
+
+// The in-wave steps (stride M, M / 2, .., 1) of a merge.
+template <int M>
+__device__ __forceinline__ uint64_t merge_in_wave(uint64_t x, int t, bool desc) {
+  x = keep_one(x, lane_xor_u64<M>(x), ((t & M) == 0) == desc);
+  if constexpr (M > 1) {
+    return merge_in_wave<M / 2>(x, t, desc);
+  } else {
+    return x;
+  }
+}
+
+struct SortLds {
+  uint64_t slot[2][kMaxSortedK];
+};
+
+// Sorts the np2 values in L.slot[0] (a power of two, 64 to kMaxSortedK) in descending order. Thread t
+// returns elements t and t + 1024.
+__device__ __forceinline__ void sort_descending(SortLds& L, int np2, uint64_t (&x)[2]) {
+  const int t = threadIdx.x;
+  const bool two = np2 > kSelThreads;
+  x[0] = t < np2 ? L.slot[0][t] : 0u;
+  x[1] = two ? L.slot[0][t + kSelThreads] : 0u;
+  int buf = 1;
+#pragma unroll 1
+  for (int size = 2; size <= np2; size <<= 1) {
+    // Element i of a run of `size` merges in descending order where (i & size) == 0. The bit is the same
+    // for both elements of a thread but where size is the distance between them.
+    const bool d0 = (t & size) == 0, d1 = ((t + kSelThreads) & size) == 0;
+#pragma unroll 1
+    for (int stride = size >> 1; stride >= 64; stride >>= 1) {
+      if (stride == kSelThreads) {  // the thread's own two elements, in the last merge
+        const uint64_t a = x[0], b = x[1];
+        x[0] = a > b ? a : b;
+        x[1] = a > b ? b : a;
+        continue;
+      }
+      // Two buffers in turn: a buffer is written again only after the next step's barrier.
+      L.slot[buf][t] = x[0];
+      if (two) L.slot[buf][t + kSelThreads] = x[1];
+      __syncthreads();
+      x[0] = keep_one(x[0], L.slot[buf][t ^ stride], ((t & stride) == 0) == d0);
+      if (two) x[1] = keep_one(x[1], L.slot[buf][(t ^ stride) + kSelThreads], ((t & stride) == 0) == d1);
+      buf ^= 1;
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      if (e == 1 && !two) break;
+      const bool desc = e == 0 ? d0 : d1;
+      switch (min(size >> 1, 32)) {
+        case 32: x[e] = merge_in_wave<32>(x[e], t, desc); break;
+        case 16: x[e] = merge_in_wave<16>(x[e], t, desc); break;
+        case 8: x[e] = merge_in_wave<8>(x[e], t, desc); break;
+        case 4: x[e] = merge_in_wave<4>(x[e], t, desc); break;
+        case 2: x[e] = merge_in_wave<2>(x[e], t, desc); break;
+        default: x[e] = merge_in_wave<1>(x[e], t, desc); break;
+      }
+    }
+  }
+}
+
+__device__ __forceinline__ void write_sorted(SortLds& L, int np2, int k, int cand_offset, int32_t* __restrict__ out_h) {
+  uint64_t x[2];
+  sort_descending(L, np2, x);
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int i = (int)threadIdx.x + e * kSelThreads;
+    if (i < k) out_h[i] = (int32_t)(0xffffffffu - (uint32_t)x[e]) + cand_offset;
+  }
+}
+
+struct SelectRowLds {
+  alignas(16) uint32_t hist[lkv::kSelBins];
+  uint32_t list_key[lkv::kSelRank], list_id[lkv::kSelRank];
+  uint32_t mm[2 * kSelWaves];
+  uint32_t scan[2][kSelWaves];
+  uint32_t info[5];  // boundary bin, keys above it, keys in it, boundary keys listed, picks gathered
+  union {
+    SortLds sort;                            // sorted mode
+    uint32_t picked[kMaxStreamCand / 32];    // ascending mode: one bit per candidate
+  };
+};
+
+template <bool VEC>
+__device__ __forceinline__ void select_row(const float* __restrict__ row, int n, int k, int cand_offset, int sorted,
+                                           int32_t* __restrict__ out_h, SelectRowLds& L) {
+  constexpr int kBpt = lkv::kSelBins / kSelThreads;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int run = ((n + kSelWaves - 1) / kSelWaves + 255) & ~255;  // candidates a wave owns
+  const int begin = min(n, wave * run), end = min(n, begin + run);
+  int np2 = 64;  // sorted mode: slots to sort
+  while (np2 < k) np2 <<= 1;
+  lkv::clear_bins<kBpt>(L.hist + threadIdx.x * kBpt);
+  if (sorted) {
+    for (int i = k + threadIdx.x; i < np2; i += kSelThreads) L.sort.slot[0][i] = 0u;
+  } else {
+    for (int i = threadIdx.x; i < (n + 31) / 32; i += kSelThreads) L.picked[i] = 0u;
+  }
+  if (threadIdx.x == 0) L.info[4] = 0u;
+
+  // ---- the range: what at least k keys reach, and the largest key ---------------------------------
+  // n1 lanes hold a key, n2 of them two or more.
+  const int tail = n % run;
+  const int n1 = n / run * 64 + min(64, (tail + 3) / 4), n2 = n / run * 64 + min(64, (tail + 2) / 4);
+  uint32_t m1 = 0u, m2 = 0u, low = 0xffffffffu;
+  if (k <= n1) {  // uniform, as below
+    for_each_quad<VEC>(row, begin, end, lane, [&](int, const uint32_t (&key)[4], int cnt) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m1 = max(m1, e < cnt ? key[e] : 0u);
+    });
+    if (begin + 4 * lane < end) low = m1;
+  } else if (k <= 2 * n2) {
+    for_each_quad<VEC>(row, begin, end, lane, [&](int, const uint32_t (&key)[4], int cnt) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t x = e < cnt ? key[e] : 0u;
+        m2 = max(m2, min(m1, x));
+        m1 = max(m1, x);
+      }
+    });
+    if (begin + 4 * lane + 1 < end) low = m2;
+  } else {
+    for_each_quad<VEC>(row, begin, end, lane, [&](int, const uint32_t (&key)[4], int cnt) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        m1 = max(m1, e < cnt ? key[e] : 0u);
+        low = min(low, e < cnt ? key[e] : 0xffffffffu);
+      }
+    });
+  }
+  low = lkv::wave_min_u32(low);
+  m1 = lkv::wave_max_u32(m1);
   if (lane == 0) {
-    mm[2 * wave] = lmin;
-    mm[2 * wave + 1] = lmax;
+    L.mm[2 * wave] = low;
+    L.mm[2 * wave + 1] = m1;
   }
   __syncthreads();
-  uint32_t lo = mm[0], hi = mm[1];
+  uint32_t lo = L.mm[0], hi = L.mm[1];
 #pragma unroll
   for (int w = 1; w < kSelWaves; ++w) {
-    lo = min(lo, mm[2 * w]);
-    hi = max(hi, mm[2 * w + 1]);
+    lo = min(lo, L.mm[2 * w]);
+    hi = max(hi, L.mm[2 * w + 1]);
   }
+
+  // ---- the range of the k-th best: keys above it are taken, `need` of those in it --------------------
   int need = k;
-  uint32_t T;
-  bool ranked = false;  // the boundary bin was ranked directly: its best keys are marked in `taken`
-  T = lo;  // kept only if the pass cap is reached, which the narrowing rules out
+  bool whole = false, ranked = false;
 #pragma unroll 1
-  for (int pass = 0; pass < kRadixPasses; ++pass) {
-    if (lo >= hi) {
-      T = lo;
-      break;
-    }
+  for (int pass = 0; pass < lkv::kSelPasses; ++pass) {
+    if (lo >= hi) break;
     const uint32_t width = hi - lo;
     const int bits = 32 - __clz(width);
     const int shift = bits > 11 ? bits - 11 : 0;
-    const int nb = (int)(width >> shift) + 1;
-    for (int i = threadIdx.x; i < nb; i += kSelThreads) hist[i] = 0;
-    __syncthreads();
-    for (int i = i0; i < i1; ++i) {
-      const uint32_t key = orderable(bound_h[i]);
-      if (key >= lo && key <= hi) atomicAdd(&hist[(key - lo) >> shift], 1u);
+    if (pass > 0) {
+      lkv::clear_bins<kBpt>(L.hist + threadIdx.x * kBpt);
+      __syncthreads();
     }
+    for_each_quad<VEC>(row, begin, end, lane, [&](int, const uint32_t (&key)[4], int cnt) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (e < cnt && key[e] - lo <= width) atomicAdd(&L.hist[(key[e] - lo) >> shift], 1u);
+    });
     __syncthreads();
-    const int per = (nb + kSelThreads - 1) / kSelThreads;
+    uint32_t cnt[kBpt];
+    lkv::read_bins<kBpt>(L.hist + threadIdx.x * kBpt, cnt);
     uint32_t local = 0;
-    for (int j = 0; j < per; ++j) {
-      const int bin = threadIdx.x * per + j;
-      if (bin < nb) local += hist[bin];
-    }
+#pragma unroll
+    for (int b = 0; b < kBpt; ++b) local += cnt[b];
     uint32_t total;
-    const uint32_t below = block_exclusive_scan(local, scan_pass, &total);
+    const uint32_t below = lkv::workgroup_exclusive_sum<kSelThreads, true>(local, L.scan[0], &total);
     const uint32_t above = total - below - local;
     if (above < (uint32_t)need && (uint32_t)need <= above + local) {
       uint32_t acc = above;
-      for (int j = per - 1; j >= 0; --j) {
-        const int bin = threadIdx.x * per + j;
-        const uint32_t cnt = bin < nb ? hist[bin] : 0u;
-        if ((uint32_t)need <= acc + cnt) {
-          info[0] = (uint32_t)bin;
-          info[1] = acc;
-          info[2] = cnt;
-          info[3] = 0u;
-          break;
+#pragma unroll
+      for (int b = kBpt - 1; b >= 0; --b) {
+        if (acc < (uint32_t)need && (uint32_t)need <= acc + cnt[b]) {
+          L.info[0] = (uint32_t)(threadIdx.x * kBpt + b);
+          L.info[1] = acc;
+          L.info[2] = cnt[b];
+          L.info[3] = 0u;
         }
-        acc += cnt;
+        acc += cnt[b];
       }
     }
     __syncthreads();
-    const uint32_t bin = info[0];
-    need -= (int)info[1];
-    const uint32_t in_bin = info[2];
-    const uint32_t new_lo = lo + (bin << shift);
-    const uint32_t span = shift ? ((1u << shift) - 1u) : 0u;
-    hi = min(hi, new_lo + span);
+    const uint32_t new_lo = lo + (L.info[0] << shift);
+    need -= (int)L.info[1];
+    const uint32_t in_bin = L.info[2];
+    hi = min(hi, new_lo + (shift ? ((1u << shift) - 1u) : 0u));
     lo = new_lo;
-    if (lo < hi && in_bin <= (uint32_t)kSelThreads) {
-      uint32_t* list_key = list;
-      uint32_t* list_id = list + kSelThreads;
-      for (int i = i0; i < i1; ++i) {
-        const uint32_t key = orderable(bound_h[i]);
-        if (key >= lo && key <= hi) {
-          const uint32_t slot = atomicAdd(&info[3], 1u);
-          list_key[slot] = key;
-          list_id[slot] = (uint32_t)i;
-        }
+    whole = in_bin == (uint32_t)need;
+    ranked = !whole && lo < hi && in_bin <= (uint32_t)lkv::kSelRank;
+    if (whole || ranked) break;
+  }
+  // Taken are the keys above tk, and those equal to it up to index tid; of a boundary bin to be ranked,
+  // also the `need` best.
+  uint32_t tk = ranked ? hi : lo;
+  int tid = whole ? 0x7fffffff : -1;
+  if (!whole && !ranked) {
+    // Every key left equals tk: the first `need` of them in index order are taken. The wave that holds
+    // the need-th looks for its index.
+    uint32_t eq = 0;
+    for_each_quad<VEC>(row, begin, end, lane, [&](int, const uint32_t (&key)[4], int cnt) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) eq += e < cnt && key[e] == tk ? 1u : 0u;
+    });
+    uint32_t total;
+    const uint32_t mine = lkv::workgroup_exclusive_sum<kSelThreads, true>(eq, L.scan[1], &total);
+    int before = __builtin_amdgcn_readfirstlane((int)mine);  // ties in the runs of earlier waves
+    for_each_quad<VEC>(row, begin, end, lane, [&](int i, const uint32_t (&key)[4], int cnt) {
+      uint32_t m = 0u;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m |= (e < cnt && key[e] == tk ? 1u : 0u) << e;
+      const uint32_t c = __popc(m), incl = lkv::wave_inclusive_sum(c);
+      const int first = before + (int)(incl - c);  // ties before this lane's
+      if (first < need && need <= first + (int)c) {
+        for (int t = first + 1; t < need; ++t) m &= m - 1u;
+        L.info[0] = (uint32_t)(i + __ffs((int)m) - 1);
       }
-      __syncthreads();
-      const int m = (int)info[3];
-      if ((int)threadIdx.x < m) {
-        const uint32_t mk = list_key[threadIdx.x], mi = list_id[threadIdx.x];
-        int rank = 0;
-        for (int e = 0; e < m; ++e) {
-          const uint32_t ek = list_key[e], ei = list_id[e];
-          rank += (ek > mk) | ((ek == mk) & (ei < mi));
-        }
-        if (rank < need) atomicOr(&taken[mi >> 5], 1u << (mi & 31));
+      before += __builtin_amdgcn_readlane((int)incl, 63);
+    });
+    __syncthreads();
+    tid = (int)L.info[0];
+  }
+
+  // ---- the picks --------------------------------------------------------------------------------------
+  const auto pick = [&](uint32_t key, int id) {
+    if (sorted) {
+      const uint32_t slot = atomicAdd(&L.info[4], 1u);
+      if (slot < (uint32_t)k) L.sort.slot[0][slot] = ((uint64_t)key << 32) | (uint64_t)(0xffffffffu - (uint32_t)id);
+    } else {
+      atomicOr(&L.picked[id >> 5], 1u << (id & 31));
+    }
+  };
+  for_each_quad<VEC>(row, begin, end, lane, [&](int i, const uint32_t (&key)[4], int cnt) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (e >= cnt || key[e] < lo) continue;
+      if (key[e] > tk || (key[e] == tk && i + e <= tid)) {
+        pick(key[e], i + e);
+      } else if (ranked) {
+        const uint32_t slot = atomicAdd(&L.info[3], 1u);
+        L.list_key[slot] = key[e];
+        L.list_id[slot] = (uint32_t)(i + e);
       }
-      __syncthreads();
-      T = hi;
-      need = 0;
-      ranked = true;
-      break;
+    }
+  });
+  __syncthreads();
+  if (ranked) {
+    if (wave == 0) {
+      const int m = (int)L.info[3];
+      lkv::rank_boundary(L.list_key, L.list_id, m, need, lane, &tk, &tid);
+      if (lane < m) {
+        const uint32_t key = L.list_key[lane];
+        const int id = (int)L.list_id[lane];
+        if (key > tk || (key == tk && id <= tid)) pick(key, id);
+      }
     }
     __syncthreads();
   }
 
-  // ---- compaction: ascending id, ties (== T, unmarked) taken in index order ---------------------
-  uint32_t gt = 0, eq = 0;
-  for (int i = i0; i < i1; ++i) {
-    const uint32_t key = orderable(bound_h[i]);
-    const bool mk = ranked && ((taken[i >> 5] >> (i & 31)) & 1u);
-    gt += (key > T) | mk;
-    eq += (key == T) & !mk;
+  if (!sorted) {
+    const int words = (n + 31) / 32;
+    const int per = (words + kSelThreads - 1) / kSelThreads;
+    const int w0 = threadIdx.x * per;
+    uint32_t mine = 0;
+    for (int w = w0; w < min(words, w0 + per); ++w) mine += __popc(L.picked[w]);
+    uint32_t total;
+    int pos = (int)lkv::workgroup_exclusive_sum<kSelThreads, true>(mine, L.scan[0], &total);
+    for (int w = w0; w < min(words, w0 + per); ++w)
+      for (uint32_t m = L.picked[w]; m != 0u && pos < k; m &= m - 1u, ++pos) out_h[pos] = 32 * w + __ffs((int)m) - 1 + cand_offset;
+    return;
   }
-  uint32_t tot;
-  const uint32_t before_gt = block_exclusive_scan(gt, scan_out, &tot);
-  __syncthreads();  // scan_out is reused just below
-  const uint32_t before_eq = block_exclusive_scan(eq, scan_out, &tot);
-  int take_eq = need - (int)before_eq;
-  take_eq = take_eq < 0 ? 0 : (take_eq > (int)eq ? (int)eq : take_eq);
-  const uint32_t pos0 = before_gt + (uint32_t)min((int)before_eq, need);
+  // Descending key, equal keys by the lower id.
+  write_sorted(L.sort, np2, k, cand_offset, out_h);
+}
+
+// ---- the selection as one in-workgroup top-K ----------------------------------------------------------
+// The rule of select_row, by the routine the decode and residency launches run inside themselves
+// (lkv_blockselect.h), which reads the row once into registers: 1,024 threads of 8 keys (8,192 candidates
+// per head) or 12 (12,288; every key slot a thread holds costs instructions in each phase: at 8,192
+// candidates, against 512 threads of 16, the 128K-token zero-copy step measured 615.23 -> 614.47 us per
+// layer), with the wave index scalar in the scans (as lane masks, the scans' wave tests spilled
+// scalar registers), over rows that are 16-byte aligned and padded to 4 floats (the workspace's). Each
+// thread writes its ids straight to their ascending output positions, or, in sorted mode, to the sort's
+// slots. Against select_row, which reads the row three times: 512 of 8,190 in descending order 20.5 -> 16.0 us
+// with the bound launch, 768 of 12,286 ascending 19.3 -> 11.9.
+constexpr int kSelBlockThreads = 1024;
+constexpr int kSelBlockCap = kSelBlockThreads * 12;
+template <int KPT, bool SORTED>
+__global__ __launch_bounds__(kSelBlockThreads) void select_block_kernel(const float* __restrict__ bounds, int64_t bstride,
+                                                                        int n_cand, int k, int cand_offset,
+                                                                        int32_t* __restrict__ out_idx, int64_t idx_stride) {
+  static_assert(kSelBlockThreads == kSelThreads, "the sort's thread count");
+  __shared__ lkv::SelectLds<kSelBlockThreads, KPT> L;
+  const int h = blockIdx.x;
+  const float* row = bounds + (int64_t)h * bstride;
+  const lkv::SelectPick pk = lkv::block_top_k<kSelBlockThreads, KPT, true>(row, true, n_cand, k, L);
   int32_t* out_h = out_idx + (int64_t)h * idx_stride;
-  uint64_t* sortbuf = reinterpret_cast<uint64_t*>(stage);
-  for (int base = 0; base < (sorted ? 1 : k); base += kStage) {
-    const uint32_t lim = sorted ? (uint32_t)k : (uint32_t)min(base + kStage, k);
-    uint32_t pos = pos0;
-    int taken_eq = 0;
-    for (int i = i0; i < i1; ++i) {
-      const uint32_t key = orderable(bound_h[i]);
-      const bool mk = ranked && ((taken[i >> 5] >> (i & 31)) & 1u);
-      bool take = (key > T) || mk;
-      if (!take && key == T && taken_eq < take_eq) {
-        take = true;
-        ++taken_eq;
-      }
-      if (take) {
-        if (pos >= (uint32_t)base && pos < lim) {
-          if (sorted) {
-            sortbuf[pos] = ((uint64_t)key << 32) | (uint64_t)(0xffffffffu - (uint32_t)i);
-          } else {
-            stage[pos - base] = (uint32_t)i;
-          }
-        }
-        ++pos;
-      }
+  int pos = pk.pos;
+  if constexpr (!SORTED) {
+    for (uint32_t take = pk.take; take != 0u && pos < k; take &= take - 1u, ++pos) out_h[pos] = pk.i0 + __ffs((int)take) - 1 + cand_offset;
+  } else {
+    __shared__ SortLds sort;
+    int np2 = 64;
+    while (np2 < k) np2 <<= 1;
+    for (int i = k + threadIdx.x; i < np2; i += kSelThreads) sort.slot[0][i] = 0u;
+    for (uint32_t take = pk.take; take != 0u && pos < k; take &= take - 1u, ++pos) {
+      const int i = pk.i0 + __ffs((int)take) - 1;
+      sort.slot[0][pos] = ((uint64_t)lkv::orderable_key(row[i]) << 32) | (uint64_t)(0xffffffffu - (uint32_t)i);
     }
     __syncthreads();
-    if (sorted) break;
-    for (int i = threadIdx.x; i < kStage && base + i < k; i += kSelThreads) out_h[base + i] = (int32_t)stage[i] + cand_offset;
-    __syncthreads();
+    write_sorted(sort, np2, k, cand_offset, out_h);
   }
-  if (!sorted) return;
-  int kp2 = 1;
-  while (kp2 < k) kp2 <<= 1;
-  for (int i = k + threadIdx.x; i < kp2; i += kSelThreads) sortbuf[i] = 0;
-  __syncthreads();
-  for (int size = 2; size <= kp2; size <<= 1) {
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int t = threadIdx.x; t < kp2 / 2; t += kSelThreads) {
-        const int a = 2 * t - (t & (stride - 1));
-        const int b = a + stride;
-        const bool desc = (a & size) == 0;
-        const uint64_t x = sortbuf[a], y = sortbuf[b];
-        if ((x < y) == desc) {
-          sortbuf[a] = y;
-          sortbuf[b] = x;
-        }
-      }
-      __syncthreads();
-    }
-  }
-  for (int i = threadIdx.x; i < k; i += kSelThreads) {
-    const uint32_t id = 0xffffffffu - (uint32_t)(sortbuf[i] & 0xffffffffu);
-    out_h[i] = (int32_t)id + cand_offset;
-  }
+}
+
+// Rows that may be read as 16-byte vectors (the workspace's: aligned, padded to 4 floats).
+__global__ __launch_bounds__(kSelThreads) void select_stream_kernel(const float* __restrict__ bounds, int64_t bstride, int n_cand, int k,
+                                                                    int cand_offset, int sorted, int32_t* __restrict__ out_idx,
+                                                                    int64_t idx_stride) {
+  __shared__ SelectRowLds L;
+  select_row<true>(bounds + (int64_t)blockIdx.x * bstride, n_cand, k, cand_offset, sorted, out_idx + (int64_t)blockIdx.x * idx_stride, L);
+}
+
+// Any row (a caller's dense bounds).
+__global__ __launch_bounds__(kSelThreads) void select_kernel(const float* __restrict__ bounds, int64_t bstride, int n_cand, int k,
+                                                             int cand_offset, int sorted, int32_t* __restrict__ out_idx,
+                                                             int64_t idx_stride) {
+  __shared__ SelectRowLds L;
+  select_row<false>(bounds + (int64_t)blockIdx.x * bstride, n_cand, k, cand_offset, sorted, out_idx + (int64_t)blockIdx.x * idx_stride, L);
 }
 
 template <int D, int MT, int G>
@@ -833,20 +710,41 @@ int lkv_launch_bounds(hipStream_t s, const void* q, int q_dtype, const void* kmi
 
 int lkv_select_max_candidates() { return kMaxStreamCand; }
 
-int lkv_launch_select(hipStream_t s, const float* bounds, int64_t bstride, int n_kv, int n_cand, int k, int cand_offset,
-                      int32_t* out_idx, int64_t idx_stride) {
-  if (n_cand <= kSelBlockCap && rows_vector_readable(bounds, bstride, n_cand)) {
-    hipLaunchKernelGGL(select_block_kernel, dim3(n_kv), dim3(kSelBlockThreads), 0, s, bounds, bstride, n_cand, k, cand_offset,
+// Up to kSelBlockCap candidates in rows that can be read as vectors: the in-workgroup top-K, which reads the
+// row once. Any other selection reads it three times, as 16-byte vectors where the rows allow.
+template <int KPT>
+static void launch_select_block(hipStream_t s, const float* bounds, int64_t bstride, int n_kv, int n_cand, int k, int cand_offset, int sorted,
+                                int32_t* out_idx, int64_t idx_stride) {
+  if (sorted) {
+    hipLaunchKernelGGL((select_block_kernel<KPT, true>), dim3(n_kv), dim3(kSelBlockThreads), 0, s, bounds, bstride, n_cand, k, cand_offset,
                        out_idx, idx_stride);
-  } else if (n_cand <= kMaxCand) {
-    hipLaunchKernelGGL(select_kernel, dim3(n_kv), dim3(kSelThreads), 0, s, bounds, bstride, n_cand, k, cand_offset, 0, out_idx,
+  } else {
+    hipLaunchKernelGGL((select_block_kernel<KPT, false>), dim3(n_kv), dim3(kSelBlockThreads), 0, s, bounds, bstride, n_cand, k, cand_offset,
+                       out_idx, idx_stride);
+  }
+}
+
+static int launch_select(hipStream_t s, const float* bounds, int64_t bstride, int n_kv, int n_cand, int k, int cand_offset, int sorted,
+                         int32_t* out_idx, int64_t idx_stride) {
+  const bool vec = rows_vector_readable(bounds, bstride, n_cand);
+  if (vec && n_cand <= kSelBlockThreads * 8) {
+    launch_select_block<8>(s, bounds, bstride, n_kv, n_cand, k, cand_offset, sorted, out_idx, idx_stride);
+  } else if (vec && n_cand <= kSelBlockCap) {
+    launch_select_block<12>(s, bounds, bstride, n_kv, n_cand, k, cand_offset, sorted, out_idx, idx_stride);
+  } else if (vec) {
+    hipLaunchKernelGGL(select_stream_kernel, dim3(n_kv), dim3(kSelThreads), 0, s, bounds, bstride, n_cand, k, cand_offset, sorted, out_idx,
                        idx_stride);
   } else {
-    hipLaunchKernelGGL(select_stream_kernel, dim3(n_kv), dim3(kSelThreads), 0, s, bounds, bstride, n_cand, k, cand_offset, 0,
-                       out_idx, idx_stride);
+    hipLaunchKernelGGL(select_kernel, dim3(n_kv), dim3(kSelThreads), 0, s, bounds, bstride, n_cand, k, cand_offset, sorted, out_idx,
+                       idx_stride);
   }
   LKV_CHECK_LAUNCH("select");
   return LKV_OK;
+}
+
+int lkv_launch_select(hipStream_t s, const float* bounds, int64_t bstride, int n_kv, int n_cand, int k, int cand_offset,
+                      int32_t* out_idx, int64_t idx_stride) {
+  return launch_select(s, bounds, bstride, n_kv, n_cand, k, cand_offset, 0, out_idx, idx_stride);
 }
 
 extern "C" int lkv_bound_topk(uintptr_t stream, const void* q, int q_dtype, const void* kmin, const void* kmax,
@@ -889,16 +787,5 @@ extern "C" int lkv_bound_topk(uintptr_t stream, const void* q, int q_dtype, cons
   const int rc = lkv_launch_bounds(s, q, q_dtype, kmin, kmax, meta_dtype, meta_head_stride, n_kv, g, head_dim, cand_offset, n_cand,
                                    rank_mode, bounds, bstride);
   if (rc != LKV_OK || k == 0) return rc;
-  if (n_cand <= kSelBlockCap && !sorted && rows_vector_readable(bounds, bstride, n_cand)) {
-    hipLaunchKernelGGL(select_block_kernel, dim3(n_kv), dim3(kSelBlockThreads), 0, s, bounds, bstride, n_cand, k, cand_offset,
-                       out_idx, idx_stride);
-  } else if (n_cand <= kMaxCand) {
-    hipLaunchKernelGGL(select_kernel, dim3(n_kv), dim3(kSelThreads), 0, s, bounds, bstride, n_cand, k, cand_offset,
-                       sorted, out_idx, idx_stride);
-  } else {
-    hipLaunchKernelGGL(select_stream_kernel, dim3(n_kv), dim3(kSelThreads), 0, s, bounds, bstride, n_cand, k,
-                       cand_offset, sorted, out_idx, idx_stride);
-  }
-  LKV_CHECK_LAUNCH("select");
-  return LKV_OK;
+  return launch_select(s, bounds, bstride, n_kv, n_cand, k, cand_offset, sorted, out_idx, idx_stride);
 }

@@ -51,3 +51,36 @@ def test_selection_in_one_workgroup_takes_the_best_k(n: int, k: int, kind: str) 
     kernels.select_decode(q, kmax, kmax, k, cand_offset=0, n_cand=n, block_size=16, scale=0.125, sel=kernels.pool_source(store), out_idx=fused)
     assert np.array_equal(idx.cpu().numpy(), want)
     assert np.array_equal(fused.cpu().numpy(), want)
+
+
+# Around a wave's run of 256 candidates, the in-workgroup limit, and the largest count; k around whole powers
+# of two, the sort's own edges.
+LONG = [(3, 2), (255, 64), (257, 65), (4097, 1025), (8193, 700), (12289, 2048), (16640, 1), (65535, 1024), (262144, 2047)]
+
+
+@pytest.mark.parametrize("kind", ["normal", "cluster", "one value", "sorted"])
+@pytest.mark.parametrize(("n", "k"), LONG)
+def test_long_and_sorted_selections_take_the_best_k(n: int, k: int, kind: str) -> None:
+    """Ascending and descending, from the workspace's rows and from a caller's dense bounds."""
+    from lazykv_amd import kernels
+
+    h = 2
+    values, kmax, q = _metadata(kind, h, n, n + k)
+    order = [np.lexsort((np.arange(n), -values[j]))[:k] for j in range(h)]
+    for sorted_ in (False, True):
+        want = np.stack([o if sorted_ else np.sort(o) for o in order])
+        got = kernels.bound_topk(q, kmax, kmax, k, sorted_=sorted_)
+        dense = torch.empty((h, n), dtype=torch.float32, device="cuda")
+        got_dense = kernels.bound_topk(q, kmax, kmax, k, sorted_=sorted_, out_bound=dense)
+        assert np.array_equal(got.cpu().numpy(), want), sorted_
+        assert np.array_equal(got_dense.cpu().numpy(), want), sorted_
+        assert np.array_equal(dense.cpu().numpy().astype(np.float64), values)
+
+
+@pytest.mark.parametrize(("n", "k"), [(20000, 5000), (20000, 20000), (30001, 29999)])
+def test_long_selections_of_many_blocks(n: int, k: int) -> None:
+    from lazykv_amd import kernels
+
+    values, kmax, q = _metadata("normal", 2, n, n + k)
+    want = np.stack([np.sort(np.lexsort((np.arange(n), -values[j]))[:k]) for j in range(2)])
+    assert np.array_equal(kernels.bound_topk(q, kmax, kmax, k).cpu().numpy(), want)
