@@ -366,7 +366,6 @@ struct WaveState {
   float m[G];
   float l[G];
   float o[G][Lanes<D>::EPL];
-  float mh;  // matrix-core path: m of head lane % 16 (that lane's copy of m[lane % 16])
 };
 
 // Fold one chunk into the wave's running softmax. `limit`: valid tokens of this pair. Rows are
@@ -493,50 +492,6 @@ __device__ __forceinline__ void attend_two(const DecodeArgs& a, const Src& s, in
   process_two<D, MT, G, RawModel<D, MT>, NP>(a, s, block_a, block_b, h, limit, q, r, c, st);
 }
 
-// The selected pairs of an 8-wave int8 instance, four per wave per round: all four records' loads
-// are issued before the first is consumed (the HBM plan gives a wave about four), where the
-// two-per-round loop waits for a second round's loads after consuming its first two. The pairs and
-// the order they are consumed in are the two-per-round loop's, so the results are identical.
-// Blocks of at most 16 tokens (one chunk each). IDS_LDS: the ids are in LDS (a launch that selected
-// them itself), else in global memory; each is read through its own address space (a wait on a
-// generic read drains every load in flight).
-template <int D, int MT, int G, int NW, bool IDS_LDS>
-__device__ __forceinline__ void attend_selected_i8_four(const DecodeArgs& a, const int32_t* idx_h, int sel_base, int js, int je,
-                                                        int wave, int h, const float (&q)[G][Lanes<D>::EPL], int r, int c,
-                                                        WaveState<D, G>& st) {
-  using L = Lanes<D>;
-  const Src& s = a.sel;
-  const int nit = min(L::NI, (a.bs + L::RG - 1) / L::RG);
-  // No vector-memory write pending on entry or at the back edge (rows that no consumer reads, of
-  // the pairs attended before, included): the wait analysis otherwise orders each pair's loads
-  // behind the previous pair's. vmcnt(0), with expcnt and lgkmcnt left at their maximum.
-  __builtin_amdgcn_s_waitcnt(0x0F70);
-  for (int j = js + wave; j < je; j += 4 * NW) {
-    int b[4];
-    bool ok[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int jj = j + u * NW;
-      if constexpr (IDS_LDS) {
-        b[u] = jj < je ? ((const __attribute__((address_space(3))) int32_t*)idx_h)[jj - sel_base] : -1;
-      } else {
-        b[u] = jj < je ? *gmem<int32_t>(idx_h + (jj - sel_base)) : -1;
-      }
-      ok[u] = b[u] >= 0 && (int64_t)b[u] < s.nblk;
-    }
-    RawI8<D> w[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) load_pair_raw<D, MT>(s, a.bs, ok[u], b[u], h, 0, nit, a.bs, r, c, w[u]);
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (ok[u]) finish_raw(0, r, w[u]);  // wave-uniform branches: every lane shuffles
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (ok[u]) consume_chunk<D, G>(q, WidenI8<D, MT>(w[u]), w[u], 0, nit, a.bs, r, st);
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-  }
-}
-
 // ---- Q.K on the matrix cores ---------------------------------------------------------------------
 // The 8-wave model-dtype instances score a 16-token chunk with one v_mfma_f32_16x16x32 per 32
 // channels: A = the chunk's 16 key rows (lane l: row l % 16, channels 32s + 8 (l / 16) .. + 7),
@@ -562,11 +517,27 @@ struct Mfma<LKV_F16> {
   __device__ __forceinline__ static f32x4 mma(V8 a, V8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
 };
 
-// Floats of a wave's LDS broadcast area for up to NP pairs per step: p[NP][16][G], then the rows
-// m_new[G], alpha[G], psum[G].
+// Query heads in groups of 4: the rows of one v_mfma_f32_4x4x1_16b_f32. Columns past G hold head 0's query
+// times zero: their weights are finite and reach only accumulators that are never read.
+template <int G>
+constexpr int kHeadQuads = (G + 3) / 4;
+// Floats of a wave's LDS broadcast area for up to NP pairs per step: p[NP][16][heads], then the heads'
+// rescale factors.
 template <int G, int NP>
-constexpr int kMfBroadcast = (16 * NP + 3) * G;
-constexpr int kMfMaxPairs = 3;
+constexpr int kMfBroadcast = (16 * NP + 1) * 4 * kHeadQuads<G>;
+// Pairs of one step, all their loads in flight together, by what the registers hold (the accumulators of 8 heads
+// are 64 registers; a d 128 pair 32 as 16-bit rows, 56 as an int8 record).
+template <int D, int G, bool REC>
+constexpr int kMfPairs = REC ? (D == 64 && G <= 4 ? 4 : 2) : (G <= 4 ? 3 : 2);
+constexpr int kMfMaxPairs = 4;
+
+// A wave's running softmax on the matrix-core path: m and l of head lane % 16, and o of the lane's channels
+// over its rows, o[head / 4][channel][head % 4].
+template <int G>
+struct MfState {
+  float m, l;
+  f32x4 o[kHeadQuads<G>][8];
+};
 
 // The B operands: lane l holds channels 32s + 8 (l / 16) .. + 7 of query head l % 16 (the query
 // row is 16-byte aligned, which the launch checks).
@@ -589,8 +560,18 @@ struct RawMf {
   uint32_t v[Lanes<D>::NI][RawModel<D, MT>::W];
 };
 
+// The same of an int8 record: the codes in those layouts, with the key scales of the lane's channels and
+// the value scales of its rows.
+template <int D>
+struct RecMf {
+  u32x2 k[D / 32];
+  u32x4 ks[D / 32], kz[D / 32];  // float16
+  u32x2 v[Lanes<D>::NI];
+  uint16_t vs[Lanes<D>::NI], vz[Lanes<D>::NI];
+};
+
 template <int D, int MT>
-__device__ __forceinline__ void load_raw_mf(const Src& s, int block, int h, int t0, int nit, int limit, int lane, int r, int c,
+__device__ __forceinline__ void load_raw_mf(const Src& s, int, int block, int h, int t0, int nit, int limit, int lane, int r, int c,
                                             RawMf<D, MT>& raw) {
   using L = Lanes<D>;
   constexpr int EPL = L::EPL;
@@ -610,15 +591,85 @@ __device__ __forceinline__ void load_raw_mf(const Src& s, int block, int h, int 
   }
 }
 
+template <int D>
+__device__ __forceinline__ void load_raw_mf(const Src& s, int bs, int block, int h, int t0, int nit, int limit, int lane, int r, int c,
+                                            RecMf<D>& raw) {
+  using L = Lanes<D>;
+  const uint8_t* rec = (const uint8_t*)s.k + (int64_t)block * s.bstride + (int64_t)h * s.hstride;
+  const uint16_t* scales = (const uint16_t*)(rec + 2 * bs * D);
+  const int kr = t0 + lane % 16;
+  const uint8_t* krow = rec + (kr < limit ? kr : 0) * D + 8 * (lane / 16);
+#pragma unroll
+  for (int st = 0; st < D / 32; ++st) {
+    raw.k[st] = load_kv<u32x2>(krow + 32 * st);
+    raw.ks[st] = load_kv<u32x4>(scales + 32 * st + 8 * (lane / 16));
+    raw.kz[st] = load_kv<u32x4>(scales + D + 32 * st + 8 * (lane / 16));
+  }
+#pragma unroll
+  for (int i = 0; i < L::NI; ++i) {
+    const int row = t0 + r + L::RG * i;
+    const int at = i < nit && row < limit ? row : 0;
+    raw.v[i] = load_kv<u32x2>(rec + bs * D + at * D + c * L::EPL);
+    raw.vs[i] = load_kv<uint16_t>(scales + 2 * D + at);
+    raw.vz[i] = load_kv<uint16_t>(scales + 2 * D + bs + at);
+  }
+}
+
+// A value rounded to the model dtype, as the matrix cores take it (the hardware's conversions, to nearest even).
+template <int MT>
+struct MfElem;
+template <>
+struct MfElem<LKV_BF16> {
+  using T = __bf16;
+};
+template <>
+struct MfElem<LKV_F16> {
+  using T = _Float16;
+};
+
+template <int D, int MT>
+__device__ __forceinline__ typename Mfma<MT>::V8 key_frag(const RawMf<D, MT>& raw, int s) {
+  return raw.k[s];
+}
+template <int D, int MT>
+__device__ __forceinline__ typename Mfma<MT>::V8 key_frag(const RecMf<D>& raw, int s) {
+  using Wd = WidenI8<D, MT>;
+  const uint32_t w[2] = {raw.k[s].x, raw.k[s].y};
+  typename Mfma<MT>::V8 f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const uint32_t sw = raw.ks[s][e >> 1], zw = raw.kz[s][e >> 1];
+    const float sc = lkv::f16_to_f32((uint16_t)((e & 1) ? sw >> 16 : sw & 0xffffu)), ze = lkv::f16_to_f32((uint16_t)((e & 1) ? zw >> 16 : zw & 0xffffu));
+    f[e] = (typename MfElem<MT>::T)Wd::deq(Wd::u8(w, e), sc, ze);
+  }
+  return f;
+}
+template <int D, int MT>
+__device__ __forceinline__ void value_row(const RawMf<D, MT>& raw, int i, float (&x)[8]) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = Widen<D, MT>::elem(raw.v[i], e);
+}
+template <int D, int MT>
+__device__ __forceinline__ void value_row(const RecMf<D>& raw, int i, float (&x)[8]) {
+  using Wd = WidenI8<D, MT>;
+  const uint32_t w[2] = {raw.v[i].x, raw.v[i].y};
+  const float sc = lkv::f16_to_f32(raw.vs[i]), ze = lkv::f16_to_f32(raw.vz[i]);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = (float)(typename MfElem<MT>::T)Wd::deq(Wd::u8(w, e), sc, ze);
+}
+
 // Fold the same chunk (rows t0 .. t0 + 15) of NP pairs into the wave's running softmax, as
 // consume_chunk does one pair at a time, with the scores from the matrix cores: one maximum, one
 // rescale and one broadcast for all NP pairs. lim[u]: valid tokens of pair u (0 skips the pair).
-// `sp`: this wave's broadcast area.
-template <int D, int MT, int G, int NP>
-__device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D / 32], const RawMf<D, MT> (&raw)[NP], float qscale,
-                                           int t0, int nit, const int (&lim)[NP], int lane, int r, float* sp, WaveState<D, G>& st) {
+// `sp`: this wave's broadcast area. P.V runs as v_mfma_f32_4x4x1_16b_f32: 16 blocks of 4 lanes, each the
+// outer product of 4 heads' weights of the block's row (lane l: head l % 4) and its lanes' values, in
+// float32, one instruction where 4 heads took 4 fused multiply-adds, off the vector ALUs.
+template <int D, int MT, int G, int NP, typename Raw>
+__device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D / 32], const Raw (&raw)[NP], float qscale,
+                                           int t0, const int (&lim)[NP], int lane, int r, float* sp, MfState<G>& st) {
   using L = Lanes<D>;
-  constexpr int EPL = L::EPL;
+  static_assert(L::EPL == 8, "8 channels a lane");
+  constexpr int GQ = kHeadQuads<G>, GW = 4 * GQ;
   const int j = lane % 16, lg = lane / 16;
   f32x4 acc[NP];
 #pragma unroll
@@ -626,7 +677,7 @@ __device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D /
     acc[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     if (lim[u] > 0) {  // wave-uniform
 #pragma unroll
-      for (int s = 0; s < D / 32; ++s) acc[u] = Mfma<MT>::mma(raw[u].k[s], qb[s], acc[u]);
+      for (int s = 0; s < D / 32; ++s) acc[u] = Mfma<MT>::mma(key_frag<D, MT>(raw[u], s), qb[s], acc[u]);
     }
   }
   float sc[NP][4];
@@ -641,10 +692,10 @@ __device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D /
       cm = vld[u][i] ? fmaxf(cm, sc[u][i]) : cm;
     }
   cm = lkv::pair_max<32>(lkv::pair_max<16>(cm));
-  const float m_old = st.mh;
+  const float m_old = st.m;
   const float m_new = fmaxf(m_old, cm);
   const bool live = m_new != -INFINITY;  // false while nothing valid has been seen
-  const float alpha = live ? exp2f(m_old - m_new) : 1.0f;
+  const float alpha = m_old != -INFINITY ? exp2f(m_old - m_new) : 1.0f;  // nothing to rescale before the first valid chunk
   float p[NP][4];
   float ps = 0.0f;
 #pragma unroll
@@ -655,49 +706,52 @@ __device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D /
       ps += p[u][i];
     }
   ps = lkv::pair_sum<32>(lkv::pair_sum<16>(ps));
-  st.mh = live ? m_new : m_old;
-  if (j < G) {
+  st.m = m_new;
+  st.l = st.l * alpha + ps;
+  const bool rescale = __ballot(j < G && alpha != 1.0f) != 0;  // some head's maximum moved
+  if (j < GW) {
 #pragma unroll
     for (int u = 0; u < NP; ++u)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) sp[(16 * u + 4 * lg + i) * G + j] = p[u][i];
-    if (lg == 0) {
-      sp[(16 * NP) * G + j] = m_new;
-      sp[(16 * NP + 1) * G + j] = alpha;
-      sp[(16 * NP + 2) * G + j] = ps;
-    }
+      for (int i = 0; i < 4; ++i) sp[(16 * u + 4 * lg + i) * GW + j] = p[u][i];
+    if (rescale && lg == 0) sp[16 * NP * GW + j] = alpha;
   }
   // LDS operations of one wave complete in order: the wave's reads below see its writes above.
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if (rescale) {
 #pragma unroll
-  for (int jj = 0; jj < G; ++jj) {
-    const float mn = sp[(16 * NP) * G + jj], al = sp[(16 * NP + 1) * G + jj], pj = sp[(16 * NP + 2) * G + jj];
-    if (mn != -INFINITY) {
-      st.m[jj] = mn;
-      st.l[jj] = st.l[jj] * al + (r == 0 ? pj : 0.0f);  // the step's sum counts once over the row groups
+    for (int g = 0; g < GQ; ++g) {
+      const f32x4 al = *(const f32x4*)(sp + 16 * NP * GW + 4 * g);
 #pragma unroll
-      for (int e = 0; e < EPL; ++e) st.o[jj][e] *= al;
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) st.o[g][e][jj] *= al[jj];
     }
   }
 #pragma unroll
-  for (int u = 0; u < NP; ++u)
+  for (int u = 0; u < NP; ++u) {
+    if (lim[u] <= 0) continue;                // wave-uniform, as the next test
+    const bool part = t0 + 16 > lim[u];       // rows past the limit may hold non-finite data
 #pragma unroll
     for (int i = 0; i < L::NI; ++i) {
       const int row = r + L::RG * i;
-      if (!(i < nit && t0 + row < lim[u])) continue;  // masked rows may hold non-finite data
-      float pr[G];
+      float x[8];
+      value_row<D, MT>(raw[u], i, x);
+      if (part) {
+        const bool ok = t0 + row < lim[u];
 #pragma unroll
-      for (int jj = 0; jj < G; ++jj) pr[jj] = sp[(16 * u + row) * G + jj];
-      float x[EPL];
+        for (int e = 0; e < 8; ++e) x[e] = ok ? x[e] : 0.0f;  // their weights are 0
+      }
 #pragma unroll
-      for (int e = 0; e < EPL; ++e) x[e] = Widen<D, MT>::elem(raw[u].v[i], e);
+      for (int g = 0; g < GQ; ++g) {
+        const float pr = sp[(16 * u + row) * GW + 4 * g + (lane & 3)];
 #pragma unroll
-      for (int jj = 0; jj < G; ++jj)
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) st.o[jj][e] = fmaf(pr[jj], x[e], st.o[jj][e]);
+        for (int e = 0; e < 8; ++e) st.o[g][e] = __builtin_amdgcn_mfma_f32_4x4x1f32(pr, x[e], st.o[g][e], 0, 0, 0);
+      }
     }
+  }
   // The next step rewrites the area only after these reads (in order, as above).
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -732,13 +786,13 @@ __device__ __forceinline__ void segment_items(const DecodeArgs& a, const int32_t
   }
 }
 
-// Up to NP pairs on the matrix cores, each of its own source and valid-token limit: every pair's
-// loads are issued before any is consumed, and they are consumed in item order. Ids outside their
-// source are skipped (wave-uniform), never read.
-template <int D, int MT, int G, int NP>
+// Up to NP pairs on the matrix cores, each of its own source and valid-token limit (Raw: 16-bit pairs or
+// int8 records): every pair's loads are issued before any is consumed, and they are consumed in item
+// order. Ids outside their source are skipped (wave-uniform), never read.
+template <int D, int MT, int G, typename Raw, int NP>
 __device__ __forceinline__ void process_items_mf(const DecodeArgs& a, const Src (&s)[NP], const int (&blk)[NP], const int (&lim)[NP],
                                                  int h, const typename Mfma<MT>::V8 (&qb)[D / 32], int lane, int r, int c, float* sp,
-                                                 WaveState<D, G>& st) {
+                                                 MfState<G>& st) {
   bool ok[NP];
 #pragma unroll
   for (int u = 0; u < NP; ++u) ok[u] = blk[u] >= 0 && (int64_t)blk[u] < s[u].nblk;
@@ -772,11 +826,57 @@ __device__ __forceinline__ void process_items_mf(const DecodeArgs& a, const Src 
 #pragma unroll 1
   for (int t0 = 0; t0 < a.bs; t0 += 16) {
     const int nit = min(Lanes<D>::NI, (a.bs - t0 + Lanes<D>::RG - 1) / Lanes<D>::RG);
-    RawMf<D, MT> raw[NP];
+    Raw raw[NP];
 #pragma unroll
-    for (int u = 0; u < NP; ++u) load_raw_mf<D, MT>(ls[u], lb[u], h, t0, nit, ll[u], lane, r, c, raw[u]);
+    for (int u = 0; u < NP; ++u) load_raw_mf(ls[u], a.bs, lb[u], h, t0, nit, ll[u], lane, r, c, raw[u]);
     __builtin_amdgcn_sched_barrier(0);  // every load above issues before the first use below
-    consume_mf<D, MT, G, NP>(qb, raw, a.qscale, t0, nit, lk, lane, r, sp, st);
+    consume_mf<D, MT, G, NP>(qb, raw, a.qscale, t0, lk, lane, r, sp, st);
+  }
+}
+
+// Selected items j, j + NW, .. < je of the launch's selection (ids at idx_h[j - base]).
+template <int D, int MT, int G, typename Raw, int NW>
+__device__ __forceinline__ void attend_run_mf(const DecodeArgs& a, const int32_t* idx_h, int base, int j, int je, int h,
+                                              const typename Mfma<MT>::V8 (&qb)[D / 32], int lane, int r, int c, float* sp, MfState<G>& st) {
+  constexpr int NP = kMfPairs<D, G, std::is_same<Raw, RecMf<D>>::value>;
+  Src s[NP];
+  int lim[NP];
+#pragma unroll
+  for (int u = 0; u < NP; ++u) {
+    s[u] = a.sel;
+    lim[u] = a.bs;
+  }
+  for (; j < je; j += NP * NW) {
+    int blk[NP];
+#pragma unroll
+    for (int u = 0; u < NP; ++u) blk[u] = j + u * NW < je ? __builtin_amdgcn_readfirstlane(idx_h[j + u * NW - base]) : -1;
+    process_items_mf<D, MT, G, Raw, NP>(a, s, blk, lim, h, qb, lane, r, c, sp, st);
+  }
+}
+
+// Remainder blocks b, b + NW, .. < hi whose bit (b - lo) of `excl` is clear, several per step, folded into the
+// softmax together.
+template <int D, int MT, int G, typename Raw, int NW>
+__device__ __forceinline__ void attend_rest_mf(const DecodeArgs& a, const uint32_t* excl, int lo, int b, int hi, int h,
+                                               const typename Mfma<MT>::V8 (&qb)[D / 32], int lane, int r, int c, float* sp, MfState<G>& st) {
+  constexpr int NP = kMfPairs<D, G, std::is_same<Raw, RecMf<D>>::value>;
+  Src s[NP];
+  int lim[NP];
+#pragma unroll
+  for (int u = 0; u < NP; ++u) {
+    s[u] = a.rem;
+    lim[u] = a.bs;
+  }
+  while (b < hi) {
+    int pick[NP];
+#pragma unroll
+    for (int u = 0; u < NP; ++u) pick[u] = -1;
+    int have = 0;
+    while (have < NP && b < hi) {
+      if (!((excl[(b - lo) >> 5] >> ((b - lo) & 31)) & 1u)) pick[have++] = b;
+      b += NW;
+    }
+    if (have) process_items_mf<D, MT, G, Raw, NP>(a, s, pick, lim, h, qb, lane, r, c, sp, st);
   }
 }
 
@@ -955,7 +1055,8 @@ constexpr int kFuseKeysPerThread = 16;  // a decode launch selects inside itself
 template <int NT, int SEL>
 constexpr int kSelKpt = SEL * kSelUnit / NT;
 
-// MF: Q.K on the matrix cores (model-dtype instances whose query has the model dtype).
+// MF: Q.K and P.V on the matrix cores (instances whose query has the model dtype; with I8, for launches that
+// read int8 records).
 // SEL > 0: the launch selects each head's top k from its bounds itself (segment A only), from up
 // to SEL * kSelUnit candidates.
 template <int D, int MT, int G, int NT, bool I8, bool MF = false, int SEL = 0>
@@ -972,8 +1073,8 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
   __shared__ float s_m[NW][G], s_l[NW][G];
   __shared__ __align__(16) float s_o[NW][G][D];
   __shared__ uint32_t s_excl[64];  // segment B: bitmap of excluded blocks in this run
-  static_assert(!MF || (!I8 && MT != LKV_F32), "the matrix-core path reads model-dtype pairs");
-  __shared__ float s_pb[MF ? NW : 1][MF ? kMfBroadcast<G, kMfMaxPairs> : 1];
+  static_assert(!MF || MT != LKV_F32, "the matrix-core path reads 16-bit pairs and int8 records");
+  __shared__ __align__(16) float s_pb[MF ? NW : 1][MF ? kMfBroadcast<G, I8 ? kMfMaxPairs : 3> : 4];
   using SelLds = typename std::conditional<(SEL > 0), lkv::SelectLds<NT, kSelKpt<NT, (SEL > 0 ? SEL : 1)>>, char>::type;
   __shared__ SelLds s_sel;
   using V8 = typename Mfma<MT == LKV_F32 ? LKV_F16 : MT>::V8;
@@ -984,11 +1085,13 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
   float* sp = s_pb[MF ? wave : 0];
 
   float q[G][EPL];
-  lkv::load_query_rows<D, G, EPL>(a.q, a.q_dtype, h, c, q);
+  if constexpr (!MF) {
+    lkv::load_query_rows<D, G, EPL>(a.q, a.q_dtype, h, c, q);
 #pragma unroll
-  for (int j = 0; j < G; ++j)
+    for (int j = 0; j < G; ++j)
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) q[j][e] *= a.qscale;
+      for (int e = 0; e < EPL; ++e) q[j][e] *= a.qscale;
+  }
 
   // ---- fused selection: this head's top k, and the ids of this workgroup's run -----------------
   // The run's selected ids go to LDS (over the histogram, free once the selection is done), as
@@ -1021,14 +1124,22 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
     sel_base = js;
   }
 
-  WaveState<D, G> st;
-  st.mh = -INFINITY;
+  typename std::conditional<MF, MfState<G>, WaveState<D, G>>::type st;
+  if constexpr (MF) {
+    st.m = -INFINITY;
+    st.l = 0.0f;
 #pragma unroll
-  for (int j = 0; j < G; ++j) {
-    st.m[j] = -INFINITY;
-    st.l[j] = 0.0f;
+    for (int g = 0; g < kHeadQuads<G>; ++g)
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) st.o[j][e] = 0.0f;
+      for (int e = 0; e < 8; ++e) st.o[g][e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  } else {
+#pragma unroll
+    for (int j = 0; j < G; ++j) {
+      st.m[j] = -INFINITY;
+      st.l[j] = 0.0f;
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) st.o[j][e] = 0.0f;
+    }
   }
 
   if (split < a.splits_a) {
@@ -1037,18 +1148,36 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
     const int last = min(a.n_a, first + a.per_a);
     const int has_sink = a.sink_block >= 0;
     const int n_sel = a.attend_selected ? a.k : 0;
-    if constexpr (MF) {
-      // Every item of the run -- the sink, selected ids, the current block -- is a model-dtype
-      // pair, so each wave takes kMfItems of them per round, all loads in flight together: with
+    if constexpr (MF && I8) {
+      // The sink and the current block are 16-bit pairs, one wave each; the selected items int8 records (or,
+      // beside an int8 remainder, 16-bit pairs), kMfPairs of them per wave and round.
+      const int wv = __builtin_amdgcn_readfirstlane(wave);
+      const int js = max(first, has_sink) - has_sink;
+      const int je = min(last, has_sink + n_sel) - has_sink;
+      if (a.sel.dtype == LKV_INT8_RECORD) {
+        attend_run_mf<D, MT, G, RecMf<D>, NW>(a, idx_h, sel_base, js + wv, je, h, qb, lane, r, c, sp, st);
+      } else {
+        attend_run_mf<D, MT, G, RawMf<D, MT>, NW>(a, idx_h, sel_base, js + wv, je, h, qb, lane, r, c, sp, st);
+      }
+      const bool mine_sink = has_sink && first == 0 && wv == NW - 1, mine_cur = a.cur_block >= 0 && last == a.n_a && wv == NW - 1;
+      if (mine_sink || mine_cur) {  // the wave with the fewest selected items, both pairs at once in a short run
+        const Src es[2] = {a.sink, a.cur};
+        const int eb[2] = {mine_sink ? a.sink_block : -1, mine_cur ? a.cur_block : -1};
+        const int el[2] = {a.bs, a.fill};
+        process_items_mf<D, MT, G, RawMf<D, MT>, 2>(a, es, eb, el, h, qb, lane, r, c, sp, st);
+      }
+    } else if constexpr (MF) {
+      // Every item of the run -- the sink, selected ids, the current block -- is a 16-bit
+      // pair, so each wave takes kMfPairs of them per round, all loads in flight together: with
       // about two items per wave in the HBM plan, the wave that holds a third needs no second
       // round.
-      constexpr int kMfItems = kMfMaxPairs;
+      constexpr int kMfItems = kMfPairs<D, G, false>;
       const int wv = __builtin_amdgcn_readfirstlane(wave);
       for (int j0 = first + wv; j0 < last; j0 += kMfItems * NW) {
         Src is[kMfItems];
         int ib[kMfItems], il[kMfItems];
         segment_items<kMfItems, NW>(a, idx_h, sel_base, j0, last, is, ib, il);
-        process_items_mf<D, MT, G, kMfItems>(a, is, ib, il, h, qb, lane, r, c, sp, st);
+        process_items_mf<D, MT, G, RawMf<D, MT>, kMfItems>(a, is, ib, il, h, qb, lane, r, c, sp, st);
       }
     } else {
       if (has_sink && first == 0 && wave == 0) attend_two<D, MT, G, I8>(a, a.sink, a.sink_block, -1, h, a.bs, q, r, c, st);
@@ -1058,22 +1187,14 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
       const int js = max(first, has_sink) - has_sink;
       const int je = min(last, has_sink + n_sel) - has_sink;
       // The hybrid branch is compiled only into the 4-wave general instance, which every hybrid
-      // launch takes. The 8-wave vector-path instances keep two selected pairs in flight per wave
-      // (int8 records in HBM 24.4 -> 23.5 us, identical results), and int8 records of blocks of
-      // at most 16 tokens four (attend_selected_i8_four), in the same order. Float32 pools keep
-      // one (two would spill).
+      // launch takes. The 8-wave vector-path instances keep two selected pairs in flight per wave;
+      // float32 pools keep one (two would spill).
       // A fused-selection instance keeps the pairing of the instance it stands in for, so that both
       // fold each wave's chunks in the same order (with two pairs in flight a wave interleaves their
       // 16-row chunks).
       constexpr bool HYB = I8 && NT == kThreads && SEL == 0;
       constexpr int NPA = ((I8 && NT == kThreads) || MT == LKV_F32) ? 1 : 2;
       bool piped = false;  // the selected pairs were attended by a pipelined loop
-      if constexpr (I8 && NT == kThreadsHbm && NPA == 2) {
-        if (a.sel.dtype == LKV_INT8_RECORD && a.bs <= 16) {
-          attend_selected_i8_four<D, MT, G, NW, (SEL > 0)>(a, idx_h, sel_base, js, je, wave, h, q, r, c, st);
-          piped = true;
-        }
-      }
       if constexpr (HYB) {
         if (a.loc != nullptr && a.sel.dtype != LKV_INT8_RECORD && a.bs <= 16) {
           attend_hybrid_piped<D, MT, G, NW>(a, idx_h, sel_base, js, je, wave, h, q, r, c, st);
@@ -1119,26 +1240,14 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
     }
     __syncthreads();
     int b = lo + wave;
-    if constexpr (MF) {
-      // Up to kMfMaxPairs blocks per step, folded into the softmax together.
-      Src rs[kMfMaxPairs];
-      int lim[kMfMaxPairs];
-#pragma unroll
-      for (int u = 0; u < kMfMaxPairs; ++u) {
-        rs[u] = a.rem;
-        lim[u] = a.bs;
+    if constexpr (MF && I8) {
+      if (a.rem.dtype == LKV_INT8_RECORD) {
+        attend_rest_mf<D, MT, G, RecMf<D>, NW>(a, s_excl, lo, b, hi, h, qb, lane, r, c, sp, st);
+      } else {
+        attend_rest_mf<D, MT, G, RawMf<D, MT>, NW>(a, s_excl, lo, b, hi, h, qb, lane, r, c, sp, st);
       }
-      while (b < hi) {
-        int pick[kMfMaxPairs];
-#pragma unroll
-        for (int u = 0; u < kMfMaxPairs; ++u) pick[u] = -1;
-        int have = 0;
-        while (have < kMfMaxPairs && b < hi) {
-          if (!((s_excl[(b - lo) >> 5] >> ((b - lo) & 31)) & 1u)) pick[have++] = b;
-          b += NW;
-        }
-        if (have) process_items_mf<D, MT, G, kMfMaxPairs>(a, rs, pick, lim, h, qb, lane, r, c, sp, st);
-      }
+    } else if constexpr (MF) {
+      attend_rest_mf<D, MT, G, RawMf<D, MT>, NW>(a, s_excl, lo, b, hi, h, qb, lane, r, c, sp, st);
     } else {
       while (b < hi) {
         int pick[2] = {-1, -1};
@@ -1153,15 +1262,28 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
   }
 
   // ---- wave totals: sum the four row groups, then combine the waves in LDS ---------------------
-#pragma unroll
-  for (int j = 0; j < G; ++j) {
-    const float l = lkv::groups_sum<L::RG>(st.l[j]);
-    if (lane == 0) {
-      s_m[wave][j] = st.m[j];
-      s_l[wave][j] = l;
+  if constexpr (MF) {
+    if (lane < G) {  // head `lane`
+      s_m[wave][lane] = st.m;
+      s_l[wave][lane] = st.l;
     }
+    float o[G][EPL];
+#pragma unroll
+    for (int j = 0; j < G; ++j)
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) o[j][e] = st.o[j / 4][e][j % 4];
+    scatter_totals<D, G>(o, lane, &s_o[wave][0][0]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < G; ++j) {
+      const float l = lkv::groups_sum<L::RG>(st.l[j]);
+      if (lane == 0) {
+        s_m[wave][j] = st.m[j];
+        s_l[wave][j] = l;
+      }
+    }
+    scatter_totals<D, G>(st.o, lane, &s_o[wave][0][0]);
   }
-  scatter_totals<D, G>(st.o, lane, &s_o[wave][0][0]);
   __syncthreads();
   float* pml = a.part_ml + ((int64_t)h * S + split) * G * 2;
   float* po = a.part_o + ((int64_t)h * S + split) * G * D;
@@ -1350,11 +1472,10 @@ static Plan make_plan(const lkv_decode_desc* d, const PlanHints& hint = PlanHint
   if (p.per_b > 2048) p.per_b = 2048;  // the exclusion bitmap holds 2048 blocks
   p.splits_b = n_b > 0 ? (n_b + p.per_b - 1) / p.per_b : 0;
   const int n_sel = d->attend_selected ? d->k : 0;
-  if (cus > 0 && !hint.sel_host && !hint.rem_host && d->n_q / d->n_kv <= 4) {
+  if (cus > 0 && !hint.sel_host && !hint.rem_host) {
     // Everything in HBM: 8-wave workgroups, about one per CU for the gathered set (measured at
     // the 8B shape: 17.8 us against 20.2 us for 58 four-wave workgroups per head, which leave a
-    // tail of CUs with two), at least one pair per wave. (Groups of 8 query heads need more
-    // registers than an 8-wave workgroup leaves a wave, and keep the 4-wave shape.)
+    // tail of CUs with two), at least one pair per wave.
     p.nt = kThreadsHbm;
     const int per_head = cus / d->n_kv > 1 ? cus / d->n_kv : 1;
     p.per_a = (p.n_a + per_head - 1) / per_head;
@@ -1395,25 +1516,21 @@ static Plan make_plan(const lkv_decode_desc* d, const PlanHints& hint = PlanHint
   return p;
 }
 
-// The kernel instance a launch takes. HBM plans (a.nt == kThreadsHbm, G <= 4) run 8-wave
-// workgroups: matrix-core scoring when the query has the model dtype and 16-byte aligned rows, the
-// vector path otherwise, int8-capable when a source is int8 records (except D 128 with G 4, which
-// spills there and takes the 4-wave instance over the same plan). Host plans, hybrid launches and
-// groups of 8 take the 4-wave general instance. A fused-selection launch has no 8-wave vector
-// instance and takes the general one instead (lkv_select_decode then selects in its own launch, so
-// that it folds what the unfused call folds).
-enum class Inst { kGeneral, kVector8, kInt8x8, kMatrix8 };
+// The kernel instance a launch takes. HBM plans (a.nt == kThreadsHbm) run 8-wave workgroups on the matrix cores
+// when the query has the model dtype and 16-byte aligned rows: one instance for 16-bit pairs, one that also
+// reads int8 records. Other queries (and float32 pools) take the 8-wave vector path for 16-bit and
+// float32 pairs of groups of up to 4 heads, and the 4-wave general instance over the same plan for the rest.
+// Host plans and hybrid launches take the 4-wave general instance. A fused-selection launch has
+// no 8-wave vector instance and takes the general one instead (lkv_select_decode then selects in its own
+// launch, so that it folds what the unfused call folds).
+enum class Inst { kGeneral, kVector8, kMatrix8, kMatrixRec8 };
 
-static Inst pick_instance(const DecodeArgs& a, int D, int MT, int G, bool sel) {
+static Inst pick_instance(const DecodeArgs& a, int MT, int G, bool sel) {
   const bool i8 = a.sel.dtype == LKV_INT8_RECORD || a.rem.dtype == LKV_INT8_RECORD || a.sink.dtype == LKV_INT8_RECORD ||
                   a.cur.dtype == LKV_INT8_RECORD || a.loc != nullptr;
-  if (G > 4 || a.nt != kThreadsHbm || a.loc != nullptr) return Inst::kGeneral;
-  if (!i8) {
-    const bool mf = MT != LKV_F32 && a.q_dtype == MT && ((uintptr_t)a.q & 15u) == 0;
-    if (mf) return Inst::kMatrix8;
-    return sel ? Inst::kGeneral : Inst::kVector8;
-  }
-  return (D == 128 && G == 4) ? Inst::kGeneral : Inst::kInt8x8;
+  if (a.nt != kThreadsHbm || a.loc != nullptr) return Inst::kGeneral;
+  if (MT != LKV_F32 && a.q_dtype == MT && ((uintptr_t)a.q & 15u) == 0) return i8 ? Inst::kMatrixRec8 : Inst::kMatrix8;
+  return i8 || sel || G > 4 ? Inst::kGeneral : Inst::kVector8;
 }
 
 // Threads per workgroup of an instance.
@@ -1423,21 +1540,19 @@ template <int D, int MT, int G, int SEL>
 int launch_inst(hipStream_t stream, DecodeArgs& a, Inst inst) {
   const dim3 grid((a.splits_a + a.splits_b) * a.n_kv);
   bool done = false;
-  if constexpr (MT != LKV_F32 && G <= 4) {
+  if constexpr (MT != LKV_F32) {
     if (inst == Inst::kMatrix8) {
       hipLaunchKernelGGL((sparse_decode_kernel<D, MT, G, kThreadsHbm, false, true, SEL>), grid, dim3(kThreadsHbm), 0, stream, a);
+      done = true;
+    }
+    if (inst == Inst::kMatrixRec8) {
+      hipLaunchKernelGGL((sparse_decode_kernel<D, MT, G, kThreadsHbm, true, true, SEL>), grid, dim3(kThreadsHbm), 0, stream, a);
       done = true;
     }
   }
   if constexpr (G <= 4 && SEL == 0) {
     if (inst == Inst::kVector8) {
       hipLaunchKernelGGL((sparse_decode_kernel<D, MT, G, kThreadsHbm, false>), grid, dim3(kThreadsHbm), 0, stream, a);
-      done = true;
-    }
-  }
-  if constexpr (G <= 4 && !(D == 128 && G == 4)) {
-    if (inst == Inst::kInt8x8) {
-      hipLaunchKernelGGL((sparse_decode_kernel<D, MT, G, kThreadsHbm, true, false, SEL>), grid, dim3(kThreadsHbm), 0, stream, a);
       done = true;
     }
   }
@@ -1455,10 +1570,7 @@ template <int D, int MT, int G>
 int launch(hipStream_t stream, DecodeArgs& a) {
   const bool sel = a.bounds != nullptr;
   const int S = a.splits_a + a.splits_b;
-  Inst inst = pick_instance(a, D, MT, G, sel);
-  if ((inst == Inst::kMatrix8 && (MT == LKV_F32 || G > 4)) || (inst == Inst::kInt8x8 && (G > 4 || (D == 128 && G == 4))) ||
-      (inst == Inst::kVector8 && (G > 4 || sel)))
-    inst = Inst::kGeneral;  // no such instance (pick_instance never asks for one)
+  const Inst inst = pick_instance(a, MT, G, sel);
   const int rc = !sel                          ? launch_inst<D, MT, G, 0>(stream, a, inst)
                  : a.n_cand <= kSelUnit     ? launch_inst<D, MT, G, 1>(stream, a, inst)
                  : a.n_cand <= 2 * kSelUnit ? launch_inst<D, MT, G, 2>(stream, a, inst)
@@ -1964,8 +2076,8 @@ static int sparse_decode_impl(uintptr_t stream, const lkv_decode_desc* desc, con
   // kFuseKeysPerThread of the head's candidates; otherwise the selection takes a launch of its own.
   bool select_in_decode = false;
   if (fsel != nullptr && fsel->in_decode) {
-    const Inst fused = pick_instance(a, d.head_dim, mt, G, true);
-    select_in_decode = fused == pick_instance(a, d.head_dim, mt, G, false) && fsel->n_cand <= kFuseKeysPerThread * inst_threads(fused);
+    const Inst fused = pick_instance(a, mt, G, true);
+    select_in_decode = fused == pick_instance(a, mt, G, false) && fsel->n_cand <= kFuseKeysPerThread * inst_threads(fused);
   }
   if (fsel != nullptr) {
     // A remainder excludes the selected ids, so they must exist before the decode launch: chosen by

@@ -276,10 +276,12 @@ static bool rows_vector_readable(const float* bounds, int64_t bstride, int n_can
 // context took 155 us, nearly all of it in seven passes of strided 4-byte reads.) The k-th best
 // candidate (key, index) is found as block_top_k does (lkv_blockselect.h): a first range that starts at
 // the least of the lanes' own largest keys, histograms of the live range, and a boundary bin of at most
-// 64 keys ranked by every wave. One more pass writes the picks in index order; in sorted mode they are
-// gathered in LDS and sorted, each thread holding one or two in registers: only partners in other waves
-// go through LDS, 10 of the 55 steps for 1,024 picks, and the others are lane exchanges. With the bound launch, 1,024 of 65,535 in descending order: 176.0 -> 51.1 us (head_dim 64), 2,047
-// of 262,144: 654 -> 151; what is left is one CU's vector work per head, three passes over its row.
+// 64 keys ranked directly. The pass that lists that bin also gathers the keys above it, so a selection reads
+// the row three times. In ascending mode the picks are bits of a map of the candidates, read in order;
+// in sorted mode they are gathered in LDS and sorted, each thread holding one or two in registers:
+// only partners in other waves go through LDS, 10 of the 55 steps for 1,024 picks, and the others are lane
+// exchanges. With the bound launch, 1,024 of 65,535 in descending order: 176.0 -> 51.1 us (head_dim 64), 2,048
+// of 262,144: 654 -> 152. What is left is one CU's vector work per head over three passes.
 constexpr int kMaxStreamCand = 1 << 18;  // 262,144 candidates per head: 4M tokens at 16-token blocks
 
 // f(i, keys of candidates i .. i + 3, how many of them exist) over [begin, end), 256 candidates a call.
