@@ -263,14 +263,6 @@ __device__ __forceinline__ float row16_max(float x) {
   return x;
 }
 
-__device__ __forceinline__ float row16_min(float x) {
-  x = fminf(x, dpp<kDppQuadSwap1>(x));
-  x = fminf(x, dpp<kDppQuadSwap2>(x));
-  x = fminf(x, dpp<kDppHalfMirror>(x));
-  x = fminf(x, dpp<kDppMirror>(x));
-  return x;
-}
-
 // Sum over the LPR lanes of a row (16 or 8); every lane of the row receives the total.
 template <int LPR>
 __device__ __forceinline__ float row_sum(float x) {
@@ -279,6 +271,26 @@ __device__ __forceinline__ float row_sum(float x) {
   x += dpp<kDppQuadSwap2>(x);
   x += dpp<kDppHalfMirror>(x);
   if constexpr (LPR == 16) x += dpp<kDppMirror>(x);
+  return x;
+}
+
+// Minimum / maximum over the LPR lanes of a row (16 or 8), in every lane of the row.
+template <int LPR>
+__device__ __forceinline__ float row_min(float x) {
+  static_assert(LPR == 16 || LPR == 8, "rows are 16 or 8 lanes wide");
+  x = fminf(x, dpp<kDppQuadSwap1>(x));
+  x = fminf(x, dpp<kDppQuadSwap2>(x));
+  x = fminf(x, dpp<kDppHalfMirror>(x));
+  if constexpr (LPR == 16) x = fminf(x, dpp<kDppMirror>(x));
+  return x;
+}
+template <int LPR>
+__device__ __forceinline__ float row_max(float x) {
+  static_assert(LPR == 16 || LPR == 8, "rows are 16 or 8 lanes wide");
+  x = fmaxf(x, dpp<kDppQuadSwap1>(x));
+  x = fmaxf(x, dpp<kDppQuadSwap2>(x));
+  x = fmaxf(x, dpp<kDppHalfMirror>(x));
+  if constexpr (LPR == 16) x = fmaxf(x, dpp<kDppMirror>(x));
   return x;
 }
 
@@ -331,6 +343,12 @@ __device__ __forceinline__ float pair_sum(float x) {
   float a, b;
   lane_pair<M>(x, a, b);
   return a + b;
+}
+template <int M>
+__device__ __forceinline__ float pair_min(float x) {
+  float a, b;
+  lane_pair<M>(x, a, b);
+  return fminf(a, b);
 }
 template <int M>
 __device__ __forceinline__ float pair_max(float x) {
@@ -455,6 +473,13 @@ __device__ __forceinline__ float groups_sum(float x) {
   if constexpr (RG == 8) x = pair_sum<8>(x);
   x = pair_sum<16>(x);
   return pair_sum<32>(x);
+}
+template <int RG>
+__device__ __forceinline__ float groups_min(float x) {
+  static_assert(RG == 4 || RG == 8, "rows of 16 or 8 lanes");
+  if constexpr (RG == 8) x = pair_min<8>(x);
+  x = pair_min<16>(x);
+  return pair_min<32>(x);
 }
 template <int RG>
 __device__ __forceinline__ float groups_max(float x) {

@@ -39,16 +39,11 @@ struct StoreArgs {
   void* kmin;
   void* kmax;
   int meta_dtype;
+  int meta_words;  // metadata rows of the source's 16-bit dtype, at whole 32-bit words
   int64_t meta_hstride;
 };
 
 __device__ __forceinline__ float f16_round(float x) { return lkv::f16_to_f32(lkv::f32_to_f16(x)); }
-
-__device__ __forceinline__ int8_t quantise(float x, float mn, float scale) {
-  float t = rintf((x - mn) / scale);
-  t = fminf(fmaxf(t, 0.0f), 255.0f);
-  return (int8_t)(int)(t - 128.0f);
-}
 
 template <int MT, int EPL>
 __device__ __forceinline__ void store_segment(typename lkv::Elem<MT>::T* p, const float (&x)[EPL]) {
@@ -77,19 +72,6 @@ __device__ __forceinline__ void store_segment(typename lkv::Elem<MT>::T* p, cons
 }
 
 template <int EPL>
-__device__ __forceinline__ void store_bytes(int8_t* p, const int8_t (&b)[EPL]) {
-  if constexpr (EPL == 8) {
-    uint2 w;
-    __builtin_memcpy(&w, b, 8);
-    *(uint2*)p = w;
-  } else {
-    uint32_t w;
-    __builtin_memcpy(&w, b, 4);
-    *(uint32_t*)p = w;
-  }
-}
-
-template <int EPL>
 __device__ __forceinline__ void load_bytes(const int8_t* p, int8_t (&b)[EPL]) {
   if constexpr (EPL == 8) {
     uint2 w = *(const uint2*)p;
@@ -112,8 +94,10 @@ __device__ __forceinline__ void write_meta(const StoreArgs& a, int b, int h, int
   }
 }
 
+// Sources that are int8 records: 16 lanes hold a row.
 template <int D, int MT, int MODE>
-__device__ __forceinline__ void store_pair(const StoreArgs& a, int64_t pair) {
+__device__ __forceinline__ void store_record(const StoreArgs& a, int64_t pair) {
+  static_assert(MODE == MODE_META_FROM_I8 || MODE == MODE_UNPACK, "reads records");
   using T = typename lkv::Elem<MT>::T;
   constexpr int EPL = D / 16;
   const int lane = threadIdx.x & 63;
@@ -124,162 +108,328 @@ __device__ __forceinline__ void store_pair(const StoreArgs& a, int64_t pair) {
   const int rows = bs >> 2;  // rows per row group
   const bool want_meta = a.kmin != nullptr;
 
-  if constexpr (MODE == MODE_META_FROM_I8 || MODE == MODE_UNPACK) {
-    // An existing record: the metadata of its dequantised keys and, for MODE_UNPACK, the pair
-    // itself dequantised into dst (quant.py:103-105: ((q + 128) * scale) + zero, two separately
-    // rounded float32 operations, then the model dtype).
-    const uint8_t* rec = (const uint8_t*)a.sk + (int64_t)b * a.s_bstride + (int64_t)h * a.s_hstride;
-    const uint16_t* sc = (const uint16_t*)(rec + 2 * bs * D);
-    T* dk = nullptr;
-    T* dv = nullptr;
+  // An existing record: the metadata of its dequantised keys and, for MODE_UNPACK, the pair
+  // itself dequantised into dst (quant.py:103-105: ((q + 128) * scale) + zero, two separately
+  // rounded float32 operations, then the model dtype).
+  const uint8_t* rec = (const uint8_t*)a.sk + (int64_t)b * a.s_bstride + (int64_t)h * a.s_hstride;
+  const uint16_t* sc = (const uint16_t*)(rec + 2 * bs * D);
+  T* dk = nullptr;
+  T* dv = nullptr;
+  if constexpr (MODE == MODE_UNPACK) {
+    const int64_t doff = (int64_t)b * a.d_bstride + (int64_t)h * a.d_hstride + c * EPL;
+    dk = (T*)a.dk + doff;
+    dv = (T*)a.dv + doff;
+  }
+  float ks[EPL], kz[EPL], mn[EPL], mx[EPL];
+#pragma unroll
+  for (int e = 0; e < EPL; ++e) {
+    ks[e] = lkv::f16_to_f32(sc[c * EPL + e]);
+    kz[e] = lkv::f16_to_f32(sc[D + c * EPL + e]);
+    mn[e] = INFINITY;
+    mx[e] = -INFINITY;
+  }
+  for (int i = 0; i < rows; ++i) {
+    const int row = r + 4 * i;
+    int8_t q[EPL];
+    load_bytes<EPL>((const int8_t*)rec + row * D + c * EPL, q);
+    float x[EPL];
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) {
+      x[e] = lkv::round_through<MT>(((float)q[e] + 128.0f) * ks[e] + kz[e]);
+      mn[e] = fminf(mn[e], x[e]);
+      mx[e] = fmaxf(mx[e], x[e]);
+    }
     if constexpr (MODE == MODE_UNPACK) {
-      const int64_t doff = (int64_t)b * a.d_bstride + (int64_t)h * a.d_hstride + c * EPL;
-      dk = (T*)a.dk + doff;
-      dv = (T*)a.dv + doff;
-    }
-    float ks[EPL], kz[EPL], mn[EPL], mx[EPL];
+      store_segment<MT, EPL>(dk + (int64_t)row * D, x);
+      int8_t vq[EPL];
+      load_bytes<EPL>((const int8_t*)rec + bs * D + row * D + c * EPL, vq);
+      const float vs = lkv::f16_to_f32(sc[2 * D + row]);
+      const float vz = lkv::f16_to_f32(sc[2 * D + bs + row]);
+      float v[EPL];
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      ks[e] = lkv::f16_to_f32(sc[c * EPL + e]);
-      kz[e] = lkv::f16_to_f32(sc[D + c * EPL + e]);
-      mn[e] = INFINITY;
-      mx[e] = -INFINITY;
+      for (int e = 0; e < EPL; ++e) v[e] = ((float)vq[e] + 128.0f) * vs + vz;
+      store_segment<MT, EPL>(dv + (int64_t)row * D, v);
     }
-    for (int i = 0; i < rows; ++i) {
-      const int row = r + 4 * i;
-      int8_t q[EPL];
-      load_bytes<EPL>((const int8_t*)rec + row * D + c * EPL, q);
-      float x[EPL];
+  }
+  if (!want_meta) return;
 #pragma unroll
-      for (int e = 0; e < EPL; ++e) {
-        x[e] = lkv::round_through<MT>(((float)q[e] + 128.0f) * ks[e] + kz[e]);
-        mn[e] = fminf(mn[e], x[e]);
-        mx[e] = fmaxf(mx[e], x[e]);
+  for (int e = 0; e < EPL; ++e) {
+    mn[e] = lkv::groups4_min(mn[e]);
+    mx[e] = lkv::groups4_max(mx[e]);
+  }
+  if (r == 0) write_meta<D, MT>(a, b, h, c, mn, mx);
+}
+
+// ---- sources in the model dtype -----------------------------------------------------------------------
+// 8 channels a lane (16 bytes of a 16-bit type): a row is 16 lanes at d 128 and 8 lanes at d 64, and a wave-wide
+// load covers 4 or 8 rows. A pair is read once, in chunks of 16 rows: for blocks of up to 16 tokens every load of
+// the pair is issued before the first is used (longer blocks read their keys twice to make a record). Read a row
+// at a time and the keys twice, with a correctly rounded divide per value, packing 32,768 pairs of 16 x 64 float16
+// took 95 us for 134 MB read and 78 MB written; see quantise8 for the divide.
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2_a4 __attribute__((ext_vector_type(2), aligned(4)));
+
+template <int D, int MT>
+struct Rows {
+  static constexpr int LPR = D / 8;       // lanes per row
+  static constexpr int RG = 64 / LPR;     // rows per wave-wide load
+  static constexpr int NI = 16 / RG;      // loads per 16-row chunk
+  static constexpr int W = 2 * (int)sizeof(typename lkv::Elem<MT>::T);  // words of a lane's 8 channels
+};
+
+template <int D, int MT>
+struct RowChunk {
+  uint32_t w[Rows<D, MT>::NI][Rows<D, MT>::W];
+  // Rows t0 + r + RG i of the pair at p (this lane's channels); a row past the block reads row 0 instead, which
+  // changes no range, and is not stored.
+  __device__ __forceinline__ void load(const typename lkv::Elem<MT>::T* p, int t0, int bs, int r) {
+    using R = Rows<D, MT>;
+#pragma unroll
+    for (int i = 0; i < R::NI; ++i) {
+      const int row = t0 + r + R::RG * i;
+      const uint32_t* at = (const uint32_t*)(p + (int64_t)(row < bs ? row : 0) * D);
+#pragma unroll
+      for (int j = 0; j < R::W; j += 4) {
+        const u32x4_a4 x = *(const u32x4_a4*)(at + j);
+        w[i][j] = x.x;
+        w[i][j + 1] = x.y;
+        w[i][j + 2] = x.z;
+        w[i][j + 3] = x.w;
       }
-      if constexpr (MODE == MODE_UNPACK) {
-        store_segment<MT, EPL>(dk + (int64_t)row * D, x);
-        int8_t vq[EPL];
-        load_bytes<EPL>((const int8_t*)rec + bs * D + row * D + c * EPL, vq);
-        const float vs = lkv::f16_to_f32(sc[2 * D + row]);
-        const float vz = lkv::f16_to_f32(sc[2 * D + bs + row]);
-        float v[EPL];
+    }
+  }
+  __device__ __forceinline__ void store(typename lkv::Elem<MT>::T* p, int t0, int bs, int r) const {
+    using R = Rows<D, MT>;
 #pragma unroll
-        for (int e = 0; e < EPL; ++e) v[e] = ((float)vq[e] + 128.0f) * vs + vz;
-        store_segment<MT, EPL>(dv + (int64_t)row * D, v);
+    for (int i = 0; i < R::NI; ++i) {
+      const int row = t0 + r + R::RG * i;
+      if (row < bs) {
+        uint32_t* at = (uint32_t*)(p + (int64_t)row * D);
+#pragma unroll
+        for (int j = 0; j < R::W; j += 4) *(u32x4_a4*)(at + j) = u32x4_a4{w[i][j], w[i][j + 1], w[i][j + 2], w[i][j + 3]};
       }
     }
-    if (!want_meta) return;
+  }
+  __device__ __forceinline__ void widen(int i, float (&x)[8]) const {
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      mn[e] = lkv::groups4_min(mn[e]);
-      mx[e] = lkv::groups4_max(mx[e]);
+    for (int e = 0; e < 8; ++e) {
+      if constexpr (MT == LKV_F32) {
+        x[e] = lkv::bits_to_float(w[i][e]);
+      } else {
+        x[e] = lkv::Elem<MT>::load((uint16_t)((e & 1) ? w[i][e >> 1] >> 16 : w[i][e >> 1] & 0xffffu));
+      }
     }
-    if (r == 0) write_meta<D, MT>(a, b, h, c, mn, mx);
-    return;
+  }
+};
+
+// range / 255, correctly rounded where it reaches FLT_MIN (the callers take the larger of the two): one corrected
+// product with the rounded reciprocal (Markstein's division by a constant; equal to the divide for every
+// significand, subnormal to largest exponent). An infinite range stays infinite.
+__device__ __forceinline__ float over_255(float range) {
+  constexpr float y = 1.0f / 255.0f;
+  const float q = range * y;
+  const float z = fmaf(fmaf(-q, 255.0f, range), y, q);
+  return range == INFINITY ? range : z;
+}
+__device__ __forceinline__ float scale_of(float mn, float mx) { return fmaxf(over_255(mx - mn), 1.17549435e-38f); }
+
+// The codes clamp(rint((x - mn) / scale), 0, 255) - 128 of 8 values, as 8 bytes. The quotient by the hardware's reciprocal is within 1e-4 of the rounded
+// one (at most 255, three relative errors of 2^-23), so both round to the same integer unless it lies that close to a
+// half: then, for about one group of 8 in 500, the divide itself decides.
+__device__ __forceinline__ uint2 quantise8(const float (&x)[8], const float (&mn)[8], const float (&scale)[8], const float (&inv)[8]) {
+  float q[8], worst = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float t = (x[e] - mn[e]) * inv[e];
+    q[e] = rintf(t);
+    worst = fmaxf(worst, fabsf(t - q[e]));
+  }
+  if (worst > 0.499f) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) q[e] = rintf((x[e] - mn[e]) / scale[e]);
+  }
+  uint32_t w[2] = {0u, 0u};
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    // v_cvt_pk_u8_f32: a whole number of 0..255 into byte e % 4.
+    w[e >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(fminf(fmaxf(q[e], 0.0f), 255.0f), e & 3, w[e >> 2]);
+  }
+  return make_uint2(w[0] ^ 0x80808080u, w[1] ^ 0x80808080u);
+}
+
+// The block's key metadata, 8 channels of a lane of row group 0.
+template <int D, int MT>
+__device__ __forceinline__ void write_meta8(const StoreArgs& a, int b, int h, int c, const float (&mn)[8], const float (&mx)[8]) {
+  const int64_t base = (int64_t)h * a.meta_hstride + (int64_t)b * D + c * 8;
+  if constexpr (MT != LKV_F32) {
+    if (a.meta_words) {
+      uint32_t lo[4], hi[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        lo[e] = lkv::Elem<MT>::store(mn[2 * e]) | ((uint32_t)lkv::Elem<MT>::store(mn[2 * e + 1]) << 16);
+        hi[e] = lkv::Elem<MT>::store(mx[2 * e]) | ((uint32_t)lkv::Elem<MT>::store(mx[2 * e + 1]) << 16);
+      }
+      *(u32x4_a4*)((uint16_t*)a.kmin + base) = u32x4_a4{lo[0], lo[1], lo[2], lo[3]};
+      *(u32x4_a4*)((uint16_t*)a.kmax + base) = u32x4_a4{hi[0], hi[1], hi[2], hi[3]};
+      return;
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    lkv::store_any(a.kmin, base + e, a.meta_dtype, mn[e]);
+    lkv::store_any(a.kmax, base + e, a.meta_dtype, mx[e]);
+  }
+}
+
+template <int D, int MT, int MODE>
+__device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
+  using T = typename lkv::Elem<MT>::T;
+  using R = Rows<D, MT>;
+  const int lane = threadIdx.x & 63;
+  const int r = lane / R::LPR, c = lane % R::LPR;
+  const int b = a.first_block + (int)(pair / a.n_kv);
+  const int h = (int)(pair % a.n_kv);
+  const int bs = a.bs;
+  const bool want_meta = a.kmin != nullptr;
+  const int64_t soff = (int64_t)b * a.s_bstride + (int64_t)h * a.s_hstride + c * 8;
+  const T* sk = (const T*)a.sk + soff;
+  const T* sv = (const T*)a.sv + soff;
+  RowChunk<D, MT> k, v;
+  k.load(sk, 0, bs, r);
+  if constexpr (MODE != MODE_META) v.load(sv, 0, bs, r);
+
+  T* dk = nullptr;
+  T* dv = nullptr;
+  if constexpr (MODE == MODE_COPY) {
+    const int64_t doff = (int64_t)b * a.d_bstride + (int64_t)h * a.d_hstride + c * 8;
+    dk = (T*)a.dk + doff;
+    dv = (T*)a.dv + doff;
+  }
+  // ---- keys: per-channel range over the block's tokens -----------------------------------------------
+  float mn[8], mx[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    mn[e] = INFINITY;
+    mx[e] = -INFINITY;
+  }
+  for (int t0 = 0;;) {
+    if (MODE == MODE_INT8 || want_meta) {
+#pragma unroll
+      for (int i = 0; i < R::NI; ++i) {
+        float x[8];
+        k.widen(i, x);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          mn[e] = fminf(mn[e], x[e]);
+          mx[e] = fmaxf(mx[e], x[e]);
+        }
+      }
+    }
+    if constexpr (MODE == MODE_COPY) {
+      k.store(dk, t0, bs, r);
+      v.store(dv, t0, bs, r);
+    }
+    t0 += 16;
+    if (t0 >= bs) break;
+    k.load(sk, t0, bs, r);
+    if constexpr (MODE == MODE_COPY) v.load(sv, t0, bs, r);
+  }
+  if (MODE == MODE_INT8 || want_meta) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      mn[e] = lkv::groups_min<R::RG>(mn[e]);
+      mx[e] = lkv::groups_max<R::RG>(mx[e]);
+    }
+  }
+  if constexpr (MODE != MODE_INT8) {
+    if (want_meta && r == 0) write_meta8<D, MT>(a, b, h, c, mn, mx);
   } else {
-    const int64_t soff = (int64_t)b * a.s_bstride + (int64_t)h * a.s_hstride + c * EPL;
-    const T* sk = (const T*)a.sk + soff;
-    const T* sv = (const T*)a.sv + soff;
-
-    // ---- keys: per-channel range over the block's tokens -----------------------------------------
-    float mn[EPL], mx[EPL];
+    uint8_t* rec = (uint8_t*)a.dk + (int64_t)b * a.d_bstride + (int64_t)h * a.d_hstride;
+    uint16_t* sc = (uint16_t*)(rec + 2 * bs * D);
+    float scale[8], inv[8];
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      mn[e] = INFINITY;
-      mx[e] = -INFINITY;
+    for (int e = 0; e < 8; ++e) {
+      scale[e] = scale_of(mn[e], mx[e]);
+      inv[e] = __builtin_amdgcn_rcpf(scale[e]);
     }
-    for (int i = 0; i < rows; ++i) {
-      float x[EPL];
-      lkv::load_row_segment<MT, EPL>(sk + (int64_t)(r + 4 * i) * D, x);
-      if constexpr (MODE == MODE_COPY) {
-        T* dk = (T*)a.dk + (int64_t)b * a.d_bstride + (int64_t)h * a.d_hstride + (int64_t)(r + 4 * i) * D + c * EPL;
-        store_segment<MT, EPL>(dk, x);
+    if (r == 0) {
+      uint32_t s[4], z[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        s[e] = lkv::f32_to_f16(scale[2 * e]) | ((uint32_t)lkv::f32_to_f16(scale[2 * e + 1]) << 16);
+        z[e] = lkv::f32_to_f16(mn[2 * e]) | ((uint32_t)lkv::f32_to_f16(mn[2 * e + 1]) << 16);
+      }
+      *(u32x4_a4*)(sc + c * 8) = u32x4_a4{s[0], s[1], s[2], s[3]};
+      *(u32x4_a4*)(sc + D + c * 8) = u32x4_a4{z[0], z[1], z[2], z[3]};
+    }
+    float dmn[8], dmx[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      dmn[e] = INFINITY;
+      dmx[e] = -INFINITY;
+    }
+    for (int t0 = 0; t0 < bs; t0 += 16) {
+      if (bs > 16) {  // one chunk: the keys and values are still in their registers
+        k.load(sk, t0, bs, r);
+        v.load(sv, t0, bs, r);
       }
 #pragma unroll
-      for (int e = 0; e < EPL; ++e) {
-        mn[e] = fminf(mn[e], x[e]);
-        mx[e] = fmaxf(mx[e], x[e]);
+      for (int i = 0; i < R::NI; ++i) {
+        const int row = t0 + r + R::RG * i;
+        float x[8];
+        k.widen(i, x);
+        const uint2 q = quantise8(x, mn, scale, inv);
+        if (want_meta) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            // The dequantised key (quant.py:103-105), a repeated row 0 included.
+            const uint32_t u = (((e < 4 ? q.x : q.y) ^ 0x80808080u) >> (8 * (e & 3))) & 0xffu;
+            const float d = lkv::round_through<MT>((float)u * f16_round(scale[e]) + f16_round(mn[e]));
+            dmn[e] = fminf(dmn[e], d);
+            dmx[e] = fmaxf(dmx[e], d);
+          }
+        }
+        if (row < bs) *(u32x2_a4*)(rec + row * D + c * 8) = u32x2_a4{q.x, q.y};
+      }
+      // ---- values: per-token range over head_dim -------------------------------------------------------
+#pragma unroll
+      for (int i = 0; i < R::NI; ++i) {
+        const int row = t0 + r + R::RG * i;
+        float x[8];
+        v.widen(i, x);
+        float lo = x[0], hi = x[0];
+#pragma unroll
+        for (int e = 1; e < 8; ++e) {
+          lo = fminf(lo, x[e]);
+          hi = fmaxf(hi, x[e]);
+        }
+        lo = lkv::row_min<R::LPR>(lo);
+        hi = lkv::row_max<R::LPR>(hi);
+        const float vs = scale_of(lo, hi), vi = __builtin_amdgcn_rcpf(vs);
+        float lo8[8], vs8[8], vi8[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          lo8[e] = lo;
+          vs8[e] = vs;
+          vi8[e] = vi;
+        }
+        const uint2 q = quantise8(x, lo8, vs8, vi8);
+        if (row < bs) {
+          *(u32x2_a4*)(rec + bs * D + row * D + c * 8) = u32x2_a4{q.x, q.y};
+          if (c == 0) {
+            sc[2 * D + row] = lkv::f32_to_f16(vs);
+            sc[2 * D + bs + row] = lkv::f32_to_f16(lo);
+          }
+        }
       }
     }
+    if (want_meta) {
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      mn[e] = lkv::groups4_min(mn[e]);
-      mx[e] = lkv::groups4_max(mx[e]);
-    }
-
-    if constexpr (MODE == MODE_INT8) {
-      uint8_t* rec = (uint8_t*)a.dk + (int64_t)b * a.d_bstride + (int64_t)h * a.d_hstride;
-      uint16_t* sc = (uint16_t*)(rec + 2 * bs * D);
-      float scale[EPL], s16[EPL], z16[EPL], dmn[EPL], dmx[EPL];
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) {
-        scale[e] = fmaxf((mx[e] - mn[e]) / 255.0f, 1.17549435e-38f);
-        s16[e] = f16_round(scale[e]);
-        z16[e] = f16_round(mn[e]);
-        dmn[e] = INFINITY;
-        dmx[e] = -INFINITY;
+      for (int e = 0; e < 8; ++e) {
+        dmn[e] = lkv::groups_min<R::RG>(dmn[e]);
+        dmx[e] = lkv::groups_max<R::RG>(dmx[e]);
       }
-      for (int i = 0; i < rows; ++i) {
-        float x[EPL];
-        lkv::load_row_segment<MT, EPL>(sk + (int64_t)(r + 4 * i) * D, x);
-        int8_t q[EPL];
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) {
-          q[e] = quantise(x[e], mn[e], scale[e]);
-          const float d = lkv::round_through<MT>(((float)q[e] + 128.0f) * s16[e] + z16[e]);
-          dmn[e] = fminf(dmn[e], d);
-          dmx[e] = fmaxf(dmx[e], d);
-        }
-        store_bytes<EPL>((int8_t*)rec + (r + 4 * i) * D + c * EPL, q);
-      }
-      if (r == 0) {
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) {
-          sc[c * EPL + e] = lkv::f32_to_f16(scale[e]);
-          sc[D + c * EPL + e] = lkv::f32_to_f16(mn[e]);
-        }
-      }
-      if (want_meta) {
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) {
-          dmn[e] = lkv::groups4_min(dmn[e]);
-          dmx[e] = lkv::groups4_max(dmx[e]);
-        }
-        if (r == 0) write_meta<D, MT>(a, b, h, c, dmn, dmx);
-      }
-      // ---- values: per-token range over head_dim ---------------------------------------------
-      for (int i = 0; i < rows; ++i) {
-        const int row = r + 4 * i;
-        float x[EPL];
-        lkv::load_row_segment<MT, EPL>(sv + (int64_t)row * D, x);
-        float vmn = x[0], vmx = x[0];
-#pragma unroll
-        for (int e = 1; e < EPL; ++e) {
-          vmn = fminf(vmn, x[e]);
-          vmx = fmaxf(vmx, x[e]);
-        }
-        vmn = lkv::row16_min(vmn);
-        vmx = lkv::row16_max(vmx);
-        const float vscale = fmaxf((vmx - vmn) / 255.0f, 1.17549435e-38f);
-        int8_t q[EPL];
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) q[e] = quantise(x[e], vmn, vscale);
-        store_bytes<EPL>((int8_t*)rec + bs * D + row * D + c * EPL, q);
-        if (c == 0) {
-          sc[2 * D + row] = lkv::f32_to_f16(vscale);
-          sc[2 * D + bs + row] = lkv::f32_to_f16(vmn);
-        }
-      }
-    } else {
-      if (want_meta && r == 0) write_meta<D, MT>(a, b, h, c, mn, mx);
-      if constexpr (MODE == MODE_COPY) {
-        for (int i = 0; i < rows; ++i) {
-          float x[EPL];
-          lkv::load_row_segment<MT, EPL>(sv + (int64_t)(r + 4 * i) * D, x);
-          T* dv = (T*)a.dv + (int64_t)b * a.d_bstride + (int64_t)h * a.d_hstride + (int64_t)(r + 4 * i) * D + c * EPL;
-          store_segment<MT, EPL>(dv, x);
-        }
-      }
+      if (r == 0) write_meta8<D, MT>(a, b, h, c, dmn, dmx);
     }
   }
 }
@@ -290,7 +440,11 @@ template <int D, int MT, int MODE>
 __global__ __launch_bounds__(kThreads) void store_blocks_kernel(StoreArgs a) {
   const int64_t total = (int64_t)a.n_blocks * a.n_kv;
   for (int64_t pair = (int64_t)blockIdx.x * kWaves + (threadIdx.x >> 6); pair < total; pair += (int64_t)gridDim.x * kWaves)
-    store_pair<D, MT, MODE>(a, pair);  // `pair` is wave-uniform
+    if constexpr (MODE == MODE_META_FROM_I8 || MODE == MODE_UNPACK) {
+      store_record<D, MT, MODE>(a, pair);  // `pair` is wave-uniform
+    } else {
+      store_rows<D, MT, MODE>(a, pair);
+    }
 }
 
 template <int D, int MT>
@@ -388,6 +542,7 @@ extern "C" int lkv_store_blocks(uintptr_t stream, const lkv_kv_source* src, cons
   a.kmax = kmax;
   a.meta_dtype = meta_dtype;
   a.meta_hstride = meta_head_stride;
+  a.meta_words = meta_dtype == mt && (((uintptr_t)kmin | (uintptr_t)kmax) & 3u) == 0 && (meta_head_stride & 1) == 0;
   // A host-memory source or destination: a grid that keeps the host budget in flight, one pair
   // per wave (the kernel strides over the rest).
   int64_t max_wgs = INT64_MAX;
