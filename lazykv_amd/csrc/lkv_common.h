@@ -345,35 +345,37 @@ __device__ __forceinline__ float pair_sum(float x) {
   return a + b;
 }
 template <int M>
-__device__ __forceinline__ float pair_min(float x) {
-  float a, b;
-  lane_pair<M>(x, a, b);
-  return fminf(a, b);
-}
-template <int M>
 __device__ __forceinline__ float pair_max(float x) {
   float a, b;
   lane_pair<M>(x, a, b);
   return fmaxf(a, b);
 }
 
-// Two values summed over lanes l and l ^ M (M = 16 or 32), one to each lane of the pair: a's sum to
-// the lane with bit M clear, b's to the other. One exchange and one add.
+// Lanes l and l ^ M (M = 16 or 32) of two values: a's of both to the lane with bit M clear, b's of both to the
+// other, in x and y.
 template <int M>
-__device__ __forceinline__ float swap_sum(float a, float b) {
+__device__ __forceinline__ void swap_halves(float a, float b, float& x, float& y) {
   static_assert(M == 16 || M == 32, "pairs lanes 16 or 32 apart");
   const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
-  uint32_t x, y;
+  uint32_t p, q;
   if constexpr (M == 16) {
-    const auto p = __builtin_amdgcn_permlane16_swap(ua, ub, false, false);
-    x = p[0];
-    y = p[1];
+    const auto r = __builtin_amdgcn_permlane16_swap(ua, ub, false, false);
+    p = r[0];
+    q = r[1];
   } else {
-    const auto p = __builtin_amdgcn_permlane32_swap(ua, ub, false, false);
-    x = p[0];
-    y = p[1];
+    const auto r = __builtin_amdgcn_permlane32_swap(ua, ub, false, false);
+    p = r[0];
+    q = r[1];
   }
-  return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+  x = __builtin_bit_cast(float, p);
+  y = __builtin_bit_cast(float, q);
+}
+// Two values summed over lanes l and l ^ M, one sum to each lane of the pair. One exchange and one add.
+template <int M>
+__device__ __forceinline__ float swap_sum(float a, float b) {
+  float x, y;
+  swap_halves<M>(a, b, x, y);
+  return x + y;
 }
 
 // ---- whole-wave integer scans and reductions without LDS traffic ------------------------------
@@ -473,13 +475,6 @@ __device__ __forceinline__ float groups_sum(float x) {
   if constexpr (RG == 8) x = pair_sum<8>(x);
   x = pair_sum<16>(x);
   return pair_sum<32>(x);
-}
-template <int RG>
-__device__ __forceinline__ float groups_min(float x) {
-  static_assert(RG == 4 || RG == 8, "rows of 16 or 8 lanes");
-  if constexpr (RG == 8) x = pair_min<8>(x);
-  x = pair_min<16>(x);
-  return pair_min<32>(x);
 }
 template <int RG>
 __device__ __forceinline__ float groups_max(float x) {

@@ -39,7 +39,6 @@ struct StoreArgs {
   void* kmin;
   void* kmax;
   int meta_dtype;
-  int meta_words;  // metadata rows of the source's 16-bit dtype, at whole 32-bit words
   int64_t meta_hstride;
 };
 
@@ -222,6 +221,55 @@ struct RowChunk {
   }
 };
 
+// A lane's 8 channels reduced over the wave's RG row groups: each step keeps one half of the values and gives the
+// partner the other, so lane l ends with the totals of its channels own_channel(l) .. + 8 / RG - 1 in v.
+template <int RG, typename Op>
+__device__ __forceinline__ void reduce_channels(float (&v)[8], int lane, Op op) {
+  constexpr int N = RG == 8 ? 4 : 8;  // values a lane holds after the 8-lane rows' own step
+  if constexpr (RG == 8) {
+    const bool odd = (lane & 8) != 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float keep = odd ? v[i + 4] : v[i], give = odd ? v[i] : v[i + 4];
+      v[i] = op(keep, lkv::dpp<lkv::kDppRowRor8>(give));
+    }
+  }
+  float x, y;
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i) {
+    lkv::swap_halves<16>(v[i], v[i + N / 2], x, y);
+    v[i] = op(x, y);
+  }
+#pragma unroll
+  for (int i = 0; i < N / 4; ++i) {
+    lkv::swap_halves<32>(v[i], v[i + N / 4], x, y);
+    v[i] = op(x, y);
+  }
+}
+template <int RG>
+__device__ __forceinline__ int own_channel(int lane) {
+  constexpr int N = RG == 8 ? 4 : 8;
+  return (RG == 8 && (lane & 8) ? 4 : 0) + ((lane & 16) ? N / 2 : 0) + ((lane & 32) ? N / 4 : 0);
+}
+// The reverse: every lane's 8 channels from the lanes that own them.
+template <int RG>
+__device__ __forceinline__ void gather_channels(float (&v)[8], int lane) {
+  constexpr int N = RG == 8 ? 4 : 8;
+#pragma unroll
+  for (int i = 0; i < N / 4; ++i) lkv::lane_pair<32>(v[i], v[i], v[i + N / 4]);
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i) lkv::lane_pair<16>(v[i], v[i], v[i + N / 2]);
+  if constexpr (RG == 8) {
+    const bool odd = (lane & 8) != 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float mine = v[i], theirs = lkv::dpp<lkv::kDppRowRor8>(mine);
+      v[i] = odd ? theirs : mine;
+      v[i + 4] = odd ? mine : theirs;
+    }
+  }
+}
+
 // range / 255, correctly rounded where it reaches FLT_MIN (the callers take the larger of the two): one corrected
 // product with the rounded reciprocal (Markstein's division by a constant; equal to the divide for every
 // significand, subnormal to largest exponent). An infinite range stays infinite.
@@ -257,31 +305,18 @@ __device__ __forceinline__ uint2 quantise8(const float (&x)[8], const float (&mn
   return make_uint2(w[0] ^ 0x80808080u, w[1] ^ 0x80808080u);
 }
 
-// The block's key metadata, 8 channels of a lane of row group 0.
-template <int D, int MT>
-__device__ __forceinline__ void write_meta8(const StoreArgs& a, int b, int h, int c, const float (&mn)[8], const float (&mx)[8]) {
-  const int64_t base = (int64_t)h * a.meta_hstride + (int64_t)b * D + c * 8;
-  if constexpr (MT != LKV_F32) {
-    if (a.meta_words) {
-      uint32_t lo[4], hi[4];
+// The block's key metadata from the lanes that own its channels.
+template <int D, int RG>
+__device__ __forceinline__ void write_owned(const StoreArgs& a, int b, int h, int c, int lane, const float (&mn)[8], const float (&mx)[8]) {
+  const int64_t base = (int64_t)h * a.meta_hstride + (int64_t)b * D + c * 8 + own_channel<RG>(lane);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        lo[e] = lkv::Elem<MT>::store(mn[2 * e]) | ((uint32_t)lkv::Elem<MT>::store(mn[2 * e + 1]) << 16);
-        hi[e] = lkv::Elem<MT>::store(mx[2 * e]) | ((uint32_t)lkv::Elem<MT>::store(mx[2 * e + 1]) << 16);
-      }
-      *(u32x4_a4*)((uint16_t*)a.kmin + base) = u32x4_a4{lo[0], lo[1], lo[2], lo[3]};
-      *(u32x4_a4*)((uint16_t*)a.kmax + base) = u32x4_a4{hi[0], hi[1], hi[2], hi[3]};
-      return;
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    lkv::store_any(a.kmin, base + e, a.meta_dtype, mn[e]);
-    lkv::store_any(a.kmax, base + e, a.meta_dtype, mx[e]);
+  for (int i = 0; i < 8 / RG; ++i) {
+    lkv::store_any(a.kmin, base + i, a.meta_dtype, mn[i]);
+    lkv::store_any(a.kmax, base + i, a.meta_dtype, mx[i]);
   }
 }
 
-template <int D, int MT, int MODE>
+template <int D, int MT, int MODE, bool META>
 __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
   using T = typename lkv::Elem<MT>::T;
   using R = Rows<D, MT>;
@@ -290,7 +325,9 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
   const int b = a.first_block + (int)(pair / a.n_kv);
   const int h = (int)(pair % a.n_kv);
   const int bs = a.bs;
-  const bool want_meta = a.kmin != nullptr;
+  constexpr bool kRange = META || MODE == MODE_INT8;  // the keys' range is wanted
+  const auto lower = [](float p, float q) { return fminf(p, q); };
+  const auto upper = [](float p, float q) { return fmaxf(p, q); };
   const int64_t soff = (int64_t)b * a.s_bstride + (int64_t)h * a.s_hstride + c * 8;
   const T* sk = (const T*)a.sk + soff;
   const T* sv = (const T*)a.sv + soff;
@@ -313,7 +350,7 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
     mx[e] = -INFINITY;
   }
   for (int t0 = 0;;) {
-    if (MODE == MODE_INT8 || want_meta) {
+    if constexpr (kRange) {
 #pragma unroll
       for (int i = 0; i < R::NI; ++i) {
         float x[8];
@@ -334,34 +371,27 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
     k.load(sk, t0, bs, r);
     if constexpr (MODE == MODE_COPY) v.load(sv, t0, bs, r);
   }
-  if (MODE == MODE_INT8 || want_meta) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      mn[e] = lkv::groups_min<R::RG>(mn[e]);
-      mx[e] = lkv::groups_max<R::RG>(mx[e]);
-    }
+  if constexpr (kRange) {
+    reduce_channels<R::RG>(mn, lane, lower);
+    reduce_channels<R::RG>(mx, lane, upper);
   }
   if constexpr (MODE != MODE_INT8) {
-    if (want_meta && r == 0) write_meta8<D, MT>(a, b, h, c, mn, mx);
+    if constexpr (META) write_owned<D, R::RG>(a, b, h, c, lane, mn, mx);
   } else {
     uint8_t* rec = (uint8_t*)a.dk + (int64_t)b * a.d_bstride + (int64_t)h * a.d_hstride;
     uint16_t* sc = (uint16_t*)(rec + 2 * bs * D);
+    // Each channel's scale is made, and stored, by the lane that owns it.
     float scale[8], inv[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      scale[e] = scale_of(mn[e], mx[e]);
-      inv[e] = __builtin_amdgcn_rcpf(scale[e]);
+    for (int i = 0; i < 8 / R::RG; ++i) {
+      scale[i] = scale_of(mn[i], mx[i]);
+      sc[c * 8 + own_channel<R::RG>(lane) + i] = lkv::f32_to_f16(scale[i]);
+      sc[D + c * 8 + own_channel<R::RG>(lane) + i] = lkv::f32_to_f16(mn[i]);
     }
-    if (r == 0) {
-      uint32_t s[4], z[4];
+    gather_channels<R::RG>(scale, lane);
+    gather_channels<R::RG>(mn, lane);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        s[e] = lkv::f32_to_f16(scale[2 * e]) | ((uint32_t)lkv::f32_to_f16(scale[2 * e + 1]) << 16);
-        z[e] = lkv::f32_to_f16(mn[2 * e]) | ((uint32_t)lkv::f32_to_f16(mn[2 * e + 1]) << 16);
-      }
-      *(u32x4_a4*)(sc + c * 8) = u32x4_a4{s[0], s[1], s[2], s[3]};
-      *(u32x4_a4*)(sc + D + c * 8) = u32x4_a4{z[0], z[1], z[2], z[3]};
-    }
+    for (int e = 0; e < 8; ++e) inv[e] = __builtin_amdgcn_rcpf(scale[e]);
     float dmn[8], dmx[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -379,7 +409,7 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
         float x[8];
         k.widen(i, x);
         const uint2 q = quantise8(x, mn, scale, inv);
-        if (want_meta) {
+        if constexpr (META) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
             // The dequantised key (quant.py:103-105), a repeated row 0 included.
@@ -423,27 +453,24 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
         }
       }
     }
-    if (want_meta) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        dmn[e] = lkv::groups_min<R::RG>(dmn[e]);
-        dmx[e] = lkv::groups_max<R::RG>(dmx[e]);
-      }
-      if (r == 0) write_meta8<D, MT>(a, b, h, c, dmn, dmx);
+    if constexpr (META) {
+      reduce_channels<R::RG>(dmn, lane, lower);
+      reduce_channels<R::RG>(dmx, lane, upper);
+      write_owned<D, R::RG>(a, b, h, c, lane, dmn, dmx);
     }
   }
 }
 
 // One wave per (block, head) pair, the grid striding over the pairs. Waves never synchronise with
 // each other, so a grid smaller than the pair count (a host destination) is just a longer loop.
-template <int D, int MT, int MODE>
+template <int D, int MT, int MODE, bool META>
 __global__ __launch_bounds__(kThreads) void store_blocks_kernel(StoreArgs a) {
   const int64_t total = (int64_t)a.n_blocks * a.n_kv;
   for (int64_t pair = (int64_t)blockIdx.x * kWaves + (threadIdx.x >> 6); pair < total; pair += (int64_t)gridDim.x * kWaves)
     if constexpr (MODE == MODE_META_FROM_I8 || MODE == MODE_UNPACK) {
       store_record<D, MT, MODE>(a, pair);  // `pair` is wave-uniform
     } else {
-      store_rows<D, MT, MODE>(a, pair);
+      store_rows<D, MT, MODE, META>(a, pair);
     }
 }
 
@@ -453,13 +480,26 @@ int launch_store(hipStream_t s, int mode, const StoreArgs& a, int64_t max_wgs) {
   int64_t wgs = (pairs + kWaves - 1) / kWaves;
   if (wgs > max_wgs) wgs = max_wgs;
   const dim3 grid((unsigned)wgs);
+  const bool meta = a.kmin != nullptr;
   switch (mode) {
-    case MODE_META: hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_META>), grid, dim3(kThreads), 0, s, a); break;
-    case MODE_COPY: hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_COPY>), grid, dim3(kThreads), 0, s, a); break;
-    case MODE_INT8: hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_INT8>), grid, dim3(kThreads), 0, s, a); break;
-    case MODE_UNPACK: hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_UNPACK>), grid, dim3(kThreads), 0, s, a); break;
+    case MODE_META: hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_META, true>), grid, dim3(kThreads), 0, s, a); break;
+    case MODE_COPY:
+      if (meta) {
+        hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_COPY, true>), grid, dim3(kThreads), 0, s, a);
+      } else {
+        hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_COPY, false>), grid, dim3(kThreads), 0, s, a);
+      }
+      break;
+    case MODE_INT8:
+      if (meta) {
+        hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_INT8, true>), grid, dim3(kThreads), 0, s, a);
+      } else {
+        hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_INT8, false>), grid, dim3(kThreads), 0, s, a);
+      }
+      break;
+    case MODE_UNPACK: hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_UNPACK, true>), grid, dim3(kThreads), 0, s, a); break;
     default:
-      hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_META_FROM_I8>), grid, dim3(kThreads), 0, s, a);
+      hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_META_FROM_I8, true>), grid, dim3(kThreads), 0, s, a);
       break;
   }
   LKV_CHECK_LAUNCH("store_blocks");
@@ -542,7 +582,6 @@ extern "C" int lkv_store_blocks(uintptr_t stream, const lkv_kv_source* src, cons
   a.kmax = kmax;
   a.meta_dtype = meta_dtype;
   a.meta_hstride = meta_head_stride;
-  a.meta_words = meta_dtype == mt && (((uintptr_t)kmin | (uintptr_t)kmax) & 3u) == 0 && (meta_head_stride & 1) == 0;
   // A host-memory source or destination: a grid that keeps the host budget in flight, one pair
   // per wave (the kernel strides over the rest).
   int64_t max_wgs = INT64_MAX;
