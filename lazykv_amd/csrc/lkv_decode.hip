@@ -757,30 +757,45 @@ __device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D /
   __builtin_amdgcn_wave_barrier();
 }
 
-// Item j0 + u * NW (u < NP) of a segment-A run [.., last): the sink is item 0 when present, the
-// current block the last item (n_a - 1) when present, and the items between are the selected ids in
-// idx order (selected position p at idx_h[p - base]). An item past the run gets block -1 (skipped).
-// Wave-uniform; the ids are read into scalar registers.
+// What a workgroup attends of segment A on the matrix-core path: selected positions [js, je), the sink in the
+// first workgroup and the current block in the last.
+struct MfRun {
+  int js, je;
+  bool sink, cur;
+};
+__device__ __forceinline__ MfRun mf_run(const DecodeArgs& a, int split) {
+  const int n_sel = a.attend_selected ? a.k : 0;
+  MfRun m;
+  m.js = min(n_sel, split * a.per_a);
+  m.je = min(n_sel, m.js + a.per_a);
+  m.sink = a.sink_block >= 0 && split == 0;
+  m.cur = a.cur_block >= 0 && split == a.splits_a - 1;
+  return m;
+}
+
+// Items j0 + u * NW (u < NP) of a run: the sink, the selected ids in idx order (position p at idx_h[p - base]),
+// the current block. An item past the run gets block -1 (skipped). Wave-uniform; the ids are read into scalar
+// registers.
 template <int NP, int NW>
-__device__ __forceinline__ void segment_items(const DecodeArgs& a, const int32_t* idx_h, int base, int j0, int last, Src (&s)[NP],
-                                              int (&blk)[NP], int (&lim)[NP]) {
-  const int has_sink = a.sink_block >= 0;
+__device__ __forceinline__ void run_items(const DecodeArgs& a, const MfRun& run, const int32_t* idx_h, int base, int j0, Src (&s)[NP],
+                                          int (&blk)[NP], int (&lim)[NP]) {
+  const int count = run.sink + (run.je - run.js) + run.cur;
 #pragma unroll
   for (int u = 0; u < NP; ++u) {
     const int it = j0 + u * NW;
     s[u] = a.sel;
     blk[u] = -1;
     lim[u] = a.bs;
-    if (it < last) {
-      if (has_sink && it == 0) {
+    if (it < count) {
+      if (run.sink && it == 0) {
         s[u] = a.sink;
         blk[u] = a.sink_block;
-      } else if (a.cur_block >= 0 && it == a.n_a - 1) {
+      } else if (run.cur && it == count - 1) {
         s[u] = a.cur;
         blk[u] = a.cur_block;
         lim[u] = a.fill;
       } else {
-        blk[u] = __builtin_amdgcn_readfirstlane(idx_h[it - has_sink - base]);
+        blk[u] = __builtin_amdgcn_readfirstlane(idx_h[run.js + it - run.sink - base]);
       }
     }
   }
@@ -831,6 +846,18 @@ __device__ __forceinline__ void process_items_mf(const DecodeArgs& a, const Src 
     for (int u = 0; u < NP; ++u) load_raw_mf(ls[u], a.bs, lb[u], h, t0, nit, ll[u], lane, r, c, raw[u]);
     __builtin_amdgcn_sched_barrier(0);  // every load above issues before the first use below
     consume_mf<D, MT, G, NP>(qb, raw, a.qscale, t0, lk, lane, r, sp, st);
+  }
+}
+
+// Items j0, j0 + NW, .. < count of a run of 16-bit pairs.
+template <int D, int MT, int G, int NP, int NW>
+__device__ __forceinline__ void attend_items_mf(const DecodeArgs& a, const MfRun& run, const int32_t* idx_h, int base, int j0, int count, int h,
+                                                const typename Mfma<MT>::V8 (&qb)[D / 32], int lane, int r, int c, float* sp, MfState<G>& st) {
+  for (; j0 < count; j0 += NP * NW) {
+    Src s[NP];
+    int blk[NP], lim[NP];
+    run_items<NP, NW>(a, run, idx_h, base, j0, s, blk, lim);
+    process_items_mf<D, MT, G, RawMf<D, MT>, NP>(a, s, blk, lim, h, qb, lane, r, c, sp, st);
   }
 }
 
@@ -1093,6 +1120,29 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
       for (int e = 0; e < EPL; ++e) q[j][e] *= a.qscale;
   }
 
+  MfRun run{0, 0, false, false};
+  if constexpr (MF) run = mf_run(a, split);
+  // Beside int8 records the sink and the current block are 16-bit pairs of their own, one wave each: loaded here,
+  // they arrive during the selection and the records, and are folded last. (Blocks of more than 16 tokens load them
+  // then, and at d 128 the launches that read given ids, and 8 heads, which have no registers left for it.)
+  constexpr bool kEarlyEnd = MF && I8 && (D == 64 || (G <= 4 && SEL > 0));
+  Src end_src = a.sink;
+  int end_block = -1, end_lim[1] = {a.bs};
+  typename std::conditional<kEarlyEnd, RawMf<D, MT == LKV_F32 ? LKV_F16 : MT>, char>::type end_raw[1];
+  if constexpr (MF && I8) {
+    const int wv = __builtin_amdgcn_readfirstlane(wave);
+    if (split < a.splits_a && run.sink && wv == NW - 1) end_block = a.sink_block;
+    if (split < a.splits_a && run.cur && wv == NW - 2) {
+      end_src = a.cur;
+      end_block = a.cur_block;
+      end_lim[0] = a.fill;
+    }
+    if constexpr (kEarlyEnd) {
+      if (end_block >= 0 && a.bs <= 16)
+        load_raw_mf(end_src, a.bs, end_block, h, 0, min(L::NI, (a.bs + L::RG - 1) / L::RG), end_lim[0], lane, r, c, end_raw[0]);
+    }
+  }
+
   // ---- fused selection: this head's top k, and the ids of this workgroup's run -----------------
   // The run's selected ids go to LDS (over the histogram, free once the selection is done), as
   // positions [sel_base, sel_base + run) of the ascending selected list.
@@ -1102,11 +1152,14 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
     idx_h = a.idx + (int64_t)h * a.idx_stride;
   } else {
     const lkv::SelectPick pk = lkv::block_top_k<NT, kSelKpt<NT, SEL>>(a.bounds + (int64_t)h * a.bound_stride, a.bounds_aligned != 0, a.n_cand, a.k, s_sel);
-    const int has_sink = a.sink_block >= 0;
-    const int first = split * a.per_a;
-    const int last = min(a.n_a, first + a.per_a);
-    const int js = max(first, has_sink) - has_sink;
-    const int je = min(last, has_sink + a.k) - has_sink;
+    int js = run.js, je = run.je;
+    if constexpr (!MF) {
+      const int has_sink = a.sink_block >= 0;
+      const int first = split * a.per_a;
+      const int last = min(a.n_a, first + a.per_a);
+      js = max(first, has_sink) - has_sink;
+      je = min(last, has_sink + a.k) - has_sink;
+    }
     int32_t* ids = (int32_t*)s_sel.hist;
     int32_t* out_h = (a.idx_out != nullptr && split == 0) ? a.idx_out + (int64_t)h * a.idx_out_stride : nullptr;
     // Most threads' few picks lie outside this workgroup's run.
@@ -1149,35 +1202,34 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
     const int has_sink = a.sink_block >= 0;
     const int n_sel = a.attend_selected ? a.k : 0;
     if constexpr (MF && I8) {
-      // The sink and the current block are 16-bit pairs, one wave each; the selected items int8 records (or,
-      // beside an int8 remainder, 16-bit pairs), kMfPairs of them per wave and round.
-      const int wv = __builtin_amdgcn_readfirstlane(wave);
-      const int js = max(first, has_sink) - has_sink;
-      const int je = min(last, has_sink + n_sel) - has_sink;
+      // The selected items are int8 records (or, beside an int8 remainder, 16-bit pairs), kMfPairs of them per
+      // wave and round.
+      const int j0 = run.js + __builtin_amdgcn_readfirstlane(wave);
       if (a.sel.dtype == LKV_INT8_RECORD) {
-        attend_run_mf<D, MT, G, RecMf<D>, NW>(a, idx_h, sel_base, js + wv, je, h, qb, lane, r, c, sp, st);
+        attend_run_mf<D, MT, G, RecMf<D>, NW>(a, idx_h, sel_base, j0, run.je, h, qb, lane, r, c, sp, st);
       } else {
-        attend_run_mf<D, MT, G, RawMf<D, MT>, NW>(a, idx_h, sel_base, js + wv, je, h, qb, lane, r, c, sp, st);
+        attend_run_mf<D, MT, G, RawMf<D, MT>, NW>(a, idx_h, sel_base, j0, run.je, h, qb, lane, r, c, sp, st);
       }
-      const bool mine_sink = has_sink && first == 0 && wv == NW - 1, mine_cur = a.cur_block >= 0 && last == a.n_a && wv == NW - 1;
-      if (mine_sink || mine_cur) {  // the wave with the fewest selected items, both pairs at once in a short run
-        const Src es[2] = {a.sink, a.cur};
-        const int eb[2] = {mine_sink ? a.sink_block : -1, mine_cur ? a.cur_block : -1};
-        const int el[2] = {a.bs, a.fill};
-        process_items_mf<D, MT, G, RawMf<D, MT>, 2>(a, es, eb, el, h, qb, lane, r, c, sp, st);
+      if (end_block >= 0) {  // wave-uniform
+        if (kEarlyEnd && a.bs <= 16) {
+          if constexpr (kEarlyEnd) consume_mf<D, MT, G, 1>(qb, end_raw, a.qscale, 0, end_lim, lane, r, sp, st);
+        } else {
+          const Src es[1] = {end_src};
+          const int eb[1] = {end_block};
+          process_items_mf<D, MT, G, RawMf<D, MT>, 1>(a, es, eb, end_lim, h, qb, lane, r, c, sp, st);
+        }
       }
     } else if constexpr (MF) {
       // Every item of the run -- the sink, selected ids, the current block -- is a 16-bit
       // pair, so each wave takes kMfPairs of them per round, all loads in flight together: with
       // about two items per wave in the HBM plan, the wave that holds a third needs no second
-      // round.
-      constexpr int kMfItems = kMfPairs<D, G, false>;
+      // round. A run of at most two a wave leaves the third out.
       const int wv = __builtin_amdgcn_readfirstlane(wave);
-      for (int j0 = first + wv; j0 < last; j0 += kMfItems * NW) {
-        Src is[kMfItems];
-        int ib[kMfItems], il[kMfItems];
-        segment_items<kMfItems, NW>(a, idx_h, sel_base, j0, last, is, ib, il);
-        process_items_mf<D, MT, G, RawMf<D, MT>, kMfItems>(a, is, ib, il, h, qb, lane, r, c, sp, st);
+      const int count = run.sink + (run.je - run.js) + run.cur;
+      if (count <= 2 * NW) {
+        attend_items_mf<D, MT, G, 2, NW>(a, run, idx_h, sel_base, wv, count, h, qb, lane, r, c, sp, st);
+      } else {
+        attend_items_mf<D, MT, G, kMfPairs<D, G, false>, NW>(a, run, idx_h, sel_base, wv, count, h, qb, lane, r, c, sp, st);
       }
     } else {
       if (has_sink && first == 0 && wave == 0) attend_two<D, MT, G, I8>(a, a.sink, a.sink_block, -1, h, a.bs, q, r, c, st);
@@ -1516,6 +1568,18 @@ static Plan make_plan(const lkv_decode_desc* d, const PlanHints& hint = PlanHint
   return p;
 }
 
+// Segment A of a launch on the matrix cores is cut by selected items alone; the sink and the current block come
+// on top of the first and the last workgroup's. With 512 or 1,024 selected items of 8 KV heads on 256 CUs every
+// wave then holds exactly 2 or 4, where cutting all 514 or 1,026 items gave one wave of each workgroup 3 or 5: the
+// fifth int8 record needs a second round of loads.
+static void plan_matrix(Plan& p, const lkv_decode_desc* d, int cus) {
+  const int n_sel = d->attend_selected ? d->k : 0;
+  const int per_head = cus / d->n_kv > 1 ? cus / d->n_kv : 1;
+  p.per_a = (n_sel + per_head - 1) / per_head;
+  if (p.per_a < kThreadsHbm / 64) p.per_a = kThreadsHbm / 64;
+  p.splits_a = p.n_a > 0 ? (n_sel > 0 ? (n_sel + p.per_a - 1) / p.per_a : 1) : 0;
+}
+
 // The kernel instance a launch takes. HBM plans (a.nt == kThreadsHbm) run 8-wave workgroups on the matrix cores
 // when the query has the model dtype and 16-byte aligned rows: one instance for 16-bit pairs, one that also
 // reads int8 records. Other queries (and float32 pools) take the 8-wave vector path for 16-bit and
@@ -1556,7 +1620,11 @@ int launch_inst(hipStream_t stream, DecodeArgs& a, Inst inst) {
       done = true;
     }
   }
-  if (!done) hipLaunchKernelGGL((sparse_decode_kernel<D, MT, G, kThreads, true, false, SEL>), grid, dim3(kThreads), 0, stream, a);
+  if constexpr (SEL * kSelUnit <= kFuseKeysPerThread * kThreads) {  // more candidates never select in a 4-wave launch
+    if (!done) hipLaunchKernelGGL((sparse_decode_kernel<D, MT, G, kThreads, true, false, SEL>), grid, dim3(kThreads), 0, stream, a);
+    done = true;
+  }
+  LKV_CHECK_ARG(done, "no decode instance selects from more than %d candidates here", kFuseKeysPerThread * kThreads);
   LKV_CHECK_LAUNCH("sparse_decode");
   return LKV_OK;
 }
@@ -1939,7 +2007,9 @@ extern "C" size_t lkv_sparse_decode_workspace_bytes(const lkv_decode_desc* d) {
   // Host plans only cut the default plan's partial count; the HBM plan may raise it.
   const Plan p = make_plan(d);
   const Plan ph = make_plan(d, PlanHints(), device_cus());
-  const size_t S = (size_t)max(p.splits_a + p.splits_b, ph.splits_a + ph.splits_b);
+  Plan pm = ph;
+  plan_matrix(pm, d, device_cus());
+  const size_t S = (size_t)max(p.splits_a + p.splits_b, max(ph.splits_a, pm.splits_a) + ph.splits_b);
   const size_t G = (size_t)(d->n_q / d->n_kv);
   return lkv_align_up((size_t)d->n_kv * S * G * 2 * 4, 256) + lkv_align_up((size_t)d->n_kv * S * G * d->head_dim * 4, 256);
 }
@@ -2028,13 +2098,8 @@ static int sparse_decode_impl(uintptr_t stream, const lkv_decode_desc* desc, con
     hint.rem_host = (rem->flags & LKV_SRC_HOST) != 0;
     hint.rem_pair = lkv_pair_bytes(rem, d.block_size, d.head_dim);
   }
-  const Plan p = make_plan(desc, hint, device_cus());
-  const int S = p.splits_a + p.splits_b;
-  LKV_CHECK_ARG(S > 0, "nothing to attend");
-  LKV_CHECK_ARG(S <= kMaxSplits, "too many partials (%d)", S);
-  const size_t need = lkv_sparse_decode_workspace_bytes(desc);
-  LKV_CHECK_ARG(ws != nullptr && ws_bytes >= need, "workspace of %zu bytes needed, got %zu", need, ws_bytes);
-
+  Plan p = make_plan(desc, hint, device_cus());
+  const int G = d.n_q / d.n_kv;
   DecodeArgs a{};
   a.q = q;
   a.q_dtype = q_dtype;
@@ -2042,6 +2107,16 @@ static int sparse_decode_impl(uintptr_t stream, const lkv_decode_desc* desc, con
   a.sink = to_src(sink);
   a.cur = to_src(cur);
   a.rem = to_src(rem);
+  a.loc = loc;
+  a.nt = p.nt;
+  const Inst inst = pick_instance(a, mt, G, false);
+  if (inst == Inst::kMatrix8 || inst == Inst::kMatrixRec8) plan_matrix(p, desc, device_cus());
+  const int S = p.splits_a + p.splits_b;
+  LKV_CHECK_ARG(S > 0, "nothing to attend");
+  LKV_CHECK_ARG(S <= kMaxSplits, "too many partials (%d)", S);
+  const size_t need = lkv_sparse_decode_workspace_bytes(desc);
+  LKV_CHECK_ARG(ws != nullptr && ws_bytes >= need, "workspace of %zu bytes needed, got %zu", need, ws_bytes);
+
   a.idx = idx;
   a.idx_stride = idx_stride;
   a.n_kv = d.n_kv;
@@ -2059,16 +2134,13 @@ static int sparse_decode_impl(uintptr_t stream, const lkv_decode_desc* desc, con
   a.splits_a = p.splits_a;
   a.per_b = p.per_b;
   a.splits_b = p.splits_b;
-  a.nt = p.nt;
   a.out = out;
   a.out_dtype = out_dtype;
   a.lse = lse;
-  const int G = d.n_q / d.n_kv;
   char* w = (char*)ws;
   a.part_ml = (float*)w;
   w += lkv_align_up((size_t)d.n_kv * S * G * 2 * 4, 256);
   a.part_o = (float*)w;
-  a.loc = loc;
   a.loc_stride = loc_stride;
   if (slots) a.slots = to_src(slots);
   // Inside the decode launch only where that launch takes the instance the unfused call takes, so
@@ -2077,7 +2149,7 @@ static int sparse_decode_impl(uintptr_t stream, const lkv_decode_desc* desc, con
   bool select_in_decode = false;
   if (fsel != nullptr && fsel->in_decode) {
     const Inst fused = pick_instance(a, mt, G, true);
-    select_in_decode = fused == pick_instance(a, mt, G, false) && fsel->n_cand <= kFuseKeysPerThread * inst_threads(fused);
+    select_in_decode = fused == inst && fsel->n_cand <= kFuseKeysPerThread * inst_threads(fused);
   }
   if (fsel != nullptr) {
     // A remainder excludes the selected ids, so they must exist before the decode launch: chosen by
