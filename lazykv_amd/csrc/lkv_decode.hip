@@ -658,15 +658,15 @@ __device__ __forceinline__ void value_row(const RecMf<D>& raw, int i, float (&x)
   for (int e = 0; e < 8; ++e) x[e] = (float)(typename MfElem<MT>::T)Wd::deq(Wd::u8(w, e), sc, ze);
 }
 
-// Fold the same chunk (rows t0 .. t0 + 15) of NP pairs into the wave's running softmax, as
-// consume_chunk does one pair at a time, with the scores from the matrix cores: one maximum, one
-// rescale and one broadcast for all NP pairs. lim[u]: valid tokens of pair u (0 skips the pair).
+// Fold a chunk (16 rows) of each of NP pairs into the wave's running softmax, as
+// consume_chunk does one at a time, with the scores from the matrix cores: one maximum, one
+// rescale and one broadcast for all NP of them. rows[u]: valid rows of chunk u (0 or less skips it).
 // `sp`: this wave's broadcast area. P.V runs as v_mfma_f32_4x4x1_16b_f32: 16 blocks of 4 lanes, each the
 // outer product of 4 heads' weights of the block's row (lane l: head l % 4) and its lanes' values, in
 // float32, one instruction where 4 heads took 4 fused multiply-adds, off the vector ALUs.
 template <int D, int MT, int G, int NP, typename Raw>
 __device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D / 32], const Raw (&raw)[NP], float qscale,
-                                           int t0, const int (&lim)[NP], int lane, int r, float* sp, MfState<G>& st) {
+                                           const int (&rows)[NP], int lane, int r, float* sp, MfState<G>& st) {
   using L = Lanes<D>;
   static_assert(L::EPL == 8, "8 channels a lane");
   constexpr int GQ = kHeadQuads<G>, GW = 4 * GQ;
@@ -675,7 +675,7 @@ __device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D /
 #pragma unroll
   for (int u = 0; u < NP; ++u) {
     acc[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    if (lim[u] > 0) {  // wave-uniform
+    if (rows[u] > 0) {  // wave-uniform
 #pragma unroll
       for (int s = 0; s < D / 32; ++s) acc[u] = Mfma<MT>::mma(key_frag<D, MT>(raw[u], s), qb[s], acc[u]);
     }
@@ -688,7 +688,7 @@ __device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D /
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       sc[u][i] = acc[u][i] * qscale;
-      vld[u][i] = t0 + 4 * lg + i < lim[u];
+      vld[u][i] = 4 * lg + i < rows[u];
       cm = vld[u][i] ? fmaxf(cm, sc[u][i]) : cm;
     }
   cm = lkv::pair_max<32>(lkv::pair_max<16>(cm));
@@ -732,23 +732,29 @@ __device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D /
   }
 #pragma unroll
   for (int u = 0; u < NP; ++u) {
-    if (lim[u] <= 0) continue;                // wave-uniform, as the next test
-    const bool part = t0 + 16 > lim[u];       // rows past the limit may hold non-finite data
+    if (rows[u] <= 0) continue;                // wave-uniform, as the next test
+    const bool part = rows[u] < 16;           // rows past the limit may hold non-finite data
 #pragma unroll
     for (int i = 0; i < L::NI; ++i) {
       const int row = r + L::RG * i;
       float x[8];
       value_row<D, MT>(raw[u], i, x);
       if (part) {
-        const bool ok = t0 + row < lim[u];
+        const bool ok = row < rows[u];
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] = ok ? x[e] : 0.0f;  // their weights are 0
       }
+      if constexpr (G == 1) {  // one row of four: the vector ALUs are as fast
+        const float pr = sp[(16 * u + row) * GW];
 #pragma unroll
-      for (int g = 0; g < GQ; ++g) {
-        const float pr = sp[(16 * u + row) * GW + 4 * g + (lane & 3)];
+        for (int e = 0; e < 8; ++e) st.o[0][e][0] = fmaf(pr, x[e], st.o[0][e][0]);
+      } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) st.o[g][e] = __builtin_amdgcn_mfma_f32_4x4x1f32(pr, x[e], st.o[g][e], 0, 0, 0);
+        for (int g = 0; g < GQ; ++g) {
+          const float pr = sp[(16 * u + row) * GW + 4 * g + (lane & 3)];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) st.o[g][e] = __builtin_amdgcn_mfma_f32_4x4x1f32(pr, x[e], st.o[g][e], 0, 0, 0);
+        }
       }
     }
   }
@@ -773,16 +779,36 @@ __device__ __forceinline__ MfRun mf_run(const DecodeArgs& a, int split) {
   return m;
 }
 
-// Items j0 + u * NW (u < NP) of a run: the sink, the selected ids in idx order (position p at idx_h[p - base]),
-// the current block. An item past the run gets block -1 (skipped). Wave-uniform; the ids are read into scalar
-// registers.
+// The items of a run are the 16-row chunks of its pairs, so that a block of 64 tokens keeps four waves (or four of a
+// wave's slots) busy instead of one four times over. chunk_of: pair and first row of item `it`.
+__device__ __forceinline__ int chunks_of(const DecodeArgs& a) { return (a.bs + 15) >> 4; }
+// Slots per wave and round for `count` items: as few rounds as `most` slots allow, and no more slots than those need
+// (four items a wave are two rounds of two, not of three: a slot without an item loads another one again).
+__device__ __forceinline__ int slots_for(int count, int waves, int most) {
+  const int each = (count + waves - 1) / waves;
+  const int rounds = (each + most - 1) / most;
+  return rounds > 0 ? (each + rounds - 1) / rounds : 1;
+}
+__device__ __forceinline__ void chunk_of(int it, int nch, int& pair, int& t0) {
+  pair = it;
+  t0 = 0;
+  if (nch > 1) {  // wave-uniform, in scalar registers
+    pair = it / nch;
+    t0 = 16 * (it - pair * nch);
+  }
+}
+
+// Items j0 + u * NW (u < NP) of a run of 16-bit pairs: the sink, the selected ids in idx order (position p at
+// idx_h[p - base]), the current block. An item past the run gets block -1 (skipped). Wave-uniform; the ids are read
+// into scalar registers.
 template <int NP, int NW>
-__device__ __forceinline__ void run_items(const DecodeArgs& a, const MfRun& run, const int32_t* idx_h, int base, int j0, Src (&s)[NP],
-                                          int (&blk)[NP], int (&lim)[NP]) {
+__device__ __forceinline__ void run_items(const DecodeArgs& a, const MfRun& run, const int32_t* idx_h, int base, int j0, int nch, Src (&s)[NP],
+                                          int (&blk)[NP], int (&lim)[NP], int (&t0)[NP]) {
   const int count = run.sink + (run.je - run.js) + run.cur;
 #pragma unroll
   for (int u = 0; u < NP; ++u) {
-    const int it = j0 + u * NW;
+    int it;
+    chunk_of(j0 + u * NW, nch, it, t0[u]);
     s[u] = a.sel;
     blk[u] = -1;
     lim[u] = a.bs;
@@ -801,71 +827,80 @@ __device__ __forceinline__ void run_items(const DecodeArgs& a, const MfRun& run,
   }
 }
 
-// Up to NP pairs on the matrix cores, each of its own source and valid-token limit (Raw: 16-bit pairs or
-// int8 records): every pair's loads are issued before any is consumed, and they are consumed in item
+// Chunks of up to NP pairs on the matrix cores, each of its own source, valid-token limit and first row t0 (Raw:
+// 16-bit pairs or int8 records): every chunk's loads are issued before any is consumed, and they are consumed in
 // order. Ids outside their source are skipped (wave-uniform), never read.
 template <int D, int MT, int G, typename Raw, int NP>
-__device__ __forceinline__ void process_items_mf(const DecodeArgs& a, const Src (&s)[NP], const int (&blk)[NP], const int (&lim)[NP],
-                                                 int h, const typename Mfma<MT>::V8 (&qb)[D / 32], int lane, int r, int c, float* sp,
-                                                 MfState<G>& st) {
+__device__ __forceinline__ void process_chunks_mf(const DecodeArgs& a, const Src (&s)[NP], const int (&blk)[NP], const int (&lim)[NP],
+                                                  const int (&t0)[NP], int h, const typename Mfma<MT>::V8 (&qb)[D / 32], int lane, int r,
+                                                  int c, float* sp, MfState<G>& st) {
   bool ok[NP];
+  int rows[NP];  // valid rows per chunk; 0 for a skipped one
 #pragma unroll
-  for (int u = 0; u < NP; ++u) ok[u] = blk[u] >= 0 && (int64_t)blk[u] < s[u].nblk;
-  int lk[NP];  // valid tokens per pair; 0 for a skipped pair
-#pragma unroll
-  for (int u = 0; u < NP; ++u) lk[u] = ok[u] ? lim[u] : 0;
-  // A skipped pair loads the first live pair again (its lk of 0 masks it), so every pair's loads
+  for (int u = 0; u < NP; ++u) {
+    ok[u] = blk[u] >= 0 && (int64_t)blk[u] < s[u].nblk && t0[u] < lim[u];
+    rows[u] = ok[u] ? lim[u] - t0[u] : 0;
+  }
+  // A skipped chunk loads the first live one again (its 0 rows mask it), so every chunk's loads
   // are issued unconditionally, back to back: under a per-pair branch the compiler put waits
   // between one pair's loads and the next (registers of in-flight loads reused across the
   // branches), and the pairs of a round arrived one memory latency apart.
-  // The first live pair, picked by unrolled selects (an index into s would put it in scratch).
+  // The first live chunk, picked by unrolled selects (an index into s would put it in scratch).
   Src fs = s[0];
-  int fb = -1, fl = 0;
+  int fb = -1, fl = 0, ft = 0;
 #pragma unroll
   for (int u = NP - 1; u >= 0; --u) {
     if (ok[u]) {
       fs = s[u];
       fb = blk[u];
       fl = lim[u];
+      ft = t0[u];
     }
   }
   if (fb < 0) return;  // wave-uniform: nothing live
-  Src ls[NP];
-  int lb[NP], ll[NP];
+  Raw raw[NP];
 #pragma unroll
   for (int u = 0; u < NP; ++u) {
-    ls[u] = ok[u] ? s[u] : fs;
-    lb[u] = ok[u] ? blk[u] : fb;
-    ll[u] = ok[u] ? lim[u] : fl;
+    const Src& ls = ok[u] ? s[u] : fs;
+    const int lt = ok[u] ? t0[u] : ft;
+    const int nit = min(Lanes<D>::NI, (a.bs - lt + Lanes<D>::RG - 1) / Lanes<D>::RG);
+    load_raw_mf(ls, a.bs, ok[u] ? blk[u] : fb, h, lt, nit, ok[u] ? lim[u] : fl, lane, r, c, raw[u]);
   }
+  __builtin_amdgcn_sched_barrier(0);  // every load above issues before the first use below
+  consume_mf<D, MT, G, NP>(qb, raw, a.qscale, rows, lane, r, sp, st);
+}
+
+// Whole pairs, a chunk of each at a time.
+template <int D, int MT, int G, typename Raw, int NP>
+__device__ __forceinline__ void process_items_mf(const DecodeArgs& a, const Src (&s)[NP], const int (&blk)[NP], const int (&lim)[NP],
+                                                 int h, const typename Mfma<MT>::V8 (&qb)[D / 32], int lane, int r, int c, float* sp,
+                                                 MfState<G>& st) {
 #pragma unroll 1
-  for (int t0 = 0; t0 < a.bs; t0 += 16) {
-    const int nit = min(Lanes<D>::NI, (a.bs - t0 + Lanes<D>::RG - 1) / Lanes<D>::RG);
-    Raw raw[NP];
+  for (int t = 0; t < a.bs; t += 16) {
+    int t0[NP];
 #pragma unroll
-    for (int u = 0; u < NP; ++u) load_raw_mf(ls[u], a.bs, lb[u], h, t0, nit, ll[u], lane, r, c, raw[u]);
-    __builtin_amdgcn_sched_barrier(0);  // every load above issues before the first use below
-    consume_mf<D, MT, G, NP>(qb, raw, a.qscale, t0, lk, lane, r, sp, st);
+    for (int u = 0; u < NP; ++u) t0[u] = t;
+    process_chunks_mf<D, MT, G, Raw, NP>(a, s, blk, lim, t0, h, qb, lane, r, c, sp, st);
   }
 }
 
-// Items j0, j0 + NW, .. < count of a run of 16-bit pairs.
+// Items j0, j0 + NW, .. < count (chunks) of a run of 16-bit pairs.
 template <int D, int MT, int G, int NP, int NW>
 __device__ __forceinline__ void attend_items_mf(const DecodeArgs& a, const MfRun& run, const int32_t* idx_h, int base, int j0, int count, int h,
                                                 const typename Mfma<MT>::V8 (&qb)[D / 32], int lane, int r, int c, float* sp, MfState<G>& st) {
+  const int nch = chunks_of(a);
   for (; j0 < count; j0 += NP * NW) {
     Src s[NP];
-    int blk[NP], lim[NP];
-    run_items<NP, NW>(a, run, idx_h, base, j0, s, blk, lim);
-    process_items_mf<D, MT, G, RawMf<D, MT>, NP>(a, s, blk, lim, h, qb, lane, r, c, sp, st);
+    int blk[NP], lim[NP], t0[NP];
+    run_items<NP, NW>(a, run, idx_h, base, j0, nch, s, blk, lim, t0);
+    process_chunks_mf<D, MT, G, RawMf<D, MT>, NP>(a, s, blk, lim, t0, h, qb, lane, r, c, sp, st);
   }
 }
 
-// Selected items j, j + NW, .. < je of the launch's selection (ids at idx_h[j - base]).
-template <int D, int MT, int G, typename Raw, int NW>
-__device__ __forceinline__ void attend_run_mf(const DecodeArgs& a, const int32_t* idx_h, int base, int j, int je, int h,
+// Items j, j + NW, .. < count (chunks) of a run's selected pairs (ids at idx_h[position - base]).
+template <int D, int MT, int G, typename Raw, int NP, int NW>
+__device__ __forceinline__ void attend_run_mf(const DecodeArgs& a, const MfRun& run, const int32_t* idx_h, int base, int j, int count, int h,
                                               const typename Mfma<MT>::V8 (&qb)[D / 32], int lane, int r, int c, float* sp, MfState<G>& st) {
-  constexpr int NP = kMfPairs<D, G, std::is_same<Raw, RecMf<D>>::value>;
   Src s[NP];
   int lim[NP];
 #pragma unroll
@@ -873,11 +908,16 @@ __device__ __forceinline__ void attend_run_mf(const DecodeArgs& a, const int32_t
     s[u] = a.sel;
     lim[u] = a.bs;
   }
-  for (; j < je; j += NP * NW) {
-    int blk[NP];
+  const int nch = chunks_of(a);
+  for (; j < count; j += NP * NW) {
+    int blk[NP], t0[NP];
 #pragma unroll
-    for (int u = 0; u < NP; ++u) blk[u] = j + u * NW < je ? __builtin_amdgcn_readfirstlane(idx_h[j + u * NW - base]) : -1;
-    process_items_mf<D, MT, G, Raw, NP>(a, s, blk, lim, h, qb, lane, r, c, sp, st);
+    for (int u = 0; u < NP; ++u) {
+      int pair;
+      chunk_of(j + u * NW, nch, pair, t0[u]);
+      blk[u] = j + u * NW < count ? __builtin_amdgcn_readfirstlane(idx_h[run.js + pair - base]) : -1;
+    }
+    process_chunks_mf<D, MT, G, Raw, NP>(a, s, blk, lim, t0, h, qb, lane, r, c, sp, st);
   }
 }
 
@@ -1202,17 +1242,24 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
     const int has_sink = a.sink_block >= 0;
     const int n_sel = a.attend_selected ? a.k : 0;
     if constexpr (MF && I8) {
-      // The selected items are int8 records (or, beside an int8 remainder, 16-bit pairs), kMfPairs of them per
-      // wave and round.
-      const int j0 = run.js + __builtin_amdgcn_readfirstlane(wave);
-      if (a.sel.dtype == LKV_INT8_RECORD) {
-        attend_run_mf<D, MT, G, RecMf<D>, NW>(a, idx_h, sel_base, j0, run.je, h, qb, lane, r, c, sp, st);
+      // The selected items are int8 records (or, beside an int8 remainder, 16-bit pairs), up to kMfPairs of them
+      // per wave and round, and no more slots than a wave has items.
+      const int j0 = __builtin_amdgcn_readfirstlane(wave);
+      const int count = (run.je - run.js) * chunks_of(a);
+      constexpr int kMost = kMfPairs<D, G, true>;
+      const int slots = slots_for(count, NW, kMost);
+      if (a.sel.dtype != LKV_INT8_RECORD) {
+        attend_run_mf<D, MT, G, RawMf<D, MT>, 2, NW>(a, run, idx_h, sel_base, j0, count, h, qb, lane, r, c, sp, st);
+      } else if (slots == 1) {
+        attend_run_mf<D, MT, G, RecMf<D>, 1, NW>(a, run, idx_h, sel_base, j0, count, h, qb, lane, r, c, sp, st);
+      } else if (slots == 2 || kMost == 2) {
+        attend_run_mf<D, MT, G, RecMf<D>, 2, NW>(a, run, idx_h, sel_base, j0, count, h, qb, lane, r, c, sp, st);
       } else {
-        attend_run_mf<D, MT, G, RawMf<D, MT>, NW>(a, idx_h, sel_base, j0, run.je, h, qb, lane, r, c, sp, st);
+        attend_run_mf<D, MT, G, RecMf<D>, kMost, NW>(a, run, idx_h, sel_base, j0, count, h, qb, lane, r, c, sp, st);
       }
       if (end_block >= 0) {  // wave-uniform
         if (kEarlyEnd && a.bs <= 16) {
-          if constexpr (kEarlyEnd) consume_mf<D, MT, G, 1>(qb, end_raw, a.qscale, 0, end_lim, lane, r, sp, st);
+          if constexpr (kEarlyEnd) consume_mf<D, MT, G, 1>(qb, end_raw, a.qscale, end_lim, lane, r, sp, st);
         } else {
           const Src es[1] = {end_src};
           const int eb[1] = {end_block};
@@ -1223,13 +1270,17 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
       // Every item of the run -- the sink, selected ids, the current block -- is a 16-bit
       // pair, so each wave takes kMfPairs of them per round, all loads in flight together: with
       // about two items per wave in the HBM plan, the wave that holds a third needs no second
-      // round. A run of at most two a wave leaves the third out.
+      // round.
       const int wv = __builtin_amdgcn_readfirstlane(wave);
-      const int count = run.sink + (run.je - run.js) + run.cur;
-      if (count <= 2 * NW) {
+      const int count = (run.sink + (run.je - run.js) + run.cur) * chunks_of(a);
+      constexpr int kMost = kMfPairs<D, G, false>;
+      const int slots = slots_for(count, NW, kMost);
+      if (slots == 1) {
+        attend_items_mf<D, MT, G, 1, NW>(a, run, idx_h, sel_base, wv, count, h, qb, lane, r, c, sp, st);
+      } else if (slots == 2 || kMost == 2) {
         attend_items_mf<D, MT, G, 2, NW>(a, run, idx_h, sel_base, wv, count, h, qb, lane, r, c, sp, st);
       } else {
-        attend_items_mf<D, MT, G, kMfPairs<D, G, false>, NW>(a, run, idx_h, sel_base, wv, count, h, qb, lane, r, c, sp, st);
+        attend_items_mf<D, MT, G, kMost, NW>(a, run, idx_h, sel_base, wv, count, h, qb, lane, r, c, sp, st);
       }
     } else {
       if (has_sink && first == 0 && wave == 0) attend_two<D, MT, G, I8>(a, a.sink, a.sink_block, -1, h, a.bs, q, r, c, st);
@@ -1576,7 +1627,8 @@ static void plan_matrix(Plan& p, const lkv_decode_desc* d, int cus) {
   const int n_sel = d->attend_selected ? d->k : 0;
   const int per_head = cus / d->n_kv > 1 ? cus / d->n_kv : 1;
   p.per_a = (n_sel + per_head - 1) / per_head;
-  if (p.per_a < kThreadsHbm / 64) p.per_a = kThreadsHbm / 64;
+  const int nch = (d->block_size + 15) / 16, least = (kThreadsHbm / 64 + nch - 1) / nch;  // a chunk per wave
+  if (p.per_a < least) p.per_a = least;
   p.splits_a = p.n_a > 0 ? (n_sel > 0 ? (n_sel + p.per_a - 1) / p.per_a : 1) : 0;
 }
 
