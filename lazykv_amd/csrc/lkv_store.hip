@@ -322,8 +322,19 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
   using R = Rows<D, MT>;
   const int lane = threadIdx.x & 63;
   const int r = lane / R::LPR, c = lane % R::LPR;
-  const int b = a.first_block + (int)(pair / a.n_kv);
-  const int h = (int)(pair % a.n_kv);
+  // A workgroup's four waves take four consecutive blocks of one head, contiguous in a dense cache: a pair per
+  // head in turn, they read and wrote at the heads' strides, a power of two apart, at once (a float16 layer of
+  // 32K tokens into a pool, dense [h, T, 64] source: 30.2 -> 23.4 us; pool to pool 47.6 -> 46.2).
+  static_assert(kWaves == 4, "four blocks of a head per workgroup");
+  const int64_t quad = (int64_t)a.n_kv * kWaves;
+  int b, h;
+  if ((pair / quad + 1) * kWaves <= a.n_blocks) {
+    b = a.first_block + (int)(pair / quad) * kWaves + (int)(pair % kWaves);
+    h = (int)((pair % quad) / kWaves);
+  } else {
+    b = a.first_block + (int)(pair / a.n_kv);
+    h = (int)(pair % a.n_kv);
+  }
   const int bs = a.bs;
   constexpr bool kRange = META || MODE == MODE_INT8;  // the keys' range is wanted
   const auto lower = [](float p, float q) { return fminf(p, q); };
