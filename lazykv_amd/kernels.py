@@ -110,18 +110,18 @@ def dense_source(keys: torch.Tensor, values: torch.Tensor, block_size: int) -> S
     """Blocks of dense per-head KV `[1, h, T, d]` or `[h, T, d]` (a full cache, lazykv/cache.py:35-36;
     the exact tier's float32 mirror, lazykv/exact.py:131-140). Rows must be contiguous and the token
     stride must be head_dim."""
-    k = keys[0] if keys.ndim == 4 else keys
-    v = values[0] if values.ndim == 4 else values
-    if k.ndim != 3 or k.shape != v.shape or k.dtype != v.dtype:
-        raise ValueError(f"expected matching [h, T, d] keys/values, got {tuple(keys.shape)} / {tuple(values.shape)}")
-    d = k.shape[-1]
-    for t in (k, v):
-        if t.stride(-1) != 1 or t.stride(-2) != d:
-            raise ValueError("dense KV rows must be contiguous with a token stride of head_dim")
-    if k.stride(0) != v.stride(0):
+    # Shapes and strides of the last three dimensions: a view of each tensor's first entry costs microseconds.
+    ks, vs = tuple(keys.shape), tuple(values.shape)
+    if len(ks) not in (3, 4) or len(vs) not in (3, 4) or ks[-3:] != vs[-3:] or keys.dtype != values.dtype or 0 in (ks[0], vs[0]):
+        raise ValueError(f"expected matching [h, T, d] keys/values, got {ks} / {vs}")
+    d = ks[-1]
+    kst, vst = keys.stride(), values.stride()
+    if kst[-1] != 1 or kst[-2] != d or vst[-1] != 1 or vst[-2] != d:
+        raise ValueError("dense KV rows must be contiguous with a token stride of head_dim")
+    if kst[-3] != vst[-3]:
         raise ValueError("keys and values must share their head stride")
-    code = _lib.dtype_code(k.dtype)
-    return Source(address(k), address(v), block_size * d, k.stride(0), code, code, k.shape[1] // block_size, (keys, values), _location(k))
+    code = _lib.dtype_code(keys.dtype)
+    return Source(address(keys), address(values), block_size * d, kst[-3], code, code, ks[-2] // block_size, (keys, values), _location(keys))
 
 
 # -- a1 + a2: bound and top-K -----------------------------------------------------------------------
@@ -129,13 +129,14 @@ def dense_source(keys: torch.Tensor, values: torch.Tensor, block_size: int) -> S
 
 def _meta_layout(kmin: torch.Tensor, kmax: torch.Tensor) -> tuple[int, int, int, int]:
     """(n_kv, n_blocks, head_dim, head_stride) of `[1, h, n, d]` or `[h, n, d]` metadata views."""
-    a = kmin[0] if kmin.ndim == 4 else kmin
-    b = kmax[0] if kmax.ndim == 4 else kmax
-    if a.ndim != 3 or a.shape != b.shape or a.dtype != b.dtype:
-        raise ValueError(f"kmin/kmax must be matching [1, h, n, d] tensors, got {tuple(kmin.shape)} / {tuple(kmax.shape)}")
-    if a.stride() != b.stride() or a.stride(-1) != 1 or a.stride(-2) != a.shape[-1]:
+    # Shapes and strides of the last three dimensions, as in dense_source.
+    a, b = tuple(kmin.shape), tuple(kmax.shape)
+    if len(a) not in (3, 4) or len(b) not in (3, 4) or a[-3:] != b[-3:] or kmin.dtype != kmax.dtype or 0 in (a[0], b[0]):
+        raise ValueError(f"kmin/kmax must be matching [1, h, n, d] tensors, got {a} / {b}")
+    sa, sb = kmin.stride()[-3:], kmax.stride()[-3:]
+    if sa != sb or sa[2] != 1 or sa[1] != a[-1]:
         raise ValueError("kmin/kmax rows must be contiguous, with equal strides")
-    return a.shape[0], a.shape[1], a.shape[2], a.stride(0)
+    return a[-3], a[-2], a[-1], sa[0]
 
 
 def bound_topk(
@@ -174,8 +175,8 @@ def bound_topk(
         raise ValueError("out_idx must be int32 [h, >=k] with contiguous rows")
     if out_bound is not None and (out_bound.dtype != torch.float32 or tuple(out_bound.shape) != (n_kv, n_cand) or not out_bound.is_contiguous()):
         raise ValueError(f"out_bound must be contiguous float32 [{n_kv}, {n_cand}]")
-    meta_base = address(kmin[0] if kmin.ndim == 4 else kmin)
-    meta_max = address(kmax[0] if kmax.ndim == 4 else kmax)
+    meta_base = address(kmin)
+    meta_max = address(kmax)
     ws = ws or default_workspace(q.device)
     ws_ptr, ws_n = ws.get(_lib.lib().lkv_bound_topk_workspace_bytes(n_kv, n_cand, k))
     rc = _lib.lib().lkv_bound_topk(
@@ -284,8 +285,8 @@ class PreparedSelectDecode:
         refs = [ctypes.byref(c) if c is not None else None for c in self._c]
         self._keep = (q, kmin, kmax, out, lse, out_idx, ws.buf, sel, sink, cur)
         self._fn = _lib.lib().lkv_select_decode
-        self._head = (ctypes.byref(self.desc), qq.data_ptr(), _lib.dtype_code(qq.dtype), address(kmin[0] if kmin.ndim == 4 else kmin),
-                      address(kmax[0] if kmax.ndim == 4 else kmax), _lib.dtype_code(kmin.dtype), hs, cand_offset)
+        self._head = (ctypes.byref(self.desc), qq.data_ptr(), _lib.dtype_code(qq.dtype), address(kmin),
+                      address(kmax), _lib.dtype_code(kmin.dtype), hs, cand_offset)
         self._tail = (rank_mode, refs[0], refs[1], refs[2], out.data_ptr(), _lib.dtype_code(out.dtype), lse.data_ptr(),
                       out_idx.data_ptr() if out_idx is not None else None, k, ws_ptr, ws_n)
         self.n_cand = n_cand
@@ -487,8 +488,8 @@ class PreparedSelectHybridDecode:
         refs = [ctypes.byref(c) if c is not None else None for c in self._c]
         self._keep = (q, kmin, kmax, out, lse, out_idx, ws.buf, host, res, sink, cur, rem)
         self._fn = _lib.lib().lkv_select_hybrid_decode
-        self._head = (ctypes.byref(self.desc), qq.data_ptr(), _lib.dtype_code(qq.dtype), address(kmin[0] if kmin.ndim == 4 else kmin),
-                      address(kmax[0] if kmax.ndim == 4 else kmax), _lib.dtype_code(kmin.dtype), hs, cand_offset)
+        self._head = (ctypes.byref(self.desc), qq.data_ptr(), _lib.dtype_code(qq.dtype), address(kmin),
+                      address(kmax), _lib.dtype_code(kmin.dtype), hs, cand_offset)
         self._tail = (rank_mode, refs[0], refs[1], ctypes.byref(self._tables), refs[2], refs[3], refs[4], out.data_ptr(), _lib.dtype_code(out.dtype),
                       lse.data_ptr(), out_idx.data_ptr() if out_idx is not None else None, k, ws_ptr, ws_n)
         self.n_cand = n_cand
@@ -643,7 +644,7 @@ class PreparedBoundTopk:
         ws_ptr, ws_n = ws.get(_lib.lib().lkv_bound_topk_workspace_bytes(n_kv, n_cand, k))
         self._keep = (q, kmin, kmax, out_idx, out_bound, ws.buf)
         self._fn = _lib.lib().lkv_bound_topk
-        self._args = (qq.data_ptr(), _lib.dtype_code(qq.dtype), address(kmin[0] if kmin.ndim == 4 else kmin), address(kmax[0] if kmax.ndim == 4 else kmax),
+        self._args = (qq.data_ptr(), _lib.dtype_code(qq.dtype), address(kmin), address(kmax),
                       _lib.dtype_code(kmin.dtype), hs, qq.shape[0], n_kv, d, cand_offset, n_cand, k, rank_mode, 0,
                       out_idx.data_ptr() if out_idx is not None else None, max(k, 1), out_bound.data_ptr() if out_bound is not None else None, ws_ptr, ws_n)
         self.device = q.device
