@@ -253,6 +253,25 @@ int lkv_store_blocks(uintptr_t stream, const lkv_kv_source* src, const lkv_kv_so
                      int block_size, int first_block, int n_blocks, void* kmin, void* kmax, int meta_dtype,
                      int64_t meta_head_stride);
 
+/* Small row copies in one launch: the token rows a tier moves around its stores -- the sink, the current
+ * block and a turn's tokens into a dense buffer (lazykv/tiered.py:334-351), a prompt's sink and tail into their slots
+ * (lazykv/tiered.py:198-206) -- where the reference makes one copy each. Copy i moves `rows` rows of
+ * `row_bytes` bytes for each of `heads` heads; strides in bytes, row_bytes and all addresses multiples of 2, device
+ * memory (or mapped host memory) on both sides; source and destination rows of one call do not overlap. rows == 0
+ * copies nothing. At most LKV_MAX_ROW_COPIES copies. */
+#define LKV_MAX_ROW_COPIES 8
+typedef struct lkv_row_copy {
+  const void* src;
+  void* dst;
+  int64_t src_head_stride;
+  int64_t src_row_stride;
+  int64_t dst_head_stride;
+  int64_t dst_row_stride;
+  int32_t rows;
+  int32_t row_bytes;
+} lkv_row_copy;
+int lkv_copy_rows(uintptr_t stream, const lkv_row_copy* copies, int n, int heads);
+
 /* quant.py pack: pairs [m, 2, bs, d] (dtype) -> records [m, P] (lazykv/quant.py:73-87) */
 int lkv_pack_int8(uintptr_t stream, const void* pairs, int dtype, int64_t m, int block_size, int head_dim,
                   void* records);

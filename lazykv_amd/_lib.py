@@ -100,6 +100,21 @@ class ResidencyTables(ctypes.Structure):
     ]
 
 
+class RowCopy(ctypes.Structure):
+    """lkv_row_copy: one small row copy (see include/lazykv_hip.h)."""
+
+    _fields_ = [
+        ("src", ctypes.c_void_p),
+        ("dst", ctypes.c_void_p),
+        ("src_head_stride", ctypes.c_int64),
+        ("src_row_stride", ctypes.c_int64),
+        ("dst_head_stride", ctypes.c_int64),
+        ("dst_row_stride", ctypes.c_int64),
+        ("rows", ctypes.c_int32),
+        ("row_bytes", ctypes.c_int32),
+    ]
+
+
 _P = ctypes.c_void_p
 _I = ctypes.c_int
 _I64 = ctypes.c_int64
@@ -147,6 +162,7 @@ SIGNATURES: dict[str, tuple] = {
     ),
     "lkv_merge_lse": (_I, [_U, _P, _P, _P, _P, _I, _I64, _I, _P, _I, _P]),
     "lkv_store_blocks": (_I, [_U, ctypes.POINTER(KVSource), ctypes.POINTER(KVSource), _I, _I, _I, _I, _I, _P, _P, _I, _I64]),
+    "lkv_copy_rows": (_I, [_U, ctypes.POINTER(RowCopy), _I, _I]),
     "lkv_pack_int8": (_I, [_U, _P, _I, _I64, _I, _I, _P]),
     "lkv_unpack_int8": (_I, [_U, _P, _I64, _I, _I, _I, _P]),
     "lkv_packed_pair_bytes": (_I64, [_I, _I]),

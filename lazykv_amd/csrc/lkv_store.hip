@@ -606,6 +606,67 @@ extern "C" int lkv_store_blocks(uintptr_t stream, const lkv_kv_source* src, cons
   return head_dim == 128 ? launch_store_mt<128>(s, mt, mode, a, max_wgs) : launch_store_mt<64>(s, mt, mode, a, max_wgs);
 }
 
+// ---- small row copies -----------------------------------------------------------------------------------
+// Up to 8 copies in one launch, a workgroup per 256 words of one copy's rows of one head. They are bound by the
+// launch: with six separate copies behind its store, a 200-token turn over a 64K-token tier (8 heads, d 128) took
+// 120.7 us, with one launch 102.6. (For two copies, torch's cost the host less: appending a token 17.2 us against 18.3.)
+namespace {
+
+struct RowCopies {
+  lkv_row_copy c[LKV_MAX_ROW_COPIES];
+};
+
+template <typename W>
+__global__ __launch_bounds__(256) void copy_rows_kernel(RowCopies a) {
+  const lkv_row_copy& c = a.c[blockIdx.z];
+  const int words = c.row_bytes / (int)sizeof(W);
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (int64_t)c.rows * words) return;
+  const int64_t row = i / words, w = i % words;
+  const char* s = (const char*)c.src + blockIdx.y * c.src_head_stride + row * c.src_row_stride;
+  char* d = (char*)c.dst + blockIdx.y * c.dst_head_stride + row * c.dst_row_stride;
+  ((W*)d)[w] = ((const W*)s)[w];
+}
+
+}  // namespace
+
+extern "C" int lkv_copy_rows(uintptr_t stream, const lkv_row_copy* copies, int n, int heads) {
+  LKV_CHECK_ARG(n >= 0 && n <= LKV_MAX_ROW_COPIES, "%d row copies: at most %d", n, LKV_MAX_ROW_COPIES);
+  LKV_CHECK_ARG(n == 0 || copies != nullptr, "NULL pointer");
+  LKV_CHECK_ARG(heads > 0 && heads <= 65535, "bad head count %d", heads);
+  RowCopies a{};
+  int used = 0;
+  int64_t most = 0;
+  uint64_t mix = 0;  // the low bits set anywhere decide the word
+  for (int i = 0; i < n; ++i) {
+    const lkv_row_copy& c = copies[i];
+    LKV_CHECK_ARG(c.rows >= 0 && c.row_bytes >= 0, "negative size");
+    if (c.rows == 0 || c.row_bytes == 0) continue;
+    LKV_CHECK_ARG(c.src != nullptr && c.dst != nullptr, "NULL pointer");
+    mix |= (uint64_t)(uintptr_t)c.src | (uint64_t)(uintptr_t)c.dst | (uint64_t)c.src_head_stride | (uint64_t)c.src_row_stride |
+           (uint64_t)c.dst_head_stride | (uint64_t)c.dst_row_stride | (uint64_t)c.row_bytes;
+    a.c[used++] = c;
+    const int64_t bytes = (int64_t)c.rows * c.row_bytes;
+    if (bytes > most) most = bytes;
+  }
+  LKV_CHECK_ARG((mix & 1) == 0, "row copies move whole 2-byte elements");
+  if (used == 0) return LKV_OK;
+  const int word = (mix & 15) == 0 ? 16 : (mix & 3) == 0 ? 4 : 2;
+  const int64_t groups = (most / word + 255) / 256;
+  LKV_CHECK_ARG(groups <= 0x7fffffff, "row copy too large");
+  const dim3 grid((unsigned)groups, (unsigned)heads, (unsigned)used);
+  hipStream_t s = (hipStream_t)stream;
+  if (word == 16) {
+    hipLaunchKernelGGL(copy_rows_kernel<uint4>, grid, dim3(256), 0, s, a);
+  } else if (word == 4) {
+    hipLaunchKernelGGL(copy_rows_kernel<uint32_t>, grid, dim3(256), 0, s, a);
+  } else {
+    hipLaunchKernelGGL(copy_rows_kernel<uint16_t>, grid, dim3(256), 0, s, a);
+  }
+  LKV_CHECK_LAUNCH("copy_rows");
+  return LKV_OK;
+}
+
 extern "C" int lkv_pack_int8(uintptr_t stream, const void* pairs, int dtype, int64_t m, int block_size, int head_dim,
                              void* records) {
   LKV_CHECK_ARG(pairs != nullptr && records != nullptr, "NULL pointer");

@@ -588,6 +588,27 @@ def store_blocks(
     _lib.check(rc, "store_blocks")
 
 
+def copy_rows(copies: list[tuple[torch.Tensor, torch.Tensor]]) -> None:
+    """`dst.copy_(src)` for each (dst, src) of `[h, rows, d]` views, up to 8 of them in one launch (lkv_copy_rows) on
+    the current stream. A copy the launch does not cover -- another shape, dtype or device, rows that are not contiguous,
+    a source that autograd follows -- is torch's."""
+    first = copies[0][0]
+    here = first.is_cuda and first.device.index == torch.cuda.current_device()
+    descs = []
+    for dst, src in copies:
+        ds, ss = dst.stride(), src.stride()
+        if (not here or dst.shape != src.shape or src.dtype != dst.dtype or src.device != first.device or dst.device != first.device
+                or ds[-1] != 1 or ss[-1] != 1 or dst.shape[0] != first.shape[0] or src.requires_grad):
+            dst.copy_(src)
+            continue
+        es = dst.element_size()
+        _, rows, d = dst.shape
+        descs.append(_lib.RowCopy(src.data_ptr(), dst.data_ptr(), ss[0] * es, ss[1] * es, ds[0] * es, ds[1] * es, rows, d * es))
+    if descs:
+        arr = (_lib.RowCopy * len(descs))(*descs)
+        _lib.check(_lib.lib().lkv_copy_rows(_lib.stream_of(first), arr, len(descs), first.shape[0]), "copy_rows")
+
+
 def packed_pair_bytes(block_size: int, head_dim: int) -> int:
     return int(_lib.lib().lkv_packed_pair_bytes(block_size, head_dim))
 

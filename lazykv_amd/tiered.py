@@ -231,11 +231,10 @@ class TieredLayer:
         if self._prompt_sealed != n_blocks:
             raise ValueError(f"{self._prompt_sealed} of the prompt's {n_blocks} full blocks are sealed")
         # The sink never leaves VRAM and stays exact even under an int8 tier (lazykv/tiered.py:200-202).
-        self.pool[0, :, 0].copy_(keys[0, :, : self.bs])
-        self.pool[0, :, 1].copy_(values[0, :, : self.bs])
+        ends = [(self.pool[0, :, 0], keys[0, :, : self.bs]), (self.pool[0, :, 1], values[0, :, : self.bs])]
         if tail:
-            self.pool[1, :, 0, :tail].copy_(keys[0, :, n_blocks * self.bs : length])
-            self.pool[1, :, 1, :tail].copy_(values[0, :, n_blocks * self.bs : length])
+            ends += [(self.pool[1, :, 0, :tail], keys[0, :, n_blocks * self.bs : length]), (self.pool[1, :, 1, :tail], values[0, :, n_blocks * self.bs : length])]
+        kernels.copy_rows(ends)
         self.n_sealed, self.fill, self.length = n_blocks, tail, length
         self._seed_slots()
 
@@ -484,14 +483,14 @@ class TieredLayer:
             kernels.store_blocks(src, dst=dst, n_kv=self.h, head_dim=self.d, block_size=bs, first_block=0, n_blocks=n)
             if self.store is None:
                 moved = n * self.h * self.pair_bytes
-            sk[0, :, :bs].copy_(self.pool[0, :, 0])
-            sv[0, :, :bs].copy_(self.pool[0, :, 1])
+        # The sink over block 0, the current block and the new tokens: one launch.
         a = n * bs
+        parts = []
+        if n:
+            parts += [(sk[0, :, :bs], self.pool[0, :, 0]), (sv[0, :, :bs], self.pool[0, :, 1])]
         if self.fill:
-            sk[0, :, a : a + self.fill].copy_(self.pool[1, :, 0, : self.fill])
-            sv[0, :, a : a + self.fill].copy_(self.pool[1, :, 1, : self.fill])
-        sk[0, :, a + self.fill : total].copy_(keys[0])
-        sv[0, :, a + self.fill : total].copy_(values[0])
+            parts += [(sk[0, :, a : a + self.fill], self.pool[1, :, 0, : self.fill]), (sv[0, :, a : a + self.fill], self.pool[1, :, 1, : self.fill])]
+        kernels.copy_rows(parts + [(sk[0, :, a + self.fill : total], keys[0]), (sv[0, :, a + self.fill : total], values[0])])
         return sk[:, :, :total], sv[:, :, :total], moved
 
     def _seal(self, counters: TierCounters | None) -> None:
