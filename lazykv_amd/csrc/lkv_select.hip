@@ -614,6 +614,7 @@ constexpr int kSelBlockCap = kSelBlockThreads * 12;
 template <int KPT, bool SORTED>
 __global__ __launch_bounds__(kSelBlockThreads) void select_block_kernel(const float* __restrict__ bounds, int64_t bstride,
                                                                         int n_cand, int k, int cand_offset,
+                                                                        const int32_t* __restrict__ map,
                                                                         int32_t* __restrict__ out_idx, int64_t idx_stride) {
   static_assert(kSelBlockThreads == kSelThreads, "the sort's thread count");
   __shared__ lkv::SelectLds<kSelBlockThreads, KPT> L;
@@ -621,9 +622,13 @@ __global__ __launch_bounds__(kSelBlockThreads) void select_block_kernel(const fl
   const float* row = bounds + (int64_t)h * bstride;
   const lkv::SelectPick pk = lkv::block_top_k<kSelBlockThreads, KPT, true>(row, true, n_cand, k, L);
   int32_t* out_h = out_idx + (int64_t)h * idx_stride;
+  const int32_t* map_h = map != nullptr ? map + (int64_t)h * bstride : nullptr;  // candidates of the parts below
   int pos = pk.pos;
   if constexpr (!SORTED) {
-    for (uint32_t take = pk.take; take != 0u && pos < k; take &= take - 1u, ++pos) out_h[pos] = pk.i0 + __ffs((int)take) - 1 + cand_offset;
+    for (uint32_t take = pk.take; take != 0u && pos < k; take &= take - 1u, ++pos) {
+      const int i = pk.i0 + __ffs((int)take) - 1;
+      out_h[pos] = (map_h != nullptr ? map_h[i] : i) + cand_offset;
+    }
   } else {
     __shared__ SortLds sort;
     int np2 = 64;
@@ -631,7 +636,8 @@ __global__ __launch_bounds__(kSelBlockThreads) void select_block_kernel(const fl
     for (int i = k + threadIdx.x; i < np2; i += kSelThreads) sort.slot[0][i] = 0u;
     for (uint32_t take = pk.take; take != 0u && pos < k; take &= take - 1u, ++pos) {
       const int i = pk.i0 + __ffs((int)take) - 1;
-      sort.slot[0][pos] = ((uint64_t)lkv::orderable_key(row[i]) << 32) | (uint64_t)(0xffffffffu - (uint32_t)i);
+      const uint32_t id = map_h != nullptr ? (uint32_t)map_h[i] : (uint32_t)i;
+      sort.slot[0][pos] = ((uint64_t)lkv::orderable_key(row[i]) << 32) | (uint64_t)(0xffffffffu - id);
     }
     __syncthreads();
     write_sorted(sort, np2, k, cand_offset, out_h);
@@ -653,6 +659,39 @@ __global__ __launch_bounds__(kSelThreads) void select_kernel(const float* __rest
   __shared__ SelectRowLds L;
   select_row<false>(bounds + (int64_t)blockIdx.x * bstride, n_cand, k, cand_offset, sorted, out_idx + (int64_t)blockIdx.x * idx_stride, L);
 }
+
+// ---- long rows in parts -----------------------------------------------------------------------------
+// A row of more than kSelBlockCap candidates as parts of kPartCand, one workgroup each: a part's own best k (by the
+// same rule, in ascending order) are the only ones of it that can be among the row's, so the row's selection is
+// that of the parts' picks, one list in ascending order, of at most kSelBlockCap. One workgroup per head reading the
+// whole row three times is bound by that CU's vector work. 1,024 of 65,535 for eight heads, with the bound launch
+// at head_dim 64: 42.8 -> 34.7 us ascending, 51.1 -> 41.8 descending. Two parts gain nothing (1,024 of 16,382: 19.7
+// and 20.0), so rows of up to two stay whole.
+constexpr int kPartCand = kSelBlockThreads * 8;
+__global__ __launch_bounds__(kSelBlockThreads) void select_part_kernel(const float* __restrict__ bounds, int64_t bstride, int n_kv, int n_cand,
+                                                                       int k, float* __restrict__ part_key, int32_t* __restrict__ part_id,
+                                                                       int64_t pstride) {
+  __shared__ lkv::SelectLds<kSelBlockThreads, 8> L;
+  const int h = blockIdx.x % n_kv, part = blockIdx.x / n_kv;
+  const int first = part * kPartCand, m = min(kPartCand, n_cand - first), kk = min(k, m);
+  const float* row = bounds + (int64_t)h * bstride + first;
+  const lkv::SelectPick pk = lkv::block_top_k<kSelBlockThreads, 8, true>(row, true, m, kk, L);
+  const int64_t at = (int64_t)h * pstride + (int64_t)part * k;
+  int pos = pk.pos;
+  for (uint32_t take = pk.take; take != 0u && pos < kk; take &= take - 1u, ++pos) {
+    const int i = pk.i0 + __ffs((int)take) - 1;
+    part_key[at + pos] = row[i];
+    part_id[at + pos] = first + i;
+  }
+}
+
+// The parts' picks of one head (0: the row is not selected in parts), and the floats between heads' lists.
+static int part_picks(int n_cand, int k) {
+  if (n_cand <= 2 * kPartCand || k <= 0) return 0;
+  const int64_t picks = (int64_t)((n_cand + kPartCand - 1) / kPartCand) * k;
+  return picks <= kSelBlockCap ? (int)picks : 0;
+}
+static size_t part_stride(int n_cand, int k) { return lkv_align_up((size_t)part_picks(n_cand, k), 4); }
 
 template <int D, int MT, int G>
 int launch_bound(hipStream_t stream, const void* q, int q_dtype, const void* kmin, const void* kmax, int64_t mhs, int n_kv,
@@ -689,10 +728,12 @@ int dispatch_g(int g, hipStream_t s, const void* q, int qd, const void* kmin, co
 
 }  // namespace
 
+static size_t bound_rows_bytes(int n_kv, int n_cand) { return lkv_align_up((size_t)n_kv * lkv_align_up((size_t)n_cand, 4) * 4, 256); }
+
+// The bound rows, and the parts' picks where a selection of k takes parts.
 extern "C" size_t lkv_bound_topk_workspace_bytes(int n_kv, int n_cand, int k) {
-  (void)k;
   if (n_kv <= 0 || n_cand <= 0) return 0;
-  return lkv_align_up((size_t)n_kv * lkv_align_up((size_t)n_cand, 4) * 4, 256);
+  return bound_rows_bytes(n_kv, n_cand) + lkv_align_up(2 * (size_t)n_kv * part_stride(n_cand, k) * 4, 256);
 }
 
 int lkv_launch_bounds(hipStream_t s, const void* q, int q_dtype, const void* kmin, const void* kmax, int meta_dtype,
@@ -713,26 +754,41 @@ int lkv_launch_bounds(hipStream_t s, const void* q, int q_dtype, const void* kmi
 int lkv_select_max_candidates() { return kMaxStreamCand; }
 
 // Up to kSelBlockCap candidates in rows that can be read as vectors: the in-workgroup top-K, which reads the
-// row once. Any other selection reads it three times, as 16-byte vectors where the rows allow.
+// row once. A longer one in parts where `parts` (2 * n_kv * part_stride words) is given and the parts' picks fit the
+// in-workgroup top-K. Any other selection reads the row three times, as 16-byte vectors where the rows allow.
 template <int KPT>
 static void launch_select_block(hipStream_t s, const float* bounds, int64_t bstride, int n_kv, int n_cand, int k, int cand_offset, int sorted,
-                                int32_t* out_idx, int64_t idx_stride) {
+                                const int32_t* map, int32_t* out_idx, int64_t idx_stride) {
   if (sorted) {
     hipLaunchKernelGGL((select_block_kernel<KPT, true>), dim3(n_kv), dim3(kSelBlockThreads), 0, s, bounds, bstride, n_cand, k, cand_offset,
-                       out_idx, idx_stride);
+                       map, out_idx, idx_stride);
   } else {
     hipLaunchKernelGGL((select_block_kernel<KPT, false>), dim3(n_kv), dim3(kSelBlockThreads), 0, s, bounds, bstride, n_cand, k, cand_offset,
-                       out_idx, idx_stride);
+                       map, out_idx, idx_stride);
   }
 }
 
 static int launch_select(hipStream_t s, const float* bounds, int64_t bstride, int n_kv, int n_cand, int k, int cand_offset, int sorted,
-                         int32_t* out_idx, int64_t idx_stride) {
+                         void* parts, int32_t* out_idx, int64_t idx_stride) {
   const bool vec = rows_vector_readable(bounds, bstride, n_cand);
   if (vec && n_cand <= kSelBlockThreads * 8) {
-    launch_select_block<8>(s, bounds, bstride, n_kv, n_cand, k, cand_offset, sorted, out_idx, idx_stride);
+    launch_select_block<8>(s, bounds, bstride, n_kv, n_cand, k, cand_offset, sorted, nullptr, out_idx, idx_stride);
   } else if (vec && n_cand <= kSelBlockCap) {
-    launch_select_block<12>(s, bounds, bstride, n_kv, n_cand, k, cand_offset, sorted, out_idx, idx_stride);
+    launch_select_block<12>(s, bounds, bstride, n_kv, n_cand, k, cand_offset, sorted, nullptr, out_idx, idx_stride);
+  } else if (vec && parts != nullptr && part_picks(n_cand, k) > 0) {
+    const int n_parts = (n_cand + kPartCand - 1) / kPartCand;
+    const int64_t ps = (int64_t)part_stride(n_cand, k);
+    float* key = (float*)parts;
+    int32_t* id = (int32_t*)(key + n_kv * ps);
+    hipLaunchKernelGGL(select_part_kernel, dim3(n_kv * n_parts), dim3(kSelBlockThreads), 0, s, bounds, bstride, n_kv, n_cand, k, key, id, ps);
+    // Only the last part can hold fewer than k candidates.
+    const int last = n_cand - (n_parts - 1) * kPartCand;
+    const int picks = (n_parts - 1) * k + (last < k ? last : k);
+    if (picks <= kSelBlockThreads * 8) {
+      launch_select_block<8>(s, key, ps, n_kv, picks, k, cand_offset, sorted, id, out_idx, idx_stride);
+    } else {
+      launch_select_block<12>(s, key, ps, n_kv, picks, k, cand_offset, sorted, id, out_idx, idx_stride);
+    }
   } else if (vec) {
     hipLaunchKernelGGL(select_stream_kernel, dim3(n_kv), dim3(kSelThreads), 0, s, bounds, bstride, n_cand, k, cand_offset, sorted, out_idx,
                        idx_stride);
@@ -746,7 +802,7 @@ static int launch_select(hipStream_t s, const float* bounds, int64_t bstride, in
 
 int lkv_launch_select(hipStream_t s, const float* bounds, int64_t bstride, int n_kv, int n_cand, int k, int cand_offset,
                       int32_t* out_idx, int64_t idx_stride) {
-  return launch_select(s, bounds, bstride, n_kv, n_cand, k, cand_offset, 0, out_idx, idx_stride);
+  return launch_select(s, bounds, bstride, n_kv, n_cand, k, cand_offset, 0, nullptr, out_idx, idx_stride);
 }
 
 extern "C" int lkv_bound_topk(uintptr_t stream, const void* q, int q_dtype, const void* kmin, const void* kmax,
@@ -777,17 +833,20 @@ extern "C" int lkv_bound_topk(uintptr_t stream, const void* q, int q_dtype, cons
   // a caller's out_bound is dense [n_kv, n_cand].
   float* bounds = out_bound;
   int64_t bstride = n_cand;
+  void* parts = nullptr;
   if (bounds == nullptr) {
-    const size_t need = lkv_bound_topk_workspace_bytes(n_kv, n_cand, k);
+    const size_t need = bound_rows_bytes(n_kv, n_cand);
     LKV_CHECK_ARG(ws != nullptr && ws_bytes >= need, "workspace of %zu bytes needed, got %zu", need, ws_bytes);
     LKV_CHECK_ARG(((uintptr_t)ws & 15) == 0, "workspace must be 16-byte aligned");
     bounds = (float*)ws;
     bstride = (int64_t)lkv_align_up((size_t)n_cand, 4);
+    // A workspace sized for fewer blocks k than this call's holds no parts: the row is then read whole.
+    if (part_picks(n_cand, k) > 0 && ws_bytes >= lkv_bound_topk_workspace_bytes(n_kv, n_cand, k)) parts = (char*)ws + need;
   }
   const int g = n_q / n_kv;
   hipStream_t s = (hipStream_t)stream;
   const int rc = lkv_launch_bounds(s, q, q_dtype, kmin, kmax, meta_dtype, meta_head_stride, n_kv, g, head_dim, cand_offset, n_cand,
                                    rank_mode, bounds, bstride);
   if (rc != LKV_OK || k == 0) return rc;
-  return launch_select(s, bounds, bstride, n_kv, n_cand, k, cand_offset, sorted, out_idx, idx_stride);
+  return launch_select(s, bounds, bstride, n_kv, n_cand, k, cand_offset, sorted, parts, out_idx, idx_stride);
 }

@@ -55,7 +55,9 @@ def test_selection_in_one_workgroup_takes_the_best_k(n: int, k: int, kind: str) 
 
 # Around a wave's run of 256 candidates, the in-workgroup limit, and the largest count; k around whole powers
 # of two, the sort's own edges.
-LONG = [(3, 2), (255, 64), (257, 65), (4097, 1025), (8193, 700), (12289, 2048), (16640, 1), (65535, 1024), (262144, 2047)]
+# Beyond 16,384 candidates in parts of 8,192 while the parts' picks are at most 12,288 (a last part of one candidate, and of
+# fewer than k, among them), else in one pass over the row.
+LONG = [(3, 2), (255, 64), (257, 65), (4097, 1025), (8193, 700), (12289, 2048), (16385, 2000), (16640, 1), (24577, 2048), (65535, 1024), (65537, 1365), (262144, 384), (262144, 2047)]
 
 
 @pytest.mark.parametrize("kind", ["normal", "cluster", "one value", "sorted"])
