@@ -658,6 +658,10 @@ __device__ __forceinline__ void value_row(const RecMf<D>& raw, int i, float (&x)
   for (int e = 0; e < 8; ++e) x[e] = (float)(typename MfElem<MT>::T)Wd::deq(Wd::u8(w, e), sc, ze);
 }
 
+// 2^x for x <= 0 by the hardware's instruction alone. exp2f returns the same from 2^-126 up; below it, where exp2f spends
+// four more instructions on a subnormal result, this is 0: beside the weight 1 of the largest score.
+__device__ __forceinline__ float weight(float x) { return __builtin_amdgcn_exp2f(x); }
+
 // Fold a chunk (16 rows) of each of NP pairs into the wave's running softmax, as
 // consume_chunk does one at a time, with the scores from the matrix cores: one maximum, one
 // rescale and one broadcast for all NP of them. rows[u]: valid rows of chunk u (0 or less skips it).
@@ -695,14 +699,14 @@ __device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D /
   const float m_old = st.m;
   const float m_new = fmaxf(m_old, cm);
   const bool live = m_new != -INFINITY;  // false while nothing valid has been seen
-  const float alpha = m_old != -INFINITY ? exp2f(m_old - m_new) : 1.0f;  // nothing to rescale before the first valid chunk
+  const float alpha = m_old != -INFINITY ? weight(m_old - m_new) : 1.0f;  // nothing to rescale before the first valid chunk
   float p[NP][4];
   float ps = 0.0f;
 #pragma unroll
   for (int u = 0; u < NP; ++u)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      p[u][i] = (vld[u][i] && live) ? exp2f(sc[u][i] - m_new) : 0.0f;
+      p[u][i] = (vld[u][i] && live) ? weight(sc[u][i] - m_new) : 0.0f;
       ps += p[u][i];
     }
   ps = lkv::pair_sum<32>(lkv::pair_sum<16>(ps));
@@ -740,6 +744,7 @@ __device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D /
       float x[8];
       value_row<D, MT>(raw[u], i, x);
       if (part) {
+        asm volatile("");  // a branch: as selects, whole chunks would pay for them too
         const bool ok = row < rows[u];
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] = ok ? x[e] : 0.0f;  // their weights are 0
