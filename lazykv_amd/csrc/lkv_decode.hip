@@ -297,6 +297,10 @@ __device__ __forceinline__ void finish_raw(int t0, int r, RawI8<D>& raw) {
 template <int D, int MT>
 __device__ __forceinline__ void finish_raw(int, int, RawModel<D, MT>&) {}
 
+// 2^x for x <= 0 by the hardware's instruction alone. exp2f returns the same from 2^-126 up; below it, where exp2f spends
+// four more instructions on a subnormal result, this is 0: beside the weight 1 of the largest score.
+__device__ __forceinline__ float weight(float x) { return __builtin_amdgcn_exp2f(x); }
+
 // Per-row widening of a raw chunk: key row i / value row i of this lane's channels, as float.
 template <int D, int MT>
 struct Widen {
@@ -657,10 +661,6 @@ __device__ __forceinline__ void value_row(const RecMf<D>& raw, int i, float (&x)
 #pragma unroll
   for (int e = 0; e < 8; ++e) x[e] = (float)(typename MfElem<MT>::T)Wd::deq(Wd::u8(w, e), sc, ze);
 }
-
-// 2^x for x <= 0 by the hardware's instruction alone. exp2f returns the same from 2^-126 up; below it, where exp2f spends
-// four more instructions on a subnormal result, this is 0: beside the weight 1 of the largest score.
-__device__ __forceinline__ float weight(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // Fold a chunk (16 rows) of each of NP pairs into the wave's running softmax, as
 // consume_chunk does one at a time, with the scores from the matrix cores: one maximum, one
@@ -1404,7 +1404,7 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
     if (M != -INFINITY) {
 #pragma unroll
       for (int w = 0; w < NW; ++w) {
-        const float wt = exp2f(s_m[w][j] - M);
+        const float wt = weight(s_m[w][j] - M);
         O += s_o[w][j][dd] * wt;
         Lsum += s_l[w][j] * wt;
       }
