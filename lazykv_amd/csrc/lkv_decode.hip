@@ -18,8 +18,8 @@
 // once. A row's channels are spread over 16 lanes at d 128 and 8 lanes at d 64, 8 channels each
 // (Lanes<D>), so a wave-wide load of 16-byte lane segments covers 4 or 8 rows. Scores are DPP
 // sums over a row's lanes; the online softmax runs in base 2 with the scale folded into q. The
-// 8-wave model-dtype instances score on the matrix cores instead (MF, below), up to three pairs
-// per softmax step.
+// 8-wave instances with a model-dtype query run Q.K and P.V on the matrix cores instead (MF, below), over
+// 16-bit pairs or int8 records, several 16-row chunks per softmax step.
 //
 // Merge. Waves combine in LDS, workgroups write (m, l, o) partials to the workspace, and a second
 // launch folds each query head's partials into out and lse. (A last-arriver merge inside one
@@ -434,8 +434,8 @@ __device__ __forceinline__ void consume_chunk(const float (&q)[G][Lanes<D>::EPL]
 
 // Pairs a wave keeps in flight in the remainder segment of the vector-path instances: one
 // (measured on runs of consecutive blocks from HBM and from host memory, two were no faster). The
-// selected segment takes two in the 8-wave instances (four for int8 records), one in the 4-wave
-// general instance; the matrix-core instances take up to three in both segments.
+// selected segment takes two in the 8-wave vector instances, one in the 4-wave general instance; the
+// matrix-core instances take kMfPairs in both segments.
 template <int G>
 constexpr int kPairs = 1;
 
@@ -496,16 +496,20 @@ __device__ __forceinline__ void attend_two(const DecodeArgs& a, const Src& s, in
   process_two<D, MT, G, RawModel<D, MT>, NP>(a, s, block_a, block_b, h, limit, q, r, c, st);
 }
 
-// ---- Q.K on the matrix cores ---------------------------------------------------------------------
-// The 8-wave model-dtype instances score a 16-token chunk with one v_mfma_f32_16x16x32 per 32
+// ---- Q.K and P.V on the matrix cores ---------------------------------------------------------------
+// The 8-wave instances with a model-dtype query score a 16-token chunk with one v_mfma_f32_16x16x32 per 32
 // channels: A = the chunk's 16 key rows (lane l: row l % 16, channels 32s + 8 (l / 16) .. + 7),
 // B = the query rows of the KV head's G query heads, in the model dtype as given (lane l: head
 // l % 16, zero for heads >= G), D = scores (lane l: rows 4 (l / 16) + i, i < 4, of head l % 16).
 // Products of two model-dtype values are exact in float32 and are summed in float32, as in the
 // vector path; the softmax scale multiplies the sum. The online softmax of a head runs in the
-// lanes that hold its scores; the weights p, and each head's new maximum, rescale factor and
-// weight sum, reach the other lanes through a small per-wave LDS area, and P.V stays on the
-// vector ALUs in the layout of consume_chunk.
+// lanes that hold its scores; the weights p, and the heads' rescale factors where a maximum moved, reach the
+// other lanes through a small per-wave LDS area, and P.V takes the values where load_raw put them (consume_mf).
+// These launches are bound by the memory's time for the pairs plus a chain of phases, in which two waves per SIMD
+// issue the vector work: the selection, widening, softmax and combine. Per layer in a replayed step, P.V on the vector
+// ALUs (and for int8 records the whole product) -> here: 17.3 -> 15.4 us at 32K tokens (16 layers, float16, d 64, 512
+// pairs a head), 23.7 -> 19.4 with 1,024 int8 records at 64K, 27.6 -> 25.9 at the 8B shape; a dense decode of 128K tokens (bfloat16,
+// d 128) 97.0 -> 91.2 us, 5.9 TB/s.
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 template <int MT>
@@ -1641,7 +1645,9 @@ static void plan_matrix(Plan& p, const lkv_decode_desc* d, int cus) {
 // when the query has the model dtype and 16-byte aligned rows: one instance for 16-bit pairs, one that also
 // reads int8 records. Other queries (and float32 pools) take the 8-wave vector path for 16-bit and
 // float32 pairs of groups of up to 4 heads, and the 4-wave general instance over the same plan for the rest.
-// Host plans and hybrid launches take the 4-wave general instance. A fused-selection launch has
+// Host plans and hybrid launches take the 4-wave general instance (the link bounds them). Two layers in a replayed step,
+// 254 of 1,024 blocks of 16 tokens, general instance -> matrix cores: 8 heads of 8, bfloat16 d 128, 58.3 -> 39 us; int8 records,
+// 8 heads of 4 at d 128, 49.4 -> 39; the 8-wave vector path for records at d 64 took 36.1 where this takes 32.4. A fused-selection launch has
 // no 8-wave vector instance and takes the general one instead (lkv_select_decode then selects in its own
 // launch, so that it folds what the unfused call folds).
 enum class Inst { kGeneral, kVector8, kMatrix8, kMatrixRec8 };
