@@ -24,17 +24,17 @@ SRC_HOST = 1
 SELECT_IN_DECODE_MAX_CAND = 8192  # lkv_select_decode chooses the top K inside the decode launch up to this many candidates
 
 
-def selects_in_decode(n_cand: int, host: bool, group: int, int8: bool = False, head_dim: int = 128, model_query: bool = True) -> bool:  # noqa: ARG001
+def selects_in_decode(n_cand: int, host: bool, group: int, int8: bool = False, head_dim: int = 128, model_query: bool = True) -> bool:
     """Whether lkv_select_decode chooses the top K inside its decode launch, as the library decides.
     The decode launch must take the instance the unfused decode takes, and hold at most 16 candidates
     per thread, never beyond SELECT_IN_DECODE_MAX_CAND. Pairs or int8 records in HBM under a
     model-dtype query (`model_query`: the pools' dtype, 16-byte aligned) take 512-thread workgroups
-    on the matrix cores. Any other query over HBM takes 256 threads for int8 records and groups of
-    more than 4 heads, and for the rest an instance that does not select: its own launch does. A host
-    pool takes 256 threads."""
+    on the matrix cores. Any other query over HBM takes 512 for int8 records under groups of at most 4
+    (256 at head_dim 128 with a group of 4), 256 for larger groups, and for the rest an instance that
+    does not select: its own launch does. A host pool takes 256 threads."""
     threads = 256
     if not host:
-        if model_query:
+        if model_query or (int8 and group <= 4 and not (head_dim == 128 and group == 4)):
             threads = 512
         elif not int8 and group <= 4:
             return False

@@ -496,6 +496,50 @@ __device__ __forceinline__ void attend_two(const DecodeArgs& a, const Src& s, in
   process_two<D, MT, G, RawModel<D, MT>, NP>(a, s, block_a, block_b, h, limit, q, r, c, st);
 }
 
+// The selected pairs of an 8-wave vector int8 instance, four per wave per round: all four records' loads
+// are issued before the first is consumed (the HBM plan gives a wave about four), where the
+// two-per-round loop waits for a second round's loads after consuming its first two. The pairs and
+// the order they are consumed in are the two-per-round loop's, so the results are identical.
+// Blocks of at most 16 tokens (one chunk each). IDS_LDS: the ids are in LDS (a launch that selected
+// them itself), else in global memory; each is read through its own address space (a wait on a
+// generic read drains every load in flight).
+template <int D, int MT, int G, int NW, bool IDS_LDS>
+__device__ __forceinline__ void attend_selected_i8_four(const DecodeArgs& a, const int32_t* idx_h, int sel_base, int js, int je,
+                                                        int wave, int h, const float (&q)[G][Lanes<D>::EPL], int r, int c,
+                                                        WaveState<D, G>& st) {
+  using L = Lanes<D>;
+  const Src& s = a.sel;
+  const int nit = min(L::NI, (a.bs + L::RG - 1) / L::RG);
+  // No vector-memory write pending on entry or at the back edge (rows that no consumer reads, of
+  // the pairs attended before, included): the wait analysis otherwise orders each pair's loads
+  // behind the previous pair's. vmcnt(0), with expcnt and lgkmcnt left at their maximum.
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+  for (int j = js + wave; j < je; j += 4 * NW) {
+    int b[4];
+    bool ok[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int jj = j + u * NW;
+      if constexpr (IDS_LDS) {
+        b[u] = jj < je ? ((const __attribute__((address_space(3))) int32_t*)idx_h)[jj - sel_base] : -1;
+      } else {
+        b[u] = jj < je ? *gmem<int32_t>(idx_h + (jj - sel_base)) : -1;
+      }
+      ok[u] = b[u] >= 0 && (int64_t)b[u] < s.nblk;
+    }
+    RawI8<D> w[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) load_pair_raw<D, MT>(s, a.bs, ok[u], b[u], h, 0, nit, a.bs, r, c, w[u]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (ok[u]) finish_raw(0, r, w[u]);  // wave-uniform branches: every lane shuffles
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (ok[u]) consume_chunk<D, G>(q, WidenI8<D, MT>(w[u]), w[u], 0, nit, a.bs, r, st);
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+  }
+}
+
 // ---- Q.K and P.V on the matrix cores ---------------------------------------------------------------
 // The 8-wave instances with a model-dtype query score a 16-token chunk with one v_mfma_f32_16x16x32 per 32
 // channels: A = the chunk's 16 key rows (lane l: row l % 16, channels 32s + 8 (l / 16) .. + 7),
@@ -1299,14 +1343,21 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
       const int js = max(first, has_sink) - has_sink;
       const int je = min(last, has_sink + n_sel) - has_sink;
       // The hybrid branch is compiled only into the 4-wave general instance, which every hybrid
-      // launch takes. The 8-wave vector-path instances keep two selected pairs in flight per wave;
-      // float32 pools keep one (two would spill).
+      // launch takes. The 8-wave vector-path instances keep two selected pairs in flight per wave, and int8
+      // records of blocks of at most 16 tokens four (attend_selected_i8_four), in the same order.
+      // Float32 pools keep one (two would spill).
       // A fused-selection instance keeps the pairing of the instance it stands in for, so that both
       // fold each wave's chunks in the same order (with two pairs in flight a wave interleaves their
       // 16-row chunks).
       constexpr bool HYB = I8 && NT == kThreads && SEL == 0;
       constexpr int NPA = ((I8 && NT == kThreads) || MT == LKV_F32) ? 1 : 2;
       bool piped = false;  // the selected pairs were attended by a pipelined loop
+      if constexpr (I8 && NT == kThreadsHbm && NPA == 2) {
+        if (a.sel.dtype == LKV_INT8_RECORD && a.bs <= 16) {
+          attend_selected_i8_four<D, MT, G, NW, (SEL > 0)>(a, idx_h, sel_base, js, je, wave, h, q, r, c, st);
+          piped = true;
+        }
+      }
       if constexpr (HYB) {
         if (a.loc != nullptr && a.sel.dtype != LKV_INT8_RECORD && a.bs <= 16) {
           attend_hybrid_piped<D, MT, G, NW>(a, idx_h, sel_base, js, je, wave, h, q, r, c, st);
@@ -1643,21 +1694,26 @@ static void plan_matrix(Plan& p, const lkv_decode_desc* d, int cus) {
 
 // The kernel instance a launch takes. HBM plans (a.nt == kThreadsHbm) run 8-wave workgroups on the matrix cores
 // when the query has the model dtype and 16-byte aligned rows: one instance for 16-bit pairs, one that also
-// reads int8 records. Other queries (and float32 pools) take the 8-wave vector path for 16-bit and
-// float32 pairs of groups of up to 4 heads, and the 4-wave general instance over the same plan for the rest.
+// reads int8 records. Other queries (and float32 pools) take the 8-wave vector path for groups of up to 4 heads,
+// int8-capable when a source is int8 records (except D 128 with G 4, which spills there), and the 4-wave
+// general instance over the same plan for the rest (a float32 query over 1,024 int8 records a head, 8 heads of 4 at d 64:
+// 24.8 us a layer on the 8-wave vector path, 29.8 on the general one; 8 heads of 8, general: 51.5 over the 4-wave
+// plan, 39.2 over this one).
 // Host plans and hybrid launches take the 4-wave general instance (the link bounds them). Two layers in a replayed step,
 // 254 of 1,024 blocks of 16 tokens, general instance -> matrix cores: 8 heads of 8, bfloat16 d 128, 58.3 -> 39 us; int8 records,
 // 8 heads of 4 at d 128, 49.4 -> 39; the 8-wave vector path for records at d 64 took 36.1 where this takes 32.4. A fused-selection launch has
 // no 8-wave vector instance and takes the general one instead (lkv_select_decode then selects in its own
 // launch, so that it folds what the unfused call folds).
-enum class Inst { kGeneral, kVector8, kMatrix8, kMatrixRec8 };
+enum class Inst { kGeneral, kVector8, kInt8x8, kMatrix8, kMatrixRec8 };
 
-static Inst pick_instance(const DecodeArgs& a, int MT, int G, bool sel) {
+static Inst pick_instance(const DecodeArgs& a, int D, int MT, int G, bool sel) {
   const bool i8 = a.sel.dtype == LKV_INT8_RECORD || a.rem.dtype == LKV_INT8_RECORD || a.sink.dtype == LKV_INT8_RECORD ||
                   a.cur.dtype == LKV_INT8_RECORD || a.loc != nullptr;
   if (a.nt != kThreadsHbm || a.loc != nullptr) return Inst::kGeneral;
   if (MT != LKV_F32 && a.q_dtype == MT && ((uintptr_t)a.q & 15u) == 0) return i8 ? Inst::kMatrixRec8 : Inst::kMatrix8;
-  return i8 || sel || G > 4 ? Inst::kGeneral : Inst::kVector8;
+  if (G > 4 || (i8 && D == 128 && G == 4)) return Inst::kGeneral;
+  if (i8) return Inst::kInt8x8;
+  return sel ? Inst::kGeneral : Inst::kVector8;
 }
 
 // Threads per workgroup of an instance.
@@ -1683,6 +1739,12 @@ int launch_inst(hipStream_t stream, DecodeArgs& a, Inst inst) {
       done = true;
     }
   }
+  if constexpr (G <= 4 && !(D == 128 && G == 4)) {
+    if (inst == Inst::kInt8x8) {
+      hipLaunchKernelGGL((sparse_decode_kernel<D, MT, G, kThreadsHbm, true, false, SEL>), grid, dim3(kThreadsHbm), 0, stream, a);
+      done = true;
+    }
+  }
   if constexpr (SEL * kSelUnit <= kFuseKeysPerThread * kThreads) {  // more candidates never select in a 4-wave launch
     if (!done) hipLaunchKernelGGL((sparse_decode_kernel<D, MT, G, kThreads, true, false, SEL>), grid, dim3(kThreads), 0, stream, a);
     done = true;
@@ -1701,7 +1763,7 @@ template <int D, int MT, int G>
 int launch(hipStream_t stream, DecodeArgs& a) {
   const bool sel = a.bounds != nullptr;
   const int S = a.splits_a + a.splits_b;
-  const Inst inst = pick_instance(a, MT, G, sel);
+  const Inst inst = pick_instance(a, D, MT, G, sel);
   const int rc = !sel                          ? launch_inst<D, MT, G, 0>(stream, a, inst)
                  : a.n_cand <= kSelUnit     ? launch_inst<D, MT, G, 1>(stream, a, inst)
                  : a.n_cand <= 2 * kSelUnit ? launch_inst<D, MT, G, 2>(stream, a, inst)
@@ -2172,7 +2234,7 @@ static int sparse_decode_impl(uintptr_t stream, const lkv_decode_desc* desc, con
   a.rem = to_src(rem);
   a.loc = loc;
   a.nt = p.nt;
-  const Inst inst = pick_instance(a, mt, G, false);
+  const Inst inst = pick_instance(a, d.head_dim, mt, G, false);
   if (inst == Inst::kMatrix8 || inst == Inst::kMatrixRec8) plan_matrix(p, desc, device_cus());
   const int S = p.splits_a + p.splits_b;
   LKV_CHECK_ARG(S > 0, "nothing to attend");
@@ -2211,7 +2273,7 @@ static int sparse_decode_impl(uintptr_t stream, const lkv_decode_desc* desc, con
   // kFuseKeysPerThread of the head's candidates; otherwise the selection takes a launch of its own.
   bool select_in_decode = false;
   if (fsel != nullptr && fsel->in_decode) {
-    const Inst fused = pick_instance(a, mt, G, true);
+    const Inst fused = pick_instance(a, d.head_dim, mt, G, true);
     select_in_decode = fused == inst && fsel->n_cand <= kFuseKeysPerThread * inst_threads(fused);
   }
   if (fsel != nullptr) {
