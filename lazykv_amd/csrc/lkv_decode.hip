@@ -297,9 +297,11 @@ __device__ __forceinline__ void finish_raw(int t0, int r, RawI8<D>& raw) {
 template <int D, int MT>
 __device__ __forceinline__ void finish_raw(int, int, RawModel<D, MT>&) {}
 
-// 2^x for x <= 0 by the hardware's instruction alone. exp2f returns the same from 2^-126 up; below it, where exp2f spends
-// four more instructions on a subnormal result, this is 0: beside the weight 1 of the largest score.
-__device__ __forceinline__ float weight(float x) { return __builtin_amdgcn_exp2f(x); }
+// 2^x for x <= 0 by the hardware's instruction alone: exp2f's result from kNormalExp up, and 0 below it, where exp2f spends
+// four more instructions a weight on a subnormal one. A wave that meets a finite x below kNormalExp takes its weights from exp2f
+// (exp2f for every weight: 16 layers at 32K tokens 248.0 -> 252.7 us, int8 records at 64K 316.3 -> 321.8).
+__device__ __forceinline__ float normal_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+constexpr float kNormalExp = -126.0f;
 
 // Per-row widening of a raw chunk: key row i / value row i of this lane's channels, as float.
 template <int D, int MT>
@@ -734,7 +736,7 @@ __device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D /
   }
   float sc[NP][4];
   bool vld[NP][4];
-  float cm = -INFINITY;
+  float cm = -INFINITY, least = INFINITY;  // `least` over all rows: one past the limit has row 0's score, a skipped chunk's 0
 #pragma unroll
   for (int u = 0; u < NP; ++u)
 #pragma unroll
@@ -742,21 +744,30 @@ __device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D /
       sc[u][i] = acc[u][i] * qscale;
       vld[u][i] = 4 * lg + i < rows[u];
       cm = vld[u][i] ? fmaxf(cm, sc[u][i]) : cm;
+      least = fminf(least, sc[u][i]);
     }
   cm = lkv::pair_max<32>(lkv::pair_max<16>(cm));
   const float m_old = st.m;
   const float m_new = fmaxf(m_old, cm);
   const bool live = m_new != -INFINITY;  // false while nothing valid has been seen
-  const float alpha = m_old != -INFINITY ? weight(m_old - m_new) : 1.0f;  // nothing to rescale before the first valid chunk
+  const float alpha = m_old != -INFINITY ? exp2f(m_old - m_new) : 1.0f;  // nothing to rescale before the first valid chunk
   float p[NP][4];
+  if (__builtin_expect(__ballot(least - m_new < kNormalExp) == 0, 1)) {
+#pragma unroll
+    for (int u = 0; u < NP; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p[u][i] = (vld[u][i] && live) ? normal_exp2(sc[u][i] - m_new) : 0.0f;
+  } else {
+#pragma unroll
+    for (int u = 0; u < NP; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p[u][i] = (vld[u][i] && live) ? exp2f(sc[u][i] - m_new) : 0.0f;
+  }
   float ps = 0.0f;
 #pragma unroll
   for (int u = 0; u < NP; ++u)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      p[u][i] = (vld[u][i] && live) ? weight(sc[u][i] - m_new) : 0.0f;
-      ps += p[u][i];
-    }
+    for (int i = 0; i < 4; ++i) ps += p[u][i];
   ps = lkv::pair_sum<32>(lkv::pair_sum<16>(ps));
   st.m = m_new;
   st.l = st.l * alpha + ps;
@@ -1456,12 +1467,26 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
 #pragma unroll
     for (int w = 0; w < NW; ++w) M = fmaxf(M, s_m[w][j]);
     float O = 0.0f, Lsum = 0.0f;
-    if (M != -INFINITY) {
+    if (M != -INFINITY) {  // wave-uniform: a wave's 64 outputs are one head's
+      // A finite difference below kNormalExp anywhere: the largest of the bits moved up by 0x00800000, which takes -inf (a wave that
+      // attended nothing) to 0.
+      constexpr uint32_t kUp = 0x00800000u;
+      float wt[NW];
+      uint32_t deepest = 0u;
 #pragma unroll
       for (int w = 0; w < NW; ++w) {
-        const float wt = weight(s_m[w][j] - M);
-        O += s_o[w][j][dd] * wt;
-        Lsum += s_l[w][j] * wt;
+        const float x = s_m[w][j] - M;
+        wt[w] = normal_exp2(x);
+        deepest = max(deepest, __float_as_uint(x) + kUp);
+      }
+      if (__builtin_expect(__ballot(deepest > __float_as_uint(kNormalExp) + kUp) != 0, 0)) {
+#pragma unroll
+        for (int w = 0; w < NW; ++w) wt[w] = exp2f(s_m[w][j] - M);
+      }
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        O += s_o[w][j][dd] * wt[w];
+        Lsum += s_l[w][j] * wt[w];
       }
     }
     po[t] = O;
