@@ -31,7 +31,8 @@ def selects_in_decode(n_cand: int, host: bool, group: int, int8: bool = False, h
     model-dtype query (`model_query`: the pools' dtype, 16-byte aligned) take 512-thread workgroups
     on the matrix cores. Any other query over HBM takes 512 for int8 records under groups of at most 4
     (256 at head_dim 128 with a group of 4), 256 for larger groups, and for the rest an instance that
-    does not select: its own launch does. A host pool takes 256 threads."""
+    does not select: its own launch does. A host pool takes 256 threads. (A workgroup that would attend
+    more than 2,048 selected blocks, which takes more than 64 KV heads, selects in its own launch too.)"""
     threads = 256
     if not host:
         if model_query or (int8 and group <= 4 and not (head_dim == 128 and group == 4)):

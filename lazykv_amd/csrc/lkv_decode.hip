@@ -2294,12 +2294,14 @@ static int sparse_decode_impl(uintptr_t stream, const lkv_decode_desc* desc, con
   a.loc_stride = loc_stride;
   if (slots) a.slots = to_src(slots);
   // Inside the decode launch only where that launch takes the instance the unfused call takes, so
-  // that both fold the same items in the same order, and while each of its threads holds at most
-  // kFuseKeysPerThread of the head's candidates; otherwise the selection takes a launch of its own.
+  // that both fold the same items in the same order, while each of its threads holds at most
+  // kFuseKeysPerThread of the head's candidates, and while a workgroup's selected ids fit the LDS of the
+  // selection's bins (a plan of one workgroup per head, for more KV heads than half the CUs, may attend more);
+  // otherwise the selection takes a launch of its own.
   bool select_in_decode = false;
   if (fsel != nullptr && fsel->in_decode) {
     const Inst fused = pick_instance(a, d.head_dim, mt, G, true);
-    select_in_decode = fused == inst && fsel->n_cand <= kFuseKeysPerThread * inst_threads(fused);
+    select_in_decode = fused == inst && fsel->n_cand <= kFuseKeysPerThread * inst_threads(fused) && p.per_a <= lkv::kSelBins;
   }
   if (fsel != nullptr) {
     // A remainder excludes the selected ids, so they must exist before the decode launch: chosen by
@@ -2310,9 +2312,7 @@ static int sparse_decode_impl(uintptr_t stream, const lkv_decode_desc* desc, con
                   "a selection inside the residency launch takes at most %d candidates", kSelCap);
     LKV_CHECK_ARG(fsel->bounds != nullptr && fsel->n_cand > 0 && d.k <= fsel->n_cand, "selection of k=%d from %d candidates", d.k,
                   fsel->n_cand);
-    LKV_CHECK_ARG(!select_in_decode || (fsel->n_cand <= kSelCap && p.per_a <= lkv::kSelBins),
-                  "a selection inside the decode launch takes at most %d candidates and %d items per workgroup", kSelCap,
-                  lkv::kSelBins);
+    LKV_CHECK_ARG(!select_in_decode || fsel->n_cand <= kSelCap, "a selection inside the decode launch takes at most %d candidates", kSelCap);
     LKV_CHECK_ARG(select_in_decode || fsel->ids != nullptr, "no room for the selected ids");
   }
   if (select_in_decode) {

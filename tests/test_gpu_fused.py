@@ -288,3 +288,30 @@ def test_selection_inside_the_decode_launch_on_designed_bounds(kind: str, h: int
         assert np.array_equal(idx_f[j].cpu().numpy(), want), (kind, j)
     assert torch.equal(idx_f, idx_2)
     assert torch.equal(out_f, out_2) and torch.equal(lse_f, lse_2)
+
+
+@pytest.mark.parametrize(("h", "g", "k"), [(256, 8, 2048), (256, 8, 2049), (256, 2, 2600), (100, 8, 6000)])
+def test_a_workgroup_of_more_ids_than_the_selection_holds_selects_in_its_own_launch(h: int, g: int, k: int) -> None:
+    """With more KV heads than half the CUs one workgroup attends all of a head's selection: up to 2,048 ids fit the
+    in-launch selection. The one-call step takes any k all the same, and equals the two-call path."""
+    from dataclasses import replace
+
+    from lazykv_amd import kernels
+
+    bs, d = 4, 64
+    n = k + 150
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    pool = torch.randn((n, 1, 2, bs, d), generator=gen, device="cuda").to(torch.float16)
+    src = replace(kernels.pool_source(pool), head_stride=0)  # every head reads the same blocks
+    kmax = torch.randn((1, h, n, d), generator=gen, device="cuda").to(torch.float16)
+    q = torch.randn((h * g, d), generator=gen, device="cuda").to(torch.float16)
+    idx = torch.empty((h, k), dtype=torch.int32, device="cuda")
+    common = dict(block_size=bs, scale=d**-0.5, sel=src, out_dtype=torch.float32)
+    out, lse = kernels.select_decode(q, kmax, kmax, k, cand_offset=0, n_cand=n, out_idx=idx, **common)
+    idx2 = kernels.bound_topk(q, kmax, kmax, k)
+    out2, lse2 = kernels.sparse_decode(q, n_kv=h, idx=idx2, **common)
+    assert torch.equal(idx, idx2) and torch.equal(out, out2) and torch.equal(lse, lse2)
+    ids = idx[h - 1].long()
+    keys, values = (pool[ids, 0, i].reshape(-1, d).double() for i in (0, 1))
+    s = (q[(h - 1) * g :].double() @ keys.T.contiguous()) * d**-0.5
+    assert torch.allclose(out[(h - 1) * g :].double(), torch.softmax(s, 1) @ values, atol=TOL, rtol=0)
