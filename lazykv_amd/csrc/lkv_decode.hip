@@ -299,7 +299,7 @@ __device__ __forceinline__ void finish_raw(int, int, RawModel<D, MT>&) {}
 
 // 2^x for x <= 0 by the hardware's instruction alone: exp2f's result from kNormalExp up, and 0 below it, where exp2f spends
 // four more instructions a weight on a subnormal one. A wave that meets a finite x below kNormalExp takes its weights from exp2f
-// (exp2f for every weight: 16 layers at 32K tokens 248.0 -> 252.7 us, int8 records at 64K 316.3 -> 321.8).
+// (exp2f for every weight: 16 layers at 32K tokens 247.4 -> 251.8 us, int8 records at 64K 315.8 -> 319.7).
 __device__ __forceinline__ float normal_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 constexpr float kNormalExp = -126.0f;
 
