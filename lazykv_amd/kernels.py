@@ -590,23 +590,38 @@ def store_blocks(
 
 def copy_rows(copies: list[tuple[torch.Tensor, torch.Tensor]]) -> None:
     """`dst.copy_(src)` for each (dst, src) of `[h, rows, d]` views, up to 8 of them in one launch (lkv_copy_rows) on
-    the current stream. A copy the launch does not cover -- another shape, dtype or device, rows that are not contiguous,
-    a source that autograd follows -- is torch's."""
+    the current stream. A copy the launch does not cover -- another shape, dtype or device, rows that are not contiguous or
+    not of whole 2-byte words, tensors that autograd follows in either mode -- is torch's."""
     first = copies[0][0]
-    here = first.is_cuda and first.device.index == torch.cuda.current_device()
-    descs = []
+    here = first.is_cuda and first.device.index == torch.cuda.current_device() and 0 < first.shape[0] <= 65535
+    descs, written = [], []
     for dst, src in copies:
         ds, ss = dst.stride(), src.stride()
+        es = dst.element_size()
         if (not here or dst.shape != src.shape or src.dtype != dst.dtype or src.device != first.device or dst.device != first.device
-                or ds[-1] != 1 or ss[-1] != 1 or dst.shape[0] != first.shape[0] or src.requires_grad):
+                or ds[-1] != 1 or ss[-1] != 1 or dst.shape[0] != first.shape[0] or src.requires_grad or dst.requires_grad
+                or (es == 1 and (ds[0] | ds[1] | ss[0] | ss[1] | dst.shape[2] | dst.data_ptr() | src.data_ptr()) & 1)
+                or type(src) not in _PLAIN or type(dst) not in _PLAIN or src.is_neg() or dst.is_neg() or _dual(src) or _dual(dst)):
             dst.copy_(src)
             continue
-        es = dst.element_size()
         _, rows, d = dst.shape
         descs.append(_lib.RowCopy(src.data_ptr(), dst.data_ptr(), ss[0] * es, ss[1] * es, ds[0] * es, ds[1] * es, rows, d * es))
-    if descs:
-        arr = (_lib.RowCopy * len(descs))(*descs)
-        _lib.check(_lib.lib().lkv_copy_rows(_lib.stream_of(first), arr, len(descs), first.shape[0]), "copy_rows")
+        written.append(dst)
+    if not descs:
+        return
+    torch.autograd.graph.increment_version(written)  # a graph that saved one of them sees the write, as after copy_
+    for i in range(0, len(descs), MAX_ROW_COPIES):
+        part = descs[i : i + MAX_ROW_COPIES]
+        _lib.check(_lib.lib().lkv_copy_rows(_lib.stream_of(first), (_lib.RowCopy * len(part))(*part), len(part), first.shape[0]), "copy_rows")
+
+
+MAX_ROW_COPIES = 8  # LKV_MAX_ROW_COPIES
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _dual(t: torch.Tensor) -> bool:
+    """Whether `t` carries a tangent of forward-mode differentiation."""
+    return torch.autograd.forward_ad.unpack_dual(t).tangent is not None
 
 
 def packed_pair_bytes(block_size: int, head_dim: int) -> int:
