@@ -985,12 +985,12 @@ __device__ __forceinline__ void attend_run_mf(const DecodeArgs& a, const MfRun& 
   }
 }
 
-// Remainder blocks b, b + NW, .. < hi whose bit (b - lo) of `excl` is clear, several per step, folded into the
-// softmax together.
-template <int D, int MT, int G, typename Raw, int NW>
-__device__ __forceinline__ void attend_rest_mf(const DecodeArgs& a, const uint32_t* excl, int lo, int b, int hi, int h,
-                                               const typename Mfma<MT>::V8 (&qb)[D / 32], int lane, int r, int c, float* sp, MfState<G>& st) {
-  constexpr int NP = kMfPairs<D, G, std::is_same<Raw, RecMf<D>>::value>;
+// Items j, j + NW, .. < count of a remainder run, the chunks of the blocks from `lo` whose bit (block - lo) of `excl` is
+// clear, up to NP per step, folded into the softmax together.
+template <int D, int MT, int G, typename Raw, int NP, int NW>
+__device__ __forceinline__ void attend_rest_slots(const DecodeArgs& a, const uint32_t* excl, int lo, int j, int count, int h,
+                                                  const typename Mfma<MT>::V8 (&qb)[D / 32], int lane, int r, int c, float* sp,
+                                                  MfState<G>& st) {
   Src s[NP];
   int lim[NP];
 #pragma unroll
@@ -998,16 +998,41 @@ __device__ __forceinline__ void attend_rest_mf(const DecodeArgs& a, const uint32
     s[u] = a.rem;
     lim[u] = a.bs;
   }
-  while (b < hi) {
-    int pick[NP];
+  const int nch = chunks_of(a);
+  while (j < count) {
+    int blk[NP], t0[NP];
 #pragma unroll
-    for (int u = 0; u < NP; ++u) pick[u] = -1;
+    for (int u = 0; u < NP; ++u) blk[u] = -1, t0[u] = 0;
     int have = 0;
-    while (have < NP && b < hi) {
-      if (!((excl[(b - lo) >> 5] >> ((b - lo) & 31)) & 1u)) pick[have++] = b;
-      b += NW;
+    while (have < NP && j < count) {
+      int b, t;
+      chunk_of(j, nch, b, t);
+      if (!((__builtin_amdgcn_readfirstlane(excl[b >> 5]) >> (b & 31)) & 1u)) {
+        blk[have] = lo + b;
+        t0[have++] = t;
+      }
+      j += NW;
     }
-    if (have) process_items_mf<D, MT, G, Raw, NP>(a, s, pick, lim, h, qb, lane, r, c, sp, st);
+    if (have) process_chunks_mf<D, MT, G, Raw, NP>(a, s, blk, lim, t0, h, qb, lane, r, c, sp, st);
+  }
+}
+
+// The remainder blocks lo .. hi - 1: chunks as items, and no more slots than a wave has items, as in segment A (a wave with
+// one block of records in four slots loaded it four times over: 125 blocks of 16 tokens a head, 8 heads of 1 at d 64,
+// 9.6 -> 7.6 us a launch; whole blocks as items, 16 of 256 tokens, 41.7 -> 20.9).
+template <int D, int MT, int G, typename Raw, int NW>
+__device__ __forceinline__ void attend_rest_mf(const DecodeArgs& a, const uint32_t* excl, int lo, int hi, int wave, int h,
+                                               const typename Mfma<MT>::V8 (&qb)[D / 32], int lane, int r, int c, float* sp, MfState<G>& st) {
+  constexpr int kMost = kMfPairs<D, G, std::is_same<Raw, RecMf<D>>::value>;
+  const int j = __builtin_amdgcn_readfirstlane(wave);
+  const int count = (hi - lo) * chunks_of(a);
+  const int slots = slots_for(count, NW, kMost);
+  if (slots == 1) {
+    attend_rest_slots<D, MT, G, Raw, 1, NW>(a, excl, lo, j, count, h, qb, lane, r, c, sp, st);
+  } else if (slots == 2 || kMost == 2) {
+    attend_rest_slots<D, MT, G, Raw, 2, NW>(a, excl, lo, j, count, h, qb, lane, r, c, sp, st);
+  } else {
+    attend_rest_slots<D, MT, G, Raw, kMost, NW>(a, excl, lo, j, count, h, qb, lane, r, c, sp, st);
   }
 }
 
@@ -1413,16 +1438,16 @@ __global__ __launch_bounds__(NT) void sparse_decode_kernel(DecodeArgs a) {
         if (bv[u] >= lo && bv[u] < hi) atomicOr(&s_excl[(bv[u] - lo) >> 5], 1u << ((bv[u] - lo) & 31));
     }
     __syncthreads();
-    int b = lo + wave;
     if constexpr (MF && I8) {
       if (a.rem.dtype == LKV_INT8_RECORD) {
-        attend_rest_mf<D, MT, G, RecMf<D>, NW>(a, s_excl, lo, b, hi, h, qb, lane, r, c, sp, st);
+        attend_rest_mf<D, MT, G, RecMf<D>, NW>(a, s_excl, lo, hi, wave, h, qb, lane, r, c, sp, st);
       } else {
-        attend_rest_mf<D, MT, G, RawMf<D, MT>, NW>(a, s_excl, lo, b, hi, h, qb, lane, r, c, sp, st);
+        attend_rest_mf<D, MT, G, RawMf<D, MT>, NW>(a, s_excl, lo, hi, wave, h, qb, lane, r, c, sp, st);
       }
     } else if constexpr (MF) {
-      attend_rest_mf<D, MT, G, RawMf<D, MT>, NW>(a, s_excl, lo, b, hi, h, qb, lane, r, c, sp, st);
+      attend_rest_mf<D, MT, G, RawMf<D, MT>, NW>(a, s_excl, lo, hi, wave, h, qb, lane, r, c, sp, st);
     } else {
+      int b = lo + wave;
       while (b < hi) {
         int pick[2] = {-1, -1};
         int have = 0;
