@@ -800,6 +800,8 @@ __device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D /
 #pragma unroll
     for (int i = 0; i < L::NI; ++i) {
       const int row = r + L::RG * i;
+      // Nothing of the chunk left (4-token blocks, every one a remainder's: 8 heads of 4 at d 128, 38.1 -> 29.6 us, records 54.6 -> 41.6).
+      if (part && L::RG * i >= rows[u]) break;
       float x[8];
       value_row<D, MT>(raw[u], i, x);
       if (part) {

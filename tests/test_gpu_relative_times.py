@@ -56,3 +56,24 @@ def test_a_model_query_attends_a_remainder_of_records_no_slower_than_a_float32_o
         times.append(_us(lambda: kernels.sparse_decode(qq, n_kv=h, block_size=bs, scale=d**-0.5, sel=src, idx=idx, rem=src, rem_range=(0, n), out=out, lse=lse, ws=ws)))
     print(f"remainder of records h={h} g={g} bs={bs}: model query {times[0]:.1f} us, float32 {times[1]:.1f}", flush=True)
     assert times[0] < 1.25 * times[1]
+
+
+@pytest.mark.parametrize(("records", "bar"), [(False, 0.61), (True, 0.475)])
+def test_small_blocks_pay_for_their_own_rows(records: bool, bar: float) -> None:
+    """Blocks of 4 tokens fill a quarter of the matrix cores' 16-row chunks: the value rows that a block does not have cost nothing.
+    Against a float32 query on the vector path, which skips them too: 38.1 us against 55.6 (pairs) and 54.6 against 100.9 (records)
+    with the rows masked; now 29.6 and 41.6."""
+    from lazykv_amd import kernels
+
+    h, g, d, bs, n, k, dt = 8, 4, 128, 4, 4096, 600, torch.bfloat16
+    pool = torch.randn((n, h, 2, bs, d), device="cuda").to(dt)
+    src = _records(h, n, bs, d, dt) if records else kernels.pool_source(pool)
+    idx = torch.stack([torch.randperm(n - 1, device="cuda")[:k].sort().values + 1 for _ in range(h)]).to(torch.int32)
+    q = torch.randn((h * g, d), device="cuda")
+    lse = torch.empty(h * g, device="cuda")
+    times = []
+    for qq in (q.to(dt), q):
+        out, ws = torch.empty_like(qq), kernels.Workspace()
+        times.append(_us(lambda: kernels.sparse_decode(qq, n_kv=h, block_size=bs, scale=d**-0.5, sel=src, idx=idx, rem=src, rem_range=(0, n), out=out, lse=lse, ws=ws)))
+    print(f"4-token blocks, records={records}: model query {times[0]:.1f} us, float32 {times[1]:.1f}", flush=True)
+    assert times[0] < bar * times[1]
