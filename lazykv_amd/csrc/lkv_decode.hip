@@ -575,10 +575,13 @@ struct Mfma<LKV_F16> {
 // times zero: their weights are finite and reach only accumulators that are never read.
 template <int G>
 constexpr int kHeadQuads = (G + 3) / 4;
+// Heads a row of the broadcast area holds: whole quads for the matrix cores, one for the vector ALUs.
+template <int G>
+constexpr int kHeadRow = G == 1 ? 1 : 4 * kHeadQuads<G>;
 // Floats of a wave's LDS broadcast area for up to NP pairs per step: p[NP][16][heads], then the heads'
 // rescale factors.
 template <int G, int NP>
-constexpr int kMfBroadcast = (16 * NP + 1) * 4 * kHeadQuads<G>;
+constexpr int kMfBroadcast = (16 * NP + 1) * kHeadRow<G>;
 // Pairs of one step, all their loads in flight together, by what the registers hold (the accumulators of 8 heads
 // are 64 registers; a d 128 pair 32 as 16-bit rows, 56 as an int8 record).
 template <int D, int G, bool REC>
@@ -723,7 +726,7 @@ __device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D /
                                            const int (&rows)[NP], int lane, int r, float* sp, MfState<G>& st) {
   using L = Lanes<D>;
   static_assert(L::EPL == 8, "8 channels a lane");
-  constexpr int GQ = kHeadQuads<G>, GW = 4 * GQ;
+  constexpr int GQ = kHeadQuads<G>, GW = kHeadRow<G>;
   const int j = lane % 16, lg = lane / 16;
   f32x4 acc[NP];
 #pragma unroll
@@ -784,13 +787,19 @@ __device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D /
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   if (rescale) {
+    if constexpr (G == 1) {
+      const float al = sp[16 * NP * GW];
 #pragma unroll
-    for (int g = 0; g < GQ; ++g) {
-      const f32x4 al = *(const f32x4*)(sp + 16 * NP * GW + 4 * g);
+      for (int e = 0; e < 8; ++e) st.o[0][e][0] *= al;
+    } else {
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
+      for (int g = 0; g < GQ; ++g) {
+        const f32x4 al = *(const f32x4*)(sp + 16 * NP * GW + 4 * g);
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj) st.o[g][e][jj] *= al[jj];
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj) st.o[g][e][jj] *= al[jj];
+      }
     }
   }
 #pragma unroll
