@@ -1753,6 +1753,18 @@ static void plan_matrix(Plan& p, const lkv_decode_desc* d, int cus) {
   p.splits_a = p.n_a > 0 ? (n_sel > 0 ? (n_sel + p.per_a - 1) / p.per_a : 1) : 0;
 }
 
+// Compute units of the current device, cached per device.
+static int device_cus() {
+  static int cached[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (cached[dev] == 0) {
+    int v = 0;
+    cached[dev] = (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) ? v : 256;
+  }
+  return cached[dev];
+}
+
 // The kernel instance a launch takes. HBM plans (a.nt == kThreadsHbm) run 8-wave workgroups on the matrix cores
 // when the query has the model dtype and 16-byte aligned rows: one instance for 16-bit pairs, one that also
 // reads int8 records. Other queries (and float32 pools) take the 8-wave vector path for groups of up to 4 heads,
@@ -1767,11 +1779,24 @@ static void plan_matrix(Plan& p, const lkv_decode_desc* d, int cus) {
 // launch, so that it folds what the unfused call folds).
 enum class Inst { kGeneral, kVector8, kInt8x8, kMatrix8, kMatrixRec8 };
 
+// Records under one query head a KV head: the matrix cores use one of their 16 columns, and widening the key codes for them
+// costs more than the vector path's products, so a selection without a remainder takes the vector path where that has a wave for
+// each block anyway: blocks of one chunk (at d 128 whole ones), or blocks that fill the waves. Decodes of given ids, matrix cores
+// -> here, 8 and 32 heads: 200 of 16 tokens at d 64 7.7 -> 6.9 and 11.9 -> 10.1 us, at d 128 9.8 -> 9.1 and 17.5 -> 17.3; 600 of 4 tokens at
+// d 64 9.5 -> 7.8 and 18.8 -> 15.3 (d 128 10.3 -> 11.2 and 24.4 -> 27.2, so not there); 60 of 64 tokens, 32 heads, 15.3 -> 13.3 (8 heads 9.6
+// and 10.7, so not there). With a remainder the matrix cores take no longer at 16 tokens and less elsewhere.
+static bool records_by_vector(const DecodeArgs& a, int D, int G) {
+  if (G != 1 || a.sel.dtype != LKV_INT8_RECORD || a.rem_first != a.rem_last) return false;
+  if (a.bs <= 16) return D == 64 || a.bs == 16;
+  return 2 * (int64_t)a.k * a.n_kv >= (int64_t)(kThreadsHbm / 64) * device_cus();
+}
+
 static Inst pick_instance(const DecodeArgs& a, int D, int MT, int G, bool sel) {
   const bool i8 = a.sel.dtype == LKV_INT8_RECORD || a.rem.dtype == LKV_INT8_RECORD || a.sink.dtype == LKV_INT8_RECORD ||
                   a.cur.dtype == LKV_INT8_RECORD || a.loc != nullptr;
   if (a.nt != kThreadsHbm || a.loc != nullptr) return Inst::kGeneral;
-  if (MT != LKV_F32 && a.q_dtype == MT && ((uintptr_t)a.q & 15u) == 0) return i8 ? Inst::kMatrixRec8 : Inst::kMatrix8;
+  const bool model_query = MT != LKV_F32 && a.q_dtype == MT && ((uintptr_t)a.q & 15u) == 0;
+  if (model_query && !records_by_vector(a, D, G)) return i8 ? Inst::kMatrixRec8 : Inst::kMatrix8;
   if (G > 4 || (i8 && D == 128 && G == 4)) return Inst::kGeneral;
   if (i8) return Inst::kInt8x8;
   return sel ? Inst::kGeneral : Inst::kVector8;
@@ -2147,18 +2172,6 @@ __global__ __launch_bounds__(kResThreads) void residency_kernel(const int32_t* _
   }
 }
 
-// Compute units of the current device, cached per device.
-static int device_cus() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cached[dev] == 0) {
-    int v = 0;
-    cached[dev] = (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) ? v : 256;
-  }
-  return cached[dev];
-}
-
 static Src to_src(const lkv_kv_source* s) {
   Src o{};
   if (s) {
@@ -2295,6 +2308,11 @@ static int sparse_decode_impl(uintptr_t stream, const lkv_decode_desc* desc, con
   a.rem = to_src(rem);
   a.loc = loc;
   a.nt = p.nt;
+  a.n_kv = d.n_kv;
+  a.bs = d.block_size;
+  a.k = d.k;
+  a.rem_first = d.rem_first;
+  a.rem_last = d.rem_last;
   const Inst inst = pick_instance(a, d.head_dim, mt, G, false);
   if (inst == Inst::kMatrix8 || inst == Inst::kMatrixRec8) plan_matrix(p, desc, device_cus());
   const int S = p.splits_a + p.splits_b;
@@ -2305,15 +2323,10 @@ static int sparse_decode_impl(uintptr_t stream, const lkv_decode_desc* desc, con
 
   a.idx = idx;
   a.idx_stride = idx_stride;
-  a.n_kv = d.n_kv;
-  a.bs = d.block_size;
-  a.k = d.k;
   a.attend_selected = attend_sel ? 1 : 0;
   a.sink_block = d.sink_block;
   a.cur_block = d.cur_block;
   a.fill = d.fill;
-  a.rem_first = d.rem_first;
-  a.rem_last = d.rem_last;
   a.qscale = d.scale * lkv::kLog2e;
   a.n_a = p.n_a;
   a.per_a = p.per_a;
