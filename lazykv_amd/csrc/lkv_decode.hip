@@ -806,6 +806,13 @@ __device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D /
   for (int u = 0; u < NP; ++u) {
     if (rows[u] <= 0) continue;                // wave-uniform, as the next test
     const bool part = rows[u] < 16;           // rows past the limit may hold non-finite data
+    // The weights of all the lane's rows, read before the branches below: one wait for LDS a chunk instead of one a row (every block a
+    // remainder's, 32 heads of 1 at d 64, 1,024 blocks of 16 tokens 29.1 -> 28.7 us; 16 layers at 32K tokens 247.9 -> 245.6).
+    float pr[L::NI][GQ];
+#pragma unroll
+    for (int i = 0; i < L::NI; ++i)
+#pragma unroll
+      for (int g = 0; g < GQ; ++g) pr[i][g] = sp[(16 * u + r + L::RG * i) * GW + (G == 1 ? 0 : 4 * g + (lane & 3))];
 #pragma unroll
     for (int i = 0; i < L::NI; ++i) {
       const int row = r + L::RG * i;
@@ -820,15 +827,13 @@ __device__ __forceinline__ void consume_mf(const typename Mfma<MT>::V8 (&qb)[D /
         for (int e = 0; e < 8; ++e) x[e] = ok ? x[e] : 0.0f;  // their weights are 0
       }
       if constexpr (G == 1) {  // one row of four: the vector ALUs are as fast
-        const float pr = sp[(16 * u + row) * GW];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) st.o[0][e][0] = fmaf(pr, x[e], st.o[0][e][0]);
+        for (int e = 0; e < 8; ++e) st.o[0][e][0] = fmaf(pr[i][0], x[e], st.o[0][e][0]);
       } else {
 #pragma unroll
         for (int g = 0; g < GQ; ++g) {
-          const float pr = sp[(16 * u + row) * GW + 4 * g + (lane & 3)];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) st.o[g][e] = __builtin_amdgcn_mfma_f32_4x4x1f32(pr, x[e], st.o[g][e], 0, 0, 0);
+          for (int e = 0; e < 8; ++e) st.o[g][e] = __builtin_amdgcn_mfma_f32_4x4x1f32(pr[i][g], x[e], st.o[g][e], 0, 0, 0);
         }
       }
     }
