@@ -4,7 +4,7 @@
 // Reference: lazykv/quant.py:59-105 (_affine, pack, unpack), lazykv/tiered.py:162-197 (the
 // boundary: host copy or pack, then metadata from the exact or the dequantised keys),
 // :353-375 (_seal: one block, blocking D2H, pack + unpack for the int8 metadata), :226-236
-// (metadata rebuilt from a stored pool). One wave handles one (block, KV head) pair; 16 lanes
+// (metadata rebuilt from a stored pool). One wave handles one (block, KV head) pair, or two of 4 tokens at head_dim 64; 16 lanes
 // hold one row, so the 4 row groups of the wave see rows r, r+4, r+8, ... of the block.
 //
 // Bit-exactness. quant.py computes in float32: mn/mx (exact), scale = max((mx-mn)/255, FLT_MIN)
@@ -172,19 +172,19 @@ template <int D, int MT>
 struct Rows {
   static constexpr int LPR = D / 8;       // lanes per row
   static constexpr int RG = 64 / LPR;     // rows per wave-wide load
-  static constexpr int NI = 16 / RG;      // loads per 16-row chunk
   static constexpr int W = 2 * (int)sizeof(typename lkv::Elem<MT>::T);  // words of a lane's 8 channels
 };
 
-template <int D, int MT>
+// A chunk of 16 rows, or, for blocks of fewer, of NI loads' RG * NI rows.
+template <int D, int MT, int NI>
 struct RowChunk {
-  uint32_t w[Rows<D, MT>::NI][Rows<D, MT>::W];
+  uint32_t w[NI][Rows<D, MT>::W];
   // Rows t0 + r + RG i of the pair at p (this lane's channels); a row past the block reads row 0 instead, which
   // changes no range, and is not stored.
   __device__ __forceinline__ void load(const typename lkv::Elem<MT>::T* p, int t0, int bs, int r) {
     using R = Rows<D, MT>;
 #pragma unroll
-    for (int i = 0; i < R::NI; ++i) {
+    for (int i = 0; i < NI; ++i) {
       const int row = t0 + r + R::RG * i;
       const uint32_t* at = (const uint32_t*)(p + (int64_t)(row < bs ? row : 0) * D);
 #pragma unroll
@@ -200,7 +200,7 @@ struct RowChunk {
   __device__ __forceinline__ void store(typename lkv::Elem<MT>::T* p, int t0, int bs, int r) const {
     using R = Rows<D, MT>;
 #pragma unroll
-    for (int i = 0; i < R::NI; ++i) {
+    for (int i = 0; i < NI; ++i) {
       const int row = t0 + r + R::RG * i;
       if (row < bs) {
         uint32_t* at = (uint32_t*)(p + (int64_t)row * D);
@@ -221,12 +221,12 @@ struct RowChunk {
   }
 };
 
-// A lane's 8 channels reduced over the wave's RG row groups: each step keeps one half of the values and gives the
-// partner the other, so lane l ends with the totals of its channels own_channel(l) .. + 8 / RG - 1 in v.
-template <int RG, typename Op>
+// A lane's 8 channels reduced over the GROUPS row groups of its pair (LPR lanes each): each step keeps one half of the values and
+// gives the partner the other, so a lane ends with the totals of its channels own_channel() .. + 8 / GROUPS - 1 in v.
+template <int LPR, int GROUPS, typename Op>
 __device__ __forceinline__ void reduce_channels(float (&v)[8], int lane, Op op) {
-  constexpr int N = RG == 8 ? 4 : 8;  // values a lane holds after the 8-lane rows' own step
-  if constexpr (RG == 8) {
+  constexpr int N = LPR == 8 ? 4 : 8;  // values a lane holds after the 8-lane rows' own step
+  if constexpr (LPR == 8) {
     const bool odd = (lane & 8) != 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -240,26 +240,30 @@ __device__ __forceinline__ void reduce_channels(float (&v)[8], int lane, Op op) 
     lkv::swap_halves<16>(v[i], v[i + N / 2], x, y);
     v[i] = op(x, y);
   }
+  if constexpr (LPR * GROUPS == 64) {
 #pragma unroll
-  for (int i = 0; i < N / 4; ++i) {
-    lkv::swap_halves<32>(v[i], v[i + N / 4], x, y);
-    v[i] = op(x, y);
+    for (int i = 0; i < N / 4; ++i) {
+      lkv::swap_halves<32>(v[i], v[i + N / 4], x, y);
+      v[i] = op(x, y);
+    }
   }
 }
-template <int RG>
+template <int LPR, int GROUPS>
 __device__ __forceinline__ int own_channel(int lane) {
-  constexpr int N = RG == 8 ? 4 : 8;
-  return (RG == 8 && (lane & 8) ? 4 : 0) + ((lane & 16) ? N / 2 : 0) + ((lane & 32) ? N / 4 : 0);
+  constexpr int N = LPR == 8 ? 4 : 8;
+  return (LPR == 8 && (lane & 8) ? 4 : 0) + ((lane & 16) ? N / 2 : 0) + (LPR * GROUPS == 64 && (lane & 32) ? N / 4 : 0);
 }
 // The reverse: every lane's 8 channels from the lanes that own them.
-template <int RG>
+template <int LPR, int GROUPS>
 __device__ __forceinline__ void gather_channels(float (&v)[8], int lane) {
-  constexpr int N = RG == 8 ? 4 : 8;
+  constexpr int N = LPR == 8 ? 4 : 8;
+  if constexpr (LPR * GROUPS == 64) {
 #pragma unroll
-  for (int i = 0; i < N / 4; ++i) lkv::lane_pair<32>(v[i], v[i], v[i + N / 4]);
+    for (int i = 0; i < N / 4; ++i) lkv::lane_pair<32>(v[i], v[i], v[i + N / 4]);
+  }
 #pragma unroll
   for (int i = 0; i < N / 2; ++i) lkv::lane_pair<16>(v[i], v[i], v[i + N / 2]);
-  if constexpr (RG == 8) {
+  if constexpr (LPR == 8) {
     const bool odd = (lane & 8) != 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -306,22 +310,25 @@ __device__ __forceinline__ uint2 quantise8(const float (&x)[8], const float (&mn
 }
 
 // The block's key metadata from the lanes that own its channels.
-template <int D, int RG>
+template <int D, int LPR, int GROUPS>
 __device__ __forceinline__ void write_owned(const StoreArgs& a, int b, int h, int c, int lane, const float (&mn)[8], const float (&mx)[8]) {
-  const int64_t base = (int64_t)h * a.meta_hstride + (int64_t)b * D + c * 8 + own_channel<RG>(lane);
+  const int64_t base = (int64_t)h * a.meta_hstride + (int64_t)b * D + c * 8 + own_channel<LPR, GROUPS>(lane);
 #pragma unroll
-  for (int i = 0; i < 8 / RG; ++i) {
+  for (int i = 0; i < 8 / GROUPS; ++i) {
     lkv::store_any(a.kmin, base + i, a.meta_dtype, mn[i]);
     lkv::store_any(a.kmax, base + i, a.meta_dtype, mx[i]);
   }
 }
 
-template <int D, int MT, int MODE, bool META>
+// PPW: pairs of the wave, each in 64 / PPW lanes (two where one load of the wave has the rows of two blocks).
+template <int D, int MT, int MODE, bool META, int NI, int PPW>
 __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
   using T = typename lkv::Elem<MT>::T;
   using R = Rows<D, MT>;
   const int lane = threadIdx.x & 63;
-  const int r = lane / R::LPR, c = lane % R::LPR;
+  static_assert(PPW == 1 || (PPW == 2 && NI == 1 && R::RG == 8), "two pairs of at most 4 rows each");
+  constexpr int GROUPS = R::RG / PPW;  // row groups of a pair
+  const int r = lane / R::LPR % GROUPS, c = lane % R::LPR;
   // A workgroup's four waves take four consecutive blocks of one head, contiguous in a dense cache: a pair per
   // head in turn, they read and wrote at the heads' strides, a power of two apart, at once (a float16 layer of
   // 32K tokens into a pool, dense [h, T, 64] source: 30.2 -> 23.4 us; pool to pool 47.6 -> 46.2).
@@ -342,7 +349,7 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
   const int64_t soff = (int64_t)b * a.s_bstride + (int64_t)h * a.s_hstride + c * 8;
   const T* sk = (const T*)a.sk + soff;
   const T* sv = (const T*)a.sv + soff;
-  RowChunk<D, MT> k, v;
+  RowChunk<D, MT, NI> k, v;
   k.load(sk, 0, bs, r);
   if constexpr (MODE != MODE_META) v.load(sv, 0, bs, r);
 
@@ -363,7 +370,7 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
   for (int t0 = 0;;) {
     if constexpr (kRange) {
 #pragma unroll
-      for (int i = 0; i < R::NI; ++i) {
+      for (int i = 0; i < NI; ++i) {
         float x[8];
         k.widen(i, x);
 #pragma unroll
@@ -383,24 +390,24 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
     if constexpr (MODE == MODE_COPY) v.load(sv, t0, bs, r);
   }
   if constexpr (kRange) {
-    reduce_channels<R::RG>(mn, lane, lower);
-    reduce_channels<R::RG>(mx, lane, upper);
+    reduce_channels<R::LPR, GROUPS>(mn, lane, lower);
+    reduce_channels<R::LPR, GROUPS>(mx, lane, upper);
   }
   if constexpr (MODE != MODE_INT8) {
-    if constexpr (META) write_owned<D, R::RG>(a, b, h, c, lane, mn, mx);
+    if constexpr (META) write_owned<D, R::LPR, GROUPS>(a, b, h, c, lane, mn, mx);
   } else {
     uint8_t* rec = (uint8_t*)a.dk + (int64_t)b * a.d_bstride + (int64_t)h * a.d_hstride;
     uint16_t* sc = (uint16_t*)(rec + 2 * bs * D);
     // Each channel's scale is made, and stored, by the lane that owns it.
     float scale[8], inv[8];
 #pragma unroll
-    for (int i = 0; i < 8 / R::RG; ++i) {
+    for (int i = 0; i < 8 / GROUPS; ++i) {
       scale[i] = scale_of(mn[i], mx[i]);
-      sc[c * 8 + own_channel<R::RG>(lane) + i] = lkv::f32_to_f16(scale[i]);
-      sc[D + c * 8 + own_channel<R::RG>(lane) + i] = lkv::f32_to_f16(mn[i]);
+      sc[c * 8 + own_channel<R::LPR, GROUPS>(lane) + i] = lkv::f32_to_f16(scale[i]);
+      sc[D + c * 8 + own_channel<R::LPR, GROUPS>(lane) + i] = lkv::f32_to_f16(mn[i]);
     }
-    gather_channels<R::RG>(scale, lane);
-    gather_channels<R::RG>(mn, lane);
+    gather_channels<R::LPR, GROUPS>(scale, lane);
+    gather_channels<R::LPR, GROUPS>(mn, lane);
 #pragma unroll
     for (int e = 0; e < 8; ++e) inv[e] = __builtin_amdgcn_rcpf(scale[e]);
     float dmn[8], dmx[8];
@@ -415,7 +422,7 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
         v.load(sv, t0, bs, r);
       }
 #pragma unroll
-      for (int i = 0; i < R::NI; ++i) {
+      for (int i = 0; i < NI; ++i) {
         const int row = t0 + r + R::RG * i;
         float x[8];
         k.widen(i, x);
@@ -434,7 +441,7 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
       }
       // ---- values: per-token range over head_dim -------------------------------------------------------
 #pragma unroll
-      for (int i = 0; i < R::NI; ++i) {
+      for (int i = 0; i < NI; ++i) {
         const int row = t0 + r + R::RG * i;
         float x[8];
         v.widen(i, x);
@@ -465,53 +472,61 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
       }
     }
     if constexpr (META) {
-      reduce_channels<R::RG>(dmn, lane, lower);
-      reduce_channels<R::RG>(dmx, lane, upper);
-      write_owned<D, R::RG>(a, b, h, c, lane, dmn, dmx);
+      reduce_channels<R::LPR, GROUPS>(dmn, lane, lower);
+      reduce_channels<R::LPR, GROUPS>(dmx, lane, upper);
+      write_owned<D, R::LPR, GROUPS>(a, b, h, c, lane, dmn, dmx);
     }
   }
 }
 
-// One wave per (block, head) pair, the grid striding over the pairs. Waves never synchronise with
+// A wave takes PPW (block, head) pairs at a time, the grid striding over the pairs. Waves never synchronise with
 // each other, so a grid smaller than the pair count (a host destination) is just a longer loop.
-template <int D, int MT, int MODE, bool META>
+template <int D, int MT, int MODE, bool META, int NI, int PPW>
 __global__ __launch_bounds__(kThreads) void store_blocks_kernel(StoreArgs a) {
   const int64_t total = (int64_t)a.n_blocks * a.n_kv;
-  for (int64_t pair = (int64_t)blockIdx.x * kWaves + (threadIdx.x >> 6); pair < total; pair += (int64_t)gridDim.x * kWaves)
+  constexpr int kLanes = 64 / PPW;
+  for (int64_t pair = (int64_t)blockIdx.x * kWaves * PPW + threadIdx.x / kLanes; pair < total; pair += (int64_t)gridDim.x * kWaves * PPW)
     if constexpr (MODE == MODE_META_FROM_I8 || MODE == MODE_UNPACK) {
       store_record<D, MT, MODE>(a, pair);  // `pair` is wave-uniform
     } else {
-      store_rows<D, MT, MODE, META>(a, pair);
+      store_rows<D, MT, MODE, META, NI, PPW>(a, pair);  // uniform over kLanes lanes, which exchange with no others
     }
+}
+
+template <int D, int MT, int MODE, bool META, int NI, int PPW>
+void launch_one(hipStream_t s, const StoreArgs& a, int64_t max_wgs) {
+  const int64_t pairs = (int64_t)a.n_blocks * a.n_kv;
+  int64_t wgs = (pairs + kWaves * PPW - 1) / (kWaves * PPW);
+  if (wgs > max_wgs) wgs = max_wgs;
+  hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE, META, NI, PPW>), dim3((unsigned)wgs), dim3(kThreads), 0, s, a);
+}
+
+// The instance for blocks of a.bs tokens: as many loads of RG rows as they fill, up to a 16-row chunk's, and two 4-token blocks in a
+// load of 8 rows. (A whole chunk's loads for all: 65,536 pairs of 4 x 64 float16 packed with their metadata in 98 us, of 4 x 128 in 157;
+// here in 45 and 85.)
+template <int D, int MT, int MODE, bool META>
+void launch_rows(hipStream_t s, const StoreArgs& a, int64_t max_wgs) {
+  constexpr int RG = Rows<D, MT>::RG;
+  if (RG == 8 && a.bs <= 4) {
+    if constexpr (RG == 8) launch_one<D, MT, MODE, META, 1, 2>(s, a, max_wgs > 1 ? max_wgs / 2 : 1);  // half the workgroups for a host budget
+  } else if (a.bs <= RG) {
+    launch_one<D, MT, MODE, META, 1, 1>(s, a, max_wgs);
+  } else if (RG == 8 || a.bs <= 2 * RG) {
+    launch_one<D, MT, MODE, META, 2, 1>(s, a, max_wgs);
+  } else {
+    if constexpr (RG == 4) launch_one<D, MT, MODE, META, 4, 1>(s, a, max_wgs);
+  }
 }
 
 template <int D, int MT>
 int launch_store(hipStream_t s, int mode, const StoreArgs& a, int64_t max_wgs) {
-  const int64_t pairs = (int64_t)a.n_blocks * a.n_kv;
-  int64_t wgs = (pairs + kWaves - 1) / kWaves;
-  if (wgs > max_wgs) wgs = max_wgs;
-  const dim3 grid((unsigned)wgs);
   const bool meta = a.kmin != nullptr;
   switch (mode) {
-    case MODE_META: hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_META, true>), grid, dim3(kThreads), 0, s, a); break;
-    case MODE_COPY:
-      if (meta) {
-        hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_COPY, true>), grid, dim3(kThreads), 0, s, a);
-      } else {
-        hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_COPY, false>), grid, dim3(kThreads), 0, s, a);
-      }
-      break;
-    case MODE_INT8:
-      if (meta) {
-        hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_INT8, true>), grid, dim3(kThreads), 0, s, a);
-      } else {
-        hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_INT8, false>), grid, dim3(kThreads), 0, s, a);
-      }
-      break;
-    case MODE_UNPACK: hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_UNPACK, true>), grid, dim3(kThreads), 0, s, a); break;
-    default:
-      hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE_META_FROM_I8, true>), grid, dim3(kThreads), 0, s, a);
-      break;
+    case MODE_META: launch_rows<D, MT, MODE_META, true>(s, a, max_wgs); break;
+    case MODE_COPY: meta ? launch_rows<D, MT, MODE_COPY, true>(s, a, max_wgs) : launch_rows<D, MT, MODE_COPY, false>(s, a, max_wgs); break;
+    case MODE_INT8: meta ? launch_rows<D, MT, MODE_INT8, true>(s, a, max_wgs) : launch_rows<D, MT, MODE_INT8, false>(s, a, max_wgs); break;
+    case MODE_UNPACK: launch_one<D, MT, MODE_UNPACK, true, 0, 1>(s, a, max_wgs); break;
+    default: launch_one<D, MT, MODE_META_FROM_I8, true, 0, 1>(s, a, max_wgs); break;
   }
   LKV_CHECK_LAUNCH("store_blocks");
   return LKV_OK;
