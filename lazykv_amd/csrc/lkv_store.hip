@@ -175,8 +175,14 @@ struct Rows {
   static constexpr int W = 2 * (int)sizeof(typename lkv::Elem<MT>::T);  // words of a lane's 8 channels
 };
 
-// A chunk of 16 rows, or, for blocks of fewer, of NI loads' RG * NI rows.
-template <int D, int MT, int NI>
+// Whether a lane's 8 channels are two runs of 4, in the row's two halves: float32 rows copied as they are, whose two 16-byte
+// accesses a lane each cover the row's lanes without gaps then (256 blocks of 16 tokens, 8 heads, d 64, into a dense cache 7.3 -> 6.1 us; 2,048
+// with their metadata 55.7 -> 49.8). Records keep 8 channels together (8 bytes of codes a store).
+template <int MT, int MODE>
+constexpr bool kSplitRow = MT == LKV_F32 && MODE != MODE_INT8;
+
+// A chunk of 16 rows, or, for blocks of fewer, of NI loads' RG * NI rows. SECOND: words from a lane's first four to its next.
+template <int D, int MT, int NI, int SECOND>
 struct RowChunk {
   uint32_t w[NI][Rows<D, MT>::W];
   // Rows t0 + r + RG i of the pair at p (this lane's channels); a row past the block reads row 0 instead, which
@@ -189,7 +195,7 @@ struct RowChunk {
       const uint32_t* at = (const uint32_t*)(p + (int64_t)(row < bs ? row : 0) * D);
 #pragma unroll
       for (int j = 0; j < R::W; j += 4) {
-        const u32x4_a4 x = *(const u32x4_a4*)(at + j);
+        const u32x4_a4 x = *(const u32x4_a4*)(at + j / 4 * SECOND);
         w[i][j] = x.x;
         w[i][j + 1] = x.y;
         w[i][j + 2] = x.z;
@@ -205,7 +211,7 @@ struct RowChunk {
       if (row < bs) {
         uint32_t* at = (uint32_t*)(p + (int64_t)row * D);
 #pragma unroll
-        for (int j = 0; j < R::W; j += 4) *(u32x4_a4*)(at + j) = u32x4_a4{w[i][j], w[i][j + 1], w[i][j + 2], w[i][j + 3]};
+        for (int j = 0; j < R::W; j += 4) *(u32x4_a4*)(at + j / 4 * SECOND) = u32x4_a4{w[i][j], w[i][j + 1], w[i][j + 2], w[i][j + 3]};
       }
     }
   }
@@ -309,10 +315,11 @@ __device__ __forceinline__ uint2 quantise8(const float (&x)[8], const float (&mn
   return make_uint2(w[0] ^ 0x80808080u, w[1] ^ 0x80808080u);
 }
 
-// The block's key metadata from the lanes that own its channels.
-template <int D, int LPR, int GROUPS>
+// The block's key metadata from the lanes that own its channels (SPLIT: kSplitRow's).
+template <int D, int LPR, int GROUPS, bool SPLIT>
 __device__ __forceinline__ void write_owned(const StoreArgs& a, int b, int h, int c, int lane, const float (&mn)[8], const float (&mx)[8]) {
-  const int64_t base = (int64_t)h * a.meta_hstride + (int64_t)b * D + c * 8 + own_channel<LPR, GROUPS>(lane);
+  const int own = own_channel<LPR, GROUPS>(lane);  // the lane's channels own .. own + 8 / GROUPS - 1 lie in one half
+  const int64_t base = (int64_t)h * a.meta_hstride + (int64_t)b * D + (SPLIT ? c * 4 + own % 4 + (own >= 4 ? D / 2 : 0) : c * 8 + own);
 #pragma unroll
   for (int i = 0; i < 8 / GROUPS; ++i) {
     lkv::store_any(a.kmin, base + i, a.meta_dtype, mn[i]);
@@ -346,17 +353,19 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
   constexpr bool kRange = META || MODE == MODE_INT8;  // the keys' range is wanted
   const auto lower = [](float p, float q) { return fminf(p, q); };
   const auto upper = [](float p, float q) { return fmaxf(p, q); };
-  const int64_t soff = (int64_t)b * a.s_bstride + (int64_t)h * a.s_hstride + c * 8;
+  constexpr bool SPLIT = kSplitRow<MT, MODE>;
+  const int first = c * (SPLIT ? 4 : 8);  // the lane's first channel
+  const int64_t soff = (int64_t)b * a.s_bstride + (int64_t)h * a.s_hstride + first;
   const T* sk = (const T*)a.sk + soff;
   const T* sv = (const T*)a.sv + soff;
-  RowChunk<D, MT, NI> k, v;
+  RowChunk<D, MT, NI, SPLIT ? D / 2 : 4> k, v;
   k.load(sk, 0, bs, r);
   if constexpr (MODE != MODE_META) v.load(sv, 0, bs, r);
 
   T* dk = nullptr;
   T* dv = nullptr;
   if constexpr (MODE == MODE_COPY) {
-    const int64_t doff = (int64_t)b * a.d_bstride + (int64_t)h * a.d_hstride + c * 8;
+    const int64_t doff = (int64_t)b * a.d_bstride + (int64_t)h * a.d_hstride + first;
     dk = (T*)a.dk + doff;
     dv = (T*)a.dv + doff;
   }
@@ -394,7 +403,7 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
     reduce_channels<R::LPR, GROUPS>(mx, lane, upper);
   }
   if constexpr (MODE != MODE_INT8) {
-    if constexpr (META) write_owned<D, R::LPR, GROUPS>(a, b, h, c, lane, mn, mx);
+    if constexpr (META) write_owned<D, R::LPR, GROUPS, SPLIT>(a, b, h, c, lane, mn, mx);
   } else {
     uint8_t* rec = (uint8_t*)a.dk + (int64_t)b * a.d_bstride + (int64_t)h * a.d_hstride;
     uint16_t* sc = (uint16_t*)(rec + 2 * bs * D);
@@ -474,7 +483,7 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
     if constexpr (META) {
       reduce_channels<R::LPR, GROUPS>(dmn, lane, lower);
       reduce_channels<R::LPR, GROUPS>(dmx, lane, upper);
-      write_owned<D, R::LPR, GROUPS>(a, b, h, c, lane, dmn, dmx);
+      write_owned<D, R::LPR, GROUPS, false>(a, b, h, c, lane, dmn, dmx);
     }
   }
 }
