@@ -327,8 +327,9 @@ __device__ __forceinline__ void write_owned(const StoreArgs& a, int b, int h, in
   }
 }
 
-// PPW: pairs of the wave, each in 64 / PPW lanes (two where one load of the wave has the rows of two blocks).
-template <int D, int MT, int MODE, bool META, int NI, int PPW>
+// PPW: pairs of the wave, each in 64 / PPW lanes (two where one load of the wave has the rows of two blocks). LONG: records of
+// blocks of more than one chunk, whose rows are loaded again when the keys' range is known.
+template <int D, int MT, int MODE, bool META, int NI, int PPW, bool LONG>
 __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
   using T = typename lkv::Elem<MT>::T;
   using R = Rows<D, MT>;
@@ -360,7 +361,7 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
   const T* sv = (const T*)a.sv + soff;
   RowChunk<D, MT, NI, SPLIT ? D / 2 : 4> k, v;
   k.load(sk, 0, bs, r);
-  if constexpr (MODE != MODE_META) v.load(sv, 0, bs, r);
+  if constexpr (MODE == MODE_COPY || (MODE == MODE_INT8 && !LONG)) v.load(sv, 0, bs, r);
 
   T* dk = nullptr;
   T* dv = nullptr;
@@ -426,7 +427,7 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
       dmx[e] = -INFINITY;
     }
     for (int t0 = 0; t0 < bs; t0 += 16) {
-      if (bs > 16) {  // one chunk: the keys and values are still in their registers
+      if constexpr (LONG) {  // one chunk's keys and values are still in their registers
         k.load(sk, t0, bs, r);
         v.load(sv, t0, bs, r);
       }
@@ -490,7 +491,7 @@ __device__ __forceinline__ void store_rows(const StoreArgs& a, int64_t pair) {
 
 // A wave takes PPW (block, head) pairs at a time, the grid striding over the pairs. Waves never synchronise with
 // each other, so a grid smaller than the pair count (a host destination) is just a longer loop.
-template <int D, int MT, int MODE, bool META, int NI, int PPW>
+template <int D, int MT, int MODE, bool META, int NI, int PPW, bool LONG>
 __global__ __launch_bounds__(kThreads) void store_blocks_kernel(StoreArgs a) {
   const int64_t total = (int64_t)a.n_blocks * a.n_kv;
   constexpr int kLanes = 64 / PPW;
@@ -498,16 +499,16 @@ __global__ __launch_bounds__(kThreads) void store_blocks_kernel(StoreArgs a) {
     if constexpr (MODE == MODE_META_FROM_I8 || MODE == MODE_UNPACK) {
       store_record<D, MT, MODE>(a, pair);  // `pair` is wave-uniform
     } else {
-      store_rows<D, MT, MODE, META, NI, PPW>(a, pair);  // uniform over kLanes lanes, which exchange with no others
+      store_rows<D, MT, MODE, META, NI, PPW, LONG>(a, pair);  // uniform over kLanes lanes, which exchange with no others
     }
 }
 
-template <int D, int MT, int MODE, bool META, int NI, int PPW>
+template <int D, int MT, int MODE, bool META, int NI, int PPW, bool LONG = false>
 void launch_one(hipStream_t s, const StoreArgs& a, int64_t max_wgs) {
   const int64_t pairs = (int64_t)a.n_blocks * a.n_kv;
   int64_t wgs = (pairs + kWaves * PPW - 1) / (kWaves * PPW);
   if (wgs > max_wgs) wgs = max_wgs;
-  hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE, META, NI, PPW>), dim3((unsigned)wgs), dim3(kThreads), 0, s, a);
+  hipLaunchKernelGGL((store_blocks_kernel<D, MT, MODE, META, NI, PPW, LONG>), dim3((unsigned)wgs), dim3(kThreads), 0, s, a);
 }
 
 // The instance for blocks of a.bs tokens: as many loads of RG rows as they fill, up to a 16-row chunk's, and two 4-token blocks in a
@@ -516,7 +517,9 @@ void launch_one(hipStream_t s, const StoreArgs& a, int64_t max_wgs) {
 template <int D, int MT, int MODE, bool META>
 void launch_rows(hipStream_t s, const StoreArgs& a, int64_t max_wgs) {
   constexpr int RG = Rows<D, MT>::RG;
-  if (RG == 8 && a.bs <= 4) {
+  if (MODE == MODE_INT8 && a.bs > 16) {
+    if constexpr (MODE == MODE_INT8) launch_one<D, MT, MODE, META, 16 / RG, 1, true>(s, a, max_wgs);
+  } else if (RG == 8 && a.bs <= 4) {
     if constexpr (RG == 8) launch_one<D, MT, MODE, META, 1, 2>(s, a, max_wgs > 1 ? max_wgs / 2 : 1);  // half the workgroups for a host budget
   } else if (a.bs <= RG) {
     launch_one<D, MT, MODE, META, 1, 1>(s, a, max_wgs);
