@@ -698,3 +698,33 @@ def test_attention_seam_refuses_a_mask_and_reads_only_the_live_prefix() -> None:
     assert len({(c.max_rel_err_decode, c.seconds_decode_growing_median) for c in checks}) == 1
     other = verify_strategies(8, 2, 64, dtype=torch.float16, candidates=("flash",))
     assert not other[0].ok and "unknown strategy" in other[0].error
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("bs", [4, 16, 48])
+def test_pack_at_and_beside_halves(bs: int, d: int) -> None:
+    """Quotients within a few last places of a half, and of the distance from one at which the divide takes over from the reciprocal's
+    estimate: every code is the exact divide's."""
+    from lazykv_amd import quant
+
+    rng = np.random.default_rng(bs + d)
+    m = 64
+    x = np.zeros((m, 2, bs, d), dtype=np.float32)
+    for axis, which in ((1, 0), (2, 1)):  # keys: a range per channel over the tokens; values: per token over the channels
+        scale = np.exp(rng.uniform(-30, 30, size=(m, 1, d) if which == 0 else (m, bs, 1))).astype(np.float32)
+        code = rng.integers(0, 255, size=(m, bs, d)) + 0.5 + rng.choice([0.0, 1e-4, -1e-4, 9e-5, -9e-5, 1e-3], size=(m, bs, d))
+        part = (code * scale).astype(np.float32)
+        for _ in range(3):  # up to three last places to either side
+            step = rng.integers(-1, 2, size=part.shape)
+            part = np.where(step == 0, part, np.nextafter(part, np.where(step > 0, np.float32(np.inf), np.float32(0)))).astype(np.float32)
+        low, high = (part[:, :1], part[:, -1:]) if which == 0 else (part[..., :1], part[..., -1:])
+        low[...] = 0.0
+        high[...] = np.float32(255) * scale
+        x[:, which] = part
+    got = quant.pack(torch.from_numpy(x).cuda()).cpu().numpy().reshape(m, -1)
+    want = []
+    for part, axis in ((x[:, 0], 1), (x[:, 1], 2)):
+        lo, mx = part.min(axis, keepdims=True), part.max(axis, keepdims=True)
+        scale = np.maximum((mx - lo) / np.float32(255), np.finfo(np.float32).tiny)
+        want.append((np.clip(np.rint((part - lo) / scale), 0, 255) - 128).astype(np.int8).reshape(m, -1))
+    assert np.array_equal(got[:, : 2 * bs * d].view(np.int8), np.concatenate(want, axis=1))
