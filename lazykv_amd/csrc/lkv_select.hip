@@ -605,13 +605,13 @@ __device__ __forceinline__ void select_row(const float* __restrict__ row, int n,
 // per head) or 12 (12,288; every key slot a thread holds costs instructions in each phase: at 8,192
 // candidates, against 512 threads of 16, the 128K-token zero-copy step measured 615.23 -> 614.47 us per
 // layer), with the wave index scalar in the scans (as lane masks, the scans' wave tests spilled
-// scalar registers), over rows that are 16-byte aligned and padded to 4 floats (the workspace's). Each
-// thread writes its ids straight to their ascending output positions, or, in sorted mode, to the sort's
+// scalar registers). VEC: rows that are 16-byte aligned and padded to 4 floats (the workspace's) are read as vectors, a caller's dense
+// rows a float at a time. Each thread writes its ids straight to their ascending output positions, or, in sorted mode, to the sort's
 // slots. Against select_row, which reads the row three times: 512 of 8,190 in descending order 20.5 -> 16.0 us
-// with the bound launch, 768 of 12,286 ascending 19.3 -> 11.9.
+// with the bound launch, 768 of 12,286 ascending 19.3 -> 11.9, from dense rows 18.5 -> 13.4.
 constexpr int kSelBlockThreads = 1024;
 constexpr int kSelBlockCap = kSelBlockThreads * 12;
-template <int KPT, bool SORTED>
+template <int KPT, bool SORTED, bool VEC>
 __global__ __launch_bounds__(kSelBlockThreads) void select_block_kernel(const float* __restrict__ bounds, int64_t bstride,
                                                                         int n_cand, int k, int cand_offset,
                                                                         const int32_t* __restrict__ map,
@@ -620,7 +620,7 @@ __global__ __launch_bounds__(kSelBlockThreads) void select_block_kernel(const fl
   __shared__ lkv::SelectLds<kSelBlockThreads, KPT> L;
   const int h = blockIdx.x;
   const float* row = bounds + (int64_t)h * bstride;
-  const lkv::SelectPick pk = lkv::block_top_k<kSelBlockThreads, KPT, true>(row, true, n_cand, k, L);
+  const lkv::SelectPick pk = lkv::block_top_k<kSelBlockThreads, KPT, true>(row, VEC, n_cand, k, L);
   int32_t* out_h = out_idx + (int64_t)h * idx_stride;
   const int32_t* map_h = map != nullptr ? map + (int64_t)h * bstride : nullptr;  // candidates of the parts below
   int pos = pk.pos;
@@ -652,7 +652,7 @@ __global__ __launch_bounds__(kSelThreads) void select_stream_kernel(const float*
   select_row<true>(bounds + (int64_t)blockIdx.x * bstride, n_cand, k, cand_offset, sorted, out_idx + (int64_t)blockIdx.x * idx_stride, L);
 }
 
-// Any row (a caller's dense bounds).
+// Any row (a caller's dense bounds of more than kSelBlockCap candidates).
 __global__ __launch_bounds__(kSelThreads) void select_kernel(const float* __restrict__ bounds, int64_t bstride, int n_cand, int k,
                                                              int cand_offset, int sorted, int32_t* __restrict__ out_idx,
                                                              int64_t idx_stride) {
@@ -753,17 +753,18 @@ int lkv_launch_bounds(hipStream_t s, const void* q, int q_dtype, const void* kmi
 
 int lkv_select_max_candidates() { return kMaxStreamCand; }
 
-// Up to kSelBlockCap candidates in rows that can be read as vectors: the in-workgroup top-K, which reads the
-// row once. A longer one in parts where `parts` (2 * n_kv * part_stride words) is given and the parts' picks fit the
-// in-workgroup top-K. Any other selection reads the row three times, as 16-byte vectors where the rows allow.
-template <int KPT>
+// Up to kSelBlockCap candidates: the in-workgroup top-K, which reads the row once, as 16-byte vectors where the rows allow (a
+// caller's dense rows may not).
+// A longer one in parts where `parts` (2 * n_kv * part_stride words) is given and the parts' picks fit the in-workgroup top-K
+// (lkv_bound_topk's own rows; the fused calls' workspaces hold no parts). Any other selection reads the row three times.
+template <int KPT, bool VEC>
 static void launch_select_block(hipStream_t s, const float* bounds, int64_t bstride, int n_kv, int n_cand, int k, int cand_offset, int sorted,
                                 const int32_t* map, int32_t* out_idx, int64_t idx_stride) {
   if (sorted) {
-    hipLaunchKernelGGL((select_block_kernel<KPT, true>), dim3(n_kv), dim3(kSelBlockThreads), 0, s, bounds, bstride, n_cand, k, cand_offset,
+    hipLaunchKernelGGL((select_block_kernel<KPT, true, VEC>), dim3(n_kv), dim3(kSelBlockThreads), 0, s, bounds, bstride, n_cand, k, cand_offset,
                        map, out_idx, idx_stride);
   } else {
-    hipLaunchKernelGGL((select_block_kernel<KPT, false>), dim3(n_kv), dim3(kSelBlockThreads), 0, s, bounds, bstride, n_cand, k, cand_offset,
+    hipLaunchKernelGGL((select_block_kernel<KPT, false, VEC>), dim3(n_kv), dim3(kSelBlockThreads), 0, s, bounds, bstride, n_cand, k, cand_offset,
                        map, out_idx, idx_stride);
   }
 }
@@ -771,10 +772,12 @@ static void launch_select_block(hipStream_t s, const float* bounds, int64_t bstr
 static int launch_select(hipStream_t s, const float* bounds, int64_t bstride, int n_kv, int n_cand, int k, int cand_offset, int sorted,
                          void* parts, int32_t* out_idx, int64_t idx_stride) {
   const bool vec = rows_vector_readable(bounds, bstride, n_cand);
-  if (vec && n_cand <= kSelBlockThreads * 8) {
-    launch_select_block<8>(s, bounds, bstride, n_kv, n_cand, k, cand_offset, sorted, nullptr, out_idx, idx_stride);
-  } else if (vec && n_cand <= kSelBlockCap) {
-    launch_select_block<12>(s, bounds, bstride, n_kv, n_cand, k, cand_offset, sorted, nullptr, out_idx, idx_stride);
+  if (n_cand <= kSelBlockThreads * 8) {
+    vec ? launch_select_block<8, true>(s, bounds, bstride, n_kv, n_cand, k, cand_offset, sorted, nullptr, out_idx, idx_stride)
+        : launch_select_block<8, false>(s, bounds, bstride, n_kv, n_cand, k, cand_offset, sorted, nullptr, out_idx, idx_stride);
+  } else if (n_cand <= kSelBlockCap) {
+    vec ? launch_select_block<12, true>(s, bounds, bstride, n_kv, n_cand, k, cand_offset, sorted, nullptr, out_idx, idx_stride)
+        : launch_select_block<12, false>(s, bounds, bstride, n_kv, n_cand, k, cand_offset, sorted, nullptr, out_idx, idx_stride);
   } else if (vec && parts != nullptr && part_picks(n_cand, k) > 0) {
     const int n_parts = (n_cand + kPartCand - 1) / kPartCand;
     const int64_t ps = (int64_t)part_stride(n_cand, k);
@@ -785,9 +788,9 @@ static int launch_select(hipStream_t s, const float* bounds, int64_t bstride, in
     const int last = n_cand - (n_parts - 1) * kPartCand;
     const int picks = (n_parts - 1) * k + (last < k ? last : k);
     if (picks <= kSelBlockThreads * 8) {
-      launch_select_block<8>(s, key, ps, n_kv, picks, k, cand_offset, sorted, id, out_idx, idx_stride);
+      launch_select_block<8, true>(s, key, ps, n_kv, picks, k, cand_offset, sorted, id, out_idx, idx_stride);
     } else {
-      launch_select_block<12>(s, key, ps, n_kv, picks, k, cand_offset, sorted, id, out_idx, idx_stride);
+      launch_select_block<12, true>(s, key, ps, n_kv, picks, k, cand_offset, sorted, id, out_idx, idx_stride);
     }
   } else if (vec) {
     hipLaunchKernelGGL(select_stream_kernel, dim3(n_kv), dim3(kSelThreads), 0, s, bounds, bstride, n_cand, k, cand_offset, sorted, out_idx,

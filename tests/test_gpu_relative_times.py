@@ -128,3 +128,20 @@ def test_copying_float32_rows_costs_their_bytes() -> None:
         times.append(_us(lambda: kernels.store_blocks(src, dst=dst, n_kv=h, head_dim=d, block_size=bs, first_block=0, n_blocks=n)))
     print(f"copies: float32 {times[0]:.2f} us, float16 {times[1]:.2f}", flush=True)
     assert times[0] < 1.08 * times[1]
+
+
+@pytest.mark.parametrize("n", [12286])
+def test_selection_from_dense_bounds_reads_them_once(n: int) -> None:
+    """Bounds written to the caller's dense rows (not whole 16-byte vectors) against the workspace's padded ones: 18.5 us against 11.3
+    where dense rows were read three times; now 13.4."""
+    from lazykv_amd import kernels
+
+    h, d, k, dt = 8, 64, n // 16, torch.float16
+    a, b = torch.randn((1, h, n, d), device="cuda").to(dt), torch.randn((1, h, n, d), device="cuda").to(dt)
+    kmin, kmax = torch.minimum(a, b), torch.maximum(a, b)
+    q = torch.randn((4 * h, d), device="cuda").to(dt)
+    idx = torch.empty((h, k), dtype=torch.int32, device="cuda")
+    ws = kernels.Workspace()
+    times = [_us(lambda: kernels.bound_topk(q, kmin, kmax, k, out_idx=idx, out_bound=o, ws=ws)) for o in (torch.empty((h, n), device="cuda"), None)]
+    print(f"selection of {k} of {n}: dense rows {times[0]:.1f} us, padded {times[1]:.1f}", flush=True)
+    assert times[0] < 1.4 * times[1]

@@ -86,3 +86,20 @@ def test_long_selections_of_many_blocks(n: int, k: int) -> None:
     values, kmax, q = _metadata("normal", 2, n, n + k)
     want = np.stack([np.sort(np.lexsort((np.arange(n), -values[j]))[:k]) for j in range(2)])
     assert np.array_equal(kernels.bound_topk(q, kmax, kmax, k).cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("kind", ["normal", "one value"])
+@pytest.mark.parametrize(("n", "k"), [(1, 1), (6, 5), (509, 200), (2045, 511), (4093, 1023), (8189, 2047), (8193, 1025), (12285, 2048), (12287, 3), (12289, 700)])
+def test_selection_from_dense_rows_of_any_alignment(n: int, k: int, kind: str) -> None:
+    """Rows that are not whole 16-byte vectors, up to the in-workgroup limit and past it; three heads, so that each row starts at another
+    alignment."""
+    from lazykv_amd import kernels
+
+    h = 3
+    values, kmax, q = _metadata(kind, h, n, n + k)
+    order = [np.lexsort((np.arange(n), -values[j]))[:k] for j in range(h)]
+    dense = torch.empty((h, n), dtype=torch.float32, device="cuda")
+    for sorted_ in (False, True):
+        want = np.stack([o if sorted_ else np.sort(o) for o in order])
+        got = kernels.bound_topk(q, kmax, kmax, k, sorted_=sorted_, out_bound=dense)
+        assert np.array_equal(got.cpu().numpy(), want), sorted_
