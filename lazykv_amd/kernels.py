@@ -593,15 +593,15 @@ def copy_rows(copies: list[tuple[torch.Tensor, torch.Tensor]]) -> None:
     the current stream. A copy the launch does not cover -- another shape, dtype or device, rows that are not contiguous or
     not of whole 2-byte words, tensors that autograd follows in either mode -- is torch's."""
     first = copies[0][0]
-    here = first.is_cuda and first.device.index == torch.cuda.current_device() and 0 < first.shape[0] <= 65535
+    here = first.is_cuda and first.device.index == torch.cuda.current_device() and 0 < first.shape[0] <= 65535 and _forward_level() < 0
     descs, written = [], []
     for dst, src in copies:
         ds, ss = dst.stride(), src.stride()
         es = dst.element_size()
         if (not here or dst.shape != src.shape or src.dtype != dst.dtype or src.device != first.device or dst.device != first.device
                 or ds[-1] != 1 or ss[-1] != 1 or dst.shape[0] != first.shape[0] or src.requires_grad or dst.requires_grad
-                or (es == 1 and (ds[0] | ds[1] | ss[0] | ss[1] | dst.shape[2] | dst.data_ptr() | src.data_ptr()) & 1)
-                or type(src) not in _PLAIN or type(dst) not in _PLAIN or src.is_neg() or dst.is_neg() or _dual(src) or _dual(dst)):
+                or type(src) not in _PLAIN or type(dst) not in _PLAIN
+                or (es == 1 and (ds[0] | ds[1] | ss[0] | ss[1] | dst.shape[2] | dst.data_ptr() | src.data_ptr()) & 1)):
             dst.copy_(src)
             continue
         _, rows, d = dst.shape
@@ -619,9 +619,9 @@ MAX_ROW_COPIES = 8  # LKV_MAX_ROW_COPIES
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
-def _dual(t: torch.Tensor) -> bool:
-    """Whether `t` carries a tangent of forward-mode differentiation."""
-    return torch.autograd.forward_ad.unpack_dual(t).tangent is not None
+def _forward_level() -> int:
+    """The level of forward-mode differentiation, whose tangents a launch would leave behind; negative outside of any."""
+    return getattr(torch.autograd.forward_ad, "_current_level", 0)
 
 
 def packed_pair_bytes(block_size: int, head_dim: int) -> int:
