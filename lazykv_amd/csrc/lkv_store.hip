@@ -637,22 +637,43 @@ extern "C" int lkv_store_blocks(uintptr_t stream, const lkv_kv_source* src, cons
 }
 
 // ---- small row copies -----------------------------------------------------------------------------------
-// Up to 8 copies in one launch, a workgroup per 256 words of one copy's rows of one head. They are bound by the
+// Up to 8 copies in one launch. Small ones are bound by the
 // launch: with six separate copies behind its store, a 200-token turn over a 64K-token tier (8 heads, d 128) took
 // 120.7 us, with one launch 102.6. (For two copies, torch's cost the host less: appending a token 17.2 us against 18.3.)
 namespace {
 
 struct RowCopies {
   lkv_row_copy c[LKV_MAX_ROW_COPIES];
+  int32_t end[LKV_MAX_ROW_COPIES];  // workgroups up to and including copy i's
 };
 
+// A workgroup per 256 words of its copy, the copies one after another. (As a grid axis of their own, as long as the longest, a turn of
+// 65,536 tokens beside the sink and the current block, 8 heads at d 128, launched 131,072 workgroups with nothing to do: 117.0 us by torch's
+// copies, 120.6 so, 94.5
+// here.)
 template <typename W>
 __global__ __launch_bounds__(256) void copy_rows_kernel(RowCopies a) {
-  const lkv_row_copy& c = a.c[blockIdx.z];
-  const int words = c.row_bytes / (int)sizeof(W);
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int g = blockIdx.x;
+  int n = 0, first = 0;
+#pragma unroll
+  for (int i = 0; i + 1 < LKV_MAX_ROW_COPIES; ++i) {
+    if (g >= a.end[i]) {
+      n = i + 1;
+      first = a.end[i];
+    }
+  }
+  const lkv_row_copy& c = a.c[n];
+  const uint32_t words = (uint32_t)c.row_bytes / (uint32_t)sizeof(W);
+  const int64_t i = (int64_t)(g - first) * 256 + threadIdx.x;
   if (i >= (int64_t)c.rows * words) return;
-  const int64_t row = i / words, w = i % words;
+  int64_t row, w;
+  if ((int64_t)c.rows * words <= 0xffffffffLL) {  // workgroup-uniform: a 64-bit division costs several of 32
+    row = (uint32_t)i / words;
+    w = (uint32_t)i % words;
+  } else {
+    row = i / words;
+    w = i % words;
+  }
   const char* s = (const char*)c.src + blockIdx.y * c.src_head_stride + row * c.src_row_stride;
   char* d = (char*)c.dst + blockIdx.y * c.dst_head_stride + row * c.dst_row_stride;
   ((W*)d)[w] = ((const W*)s)[w];
@@ -666,7 +687,6 @@ extern "C" int lkv_copy_rows(uintptr_t stream, const lkv_row_copy* copies, int n
   LKV_CHECK_ARG(heads > 0 && heads <= 65535, "bad head count %d", heads);
   RowCopies a{};
   int used = 0;
-  int64_t most = 0;
   uint64_t mix = 0;  // the low bits set anywhere decide the word
   for (int i = 0; i < n; ++i) {
     const lkv_row_copy& c = copies[i];
@@ -676,15 +696,17 @@ extern "C" int lkv_copy_rows(uintptr_t stream, const lkv_row_copy* copies, int n
     mix |= (uint64_t)(uintptr_t)c.src | (uint64_t)(uintptr_t)c.dst | (uint64_t)c.src_head_stride | (uint64_t)c.src_row_stride |
            (uint64_t)c.dst_head_stride | (uint64_t)c.dst_row_stride | (uint64_t)c.row_bytes;
     a.c[used++] = c;
-    const int64_t bytes = (int64_t)c.rows * c.row_bytes;
-    if (bytes > most) most = bytes;
   }
   LKV_CHECK_ARG((mix & 1) == 0, "row copies move whole 2-byte elements");
   if (used == 0) return LKV_OK;
   const int word = (mix & 15) == 0 ? 16 : (mix & 3) == 0 ? 4 : 2;
-  const int64_t groups = (most / word + 255) / 256;
-  LKV_CHECK_ARG(groups <= 0x7fffffff, "row copy too large");
-  const dim3 grid((unsigned)groups, (unsigned)heads, (unsigned)used);
+  int64_t groups = 0;
+  for (int i = 0; i < LKV_MAX_ROW_COPIES; ++i) {
+    if (i < used) groups += ((int64_t)a.c[i].rows * (a.c[i].row_bytes / word) + 255) / 256;
+    LKV_CHECK_ARG(groups <= 0x7fffffff, "row copy too large");
+    a.end[i] = (int32_t)groups;
+  }
+  const dim3 grid((unsigned)groups, (unsigned)heads);
   hipStream_t s = (hipStream_t)stream;
   if (word == 16) {
     hipLaunchKernelGGL(copy_rows_kernel<uint4>, grid, dim3(256), 0, s, a);
