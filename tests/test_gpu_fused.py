@@ -66,17 +66,38 @@ def test_select_decode_equals_the_two_launch_path_and_the_oracle(h: int, g: int,
     _check_one_call(h, g, n, bs, d, k, fill, dt, where)
 
 
-# Launches whose decode instance is not a matrix-core one over HBM pairs: a float32 query takes the
-# 8-wave vector instance, which has no selecting form, so the one-call step selects in its own
-# launch and then decodes as the two-call path does; int8 records at head_dim 128 with a group of 4
-# take the 4-wave instance over the HBM plan, which selects inside the launch only up to 16 keys per
-# thread of its 256 (4,096 candidates).
+# A float32 query (the last column) over HBM keeps off the matrix cores. Over 16-bit pairs it takes the 8-wave vector instance, which
+# has no selecting form, so the one-call step selects in its own launch and then decodes as the two-call path does; over int8 records
+# the 8-wave vector instance that selects inside itself (in 2,048, 4,096 or 8,192 key slots); int8 records at head_dim 128 under groups
+# of 4, and groups of 8, take the 4-wave instance over the same plan, which selects inside only up to 16 keys per thread of its 256
+# (4,096 candidates). A model-dtype query takes the matrix cores, but for int8 records under one head a KV head, the 8-wave vector
+# instance again.
 CASES_OTHER_INSTANCES = [
     (8, 4, 2048, 16, 64, 512, 16, torch.float16, "hbm", True),
     (8, 4, 8192, 16, 128, 512, 16, torch.bfloat16, "hbm", True),
     (2, 2, 700, 16, 128, 50, 7, torch.bfloat16, "hbm", True),
-    (4, 4, 4098, 16, 128, 300, 9, torch.bfloat16, "int8-hbm", False),  # 4,096 candidates: inside, 16 keys per thread
-    (4, 4, 4102, 16, 128, 300, 9, torch.bfloat16, "int8-hbm", False),  # 4,100: the selection's own launch
+    (4, 4, 4098, 16, 128, 300, 9, torch.bfloat16, "int8-hbm", False),
+    (4, 4, 4102, 16, 128, 300, 9, torch.bfloat16, "int8-hbm", False),
+    (4, 4, 4098, 16, 128, 300, 9, torch.bfloat16, "int8-hbm", True),  # 4,096 candidates: inside, 16 keys per thread
+    (4, 4, 4099, 16, 128, 300, 9, torch.bfloat16, "int8-hbm", True),  # 4,097: the selection's own launch
+    (2, 1, 2050, 16, 64, 200, 5, torch.float16, "int8-hbm", True),
+    (2, 1, 4099, 16, 64, 400, 16, torch.float16, "int8-hbm", True),
+    (2, 2, 2051, 16, 64, 200, 5, torch.bfloat16, "int8-hbm", True),
+    (2, 2, 8194, 16, 64, 600, 1, torch.float16, "int8-hbm", True),  # 8,192: the most selected inside
+    (2, 4, 2050, 16, 64, 700, 5, torch.float16, "int8-hbm", True),  # several records a wave: the four-record rounds
+    (2, 4, 4098, 16, 64, 1500, 9, torch.float16, "int8-hbm", True),
+    (2, 4, 8195, 16, 64, 600, 16, torch.float16, "int8-hbm", True),  # 8,193: the selection's own launch
+    (3, 2, 300, 32, 128, 70, 30, torch.bfloat16, "int8-hbm", True),  # blocks of two chunks
+    (1, 8, 4098, 16, 64, 300, 9, torch.float16, "hbm", True),
+    (1, 8, 4099, 16, 64, 300, 9, torch.float16, "hbm", True),
+    (1, 8, 4098, 16, 128, 300, 9, torch.bfloat16, "int8-hbm", True),
+    (1, 8, 4099, 16, 128, 300, 9, torch.bfloat16, "int8-hbm", True),
+    (2, 1, 2050, 16, 64, 200, 5, torch.float16, "int8-hbm", False),  # one head a KV head: vector, at both head sizes
+    (2, 1, 8194, 16, 128, 600, 16, torch.bfloat16, "int8-hbm", False),
+    (3, 1, 500, 4, 64, 90, 3, torch.float16, "int8-hbm", False),
+    (3, 1, 500, 4, 128, 90, 3, torch.bfloat16, "int8-hbm", False),  # too few rows a block: matrix cores
+    (2, 1, 130, 64, 64, 40, 60, torch.float16, "int8-hbm", False),  # blocks that do not fill the waves: matrix cores
+    (32, 1, 130, 64, 64, 60, 60, torch.float16, "int8-hbm", False),  # and that do: vector
 ]
 
 
