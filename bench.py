@@ -258,16 +258,25 @@ def _pmc_file() -> dict:
         return {}
 
 
-def step_kernels(fused: bool, in_decode: bool, n_cand: int) -> str:
+def select_kernels(fused: bool, n_cand: int, k: int) -> list[str]:
+    """The launches of a selection that is not made inside another, by the library's dispatch rules: select_block_kernel up to
+    12,288 candidates; beyond 16,384, lkv_bound_topk's rows in parts of 8,192 while the parts' k picks each fit select_block_kernel
+    (the one-call step has no room for parts); select_stream_kernel for the rest."""
+    if n_cand <= 12288:
+        return ["select_block_kernel"]
+    if not fused and n_cand > 16384 and -(-n_cand // 8192) * k <= 12288:
+        return ["select_part_kernel", "select_block_kernel"]
+    return ["select_stream_kernel"]
+
+
+def step_kernels(fused: bool, in_decode: bool, n_cand: int, k: int) -> str:
     """One layer's launches, as rocprof names them, by the library's dispatch rules: the matrix-core
     bound for a model-dtype query with aligned rows; the top K inside the decode launch when the
-    fused call selects there, else select_block_kernel up to 12,288 candidates and
-    select_stream_kernel beyond."""
+    fused call selects there, else in launches of its own."""
     call = "one lkv_select_decode call: " if fused else "lkv_bound_topk + lkv_sparse_decode: "
     if fused and in_decode:
         return call + "bound_kernel_mf, sparse_decode_kernel choosing the top K itself, decode_merge_wave_kernel"
-    sel = "select_block_kernel" if n_cand <= 12288 else "select_stream_kernel"
-    return call + f"bound_kernel_mf, {sel}, sparse_decode_kernel, decode_merge_wave_kernel"
+    return call + ", ".join(["bound_kernel_mf", *select_kernels(fused, n_cand, k), "sparse_decode_kernel", "decode_merge_wave_kernel"])
 
 
 def pmc_traffic(workload: str) -> dict:
@@ -586,8 +595,8 @@ def run_decode(args: argparse.Namespace, spec: dict) -> dict:
                          "(rank_dtype=None)",
             "rank_model_set_agreement": rank_agreement,
             "dense_layers": 0, "launch": "eager" if args.eager else "hip_graph",
-            "launches_per_layer": 3 if (m["fused"] and kernels._lib.selects_in_decode(n_cand, res[main_leg]["host_sel"], N_Q // H)) else 4,
-            "step_kernels": step_kernels(m["fused"], kernels._lib.selects_in_decode(n_cand, res[main_leg]["host_sel"], N_Q // H), n_cand),
+            "launches_per_layer": 3 if (m["fused"] and kernels._lib.selects_in_decode(n_cand, res[main_leg]["host_sel"], N_Q // H)) else 3 + len(select_kernels(m["fused"], n_cand, m["k"])),
+            "step_kernels": step_kernels(m["fused"], kernels._lib.selects_in_decode(n_cand, res[main_leg]["host_sel"], N_Q // H), n_cand, m["k"]),
             "host_memory": "fine-grained" if args.coherent else "coarse-grained",
         },
         "host_syncs_per_layer": 0,

@@ -62,8 +62,8 @@ def kernels() -> list[dict]:
 
 def test_every_kernel_of_the_path_is_in_the_library(kernels) -> None:  # noqa: ANN001
     names = " ".join(k[".name"] for k in kernels)
-    for want in ("bound_kernel", "select_kernel", "select_stream_kernel", "sparse_decode_kernel", "decode_merge_kernel", "decode_merge_wave_kernel",
-                 "residency_kernel", "store_blocks_kernel", "merge_lse_kernel", "stream_read_kernel"):
+    for want in ("bound_kernel", "bound_kernel_mf", "select_kernel", "select_block_kernel", "select_part_kernel", "select_stream_kernel",
+                 "sparse_decode_kernel", "decode_merge_kernel", "decode_merge_wave_kernel", "residency_kernel", "store_blocks_kernel", "copy_rows_kernel", "merge_lse_kernel", "stream_read_kernel"):
         assert want in names, want
 
 
@@ -73,7 +73,7 @@ def test_no_kernel_uses_private_memory(kernels) -> None:  # noqa: ANN001
 
 
 def _decode_group(name: str) -> int | None:
-    """G of a sparse_decode_kernel<D, MT, G, NT, I8> instance, from its mangled name."""
+    """G of a sparse_decode_kernel<D, MT, G, NT, I8, MF, SEL> instance, from its mangled name."""
     m = re.search(r"sparse_decode_kernelILi\d+ELi\d+ELi(\d+)E", name)
     return int(m.group(1)) if m else None
 
@@ -88,8 +88,22 @@ def test_no_kernel_spills_registers(kernels) -> None:  # noqa: ANN001
 
 
 def test_model_dtype_decode_kernels_fit_eight_wave_workgroups(kernels) -> None:  # noqa: ANN001
-    """The 512-thread decode kernels (no int8 code) keep at most 256 VGPRs, so two waves fit on
+    """The 512-thread decode kernels keep at most 256 VGPRs, so two waves fit on
     each SIMD and one workgroup per CU stays resident."""
     hbm = [k for k in kernels if "sparse_decode_kernel" in k[".name"] and k[".max_flat_workgroup_size"] == 512]
     assert hbm
     assert all(k[".vgpr_count"] <= 256 and k[".agpr_count"] == 0 for k in hbm), [(k[".name"], k[".vgpr_count"]) for k in hbm]
+
+
+@pytest.mark.parametrize(("fused", "n_cand", "k", "want"), [
+    (True, 8193, 600, ["select_block_kernel"]), (False, 12288, 2048, ["select_block_kernel"]), (False, 12289, 16, ["select_stream_kernel"]),
+    (False, 16384, 16, ["select_stream_kernel"]), (False, 16385, 4096, ["select_part_kernel", "select_block_kernel"]), (False, 16385, 4097, ["select_stream_kernel"]),
+    (False, 65535, 1024, ["select_part_kernel", "select_block_kernel"]), (True, 65535, 1024, ["select_stream_kernel"]),
+])
+def test_the_benchmark_names_the_kernels_a_selection_launches(kernels, fused: bool, n_cand: int, k: int, want: list[str]) -> None:  # noqa: ANN001
+    import bench
+
+    assert bench.select_kernels(fused, n_cand, k) == want
+    names = " ".join(kk[".name"] for kk in kernels)
+    assert all(w in names for w in want)
+    assert all(w in bench.step_kernels(fused, False, n_cand, k) for w in want)
