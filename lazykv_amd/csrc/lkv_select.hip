@@ -11,11 +11,16 @@
 // row (head_dim channels), so each wave-wide load covers 4 blocks; every lane keeps q+ and q- for
 // its channels of the G query heads in registers. The row sum is a 4-step DPP reduction; the max
 // over the group is taken in registers. The float32 bounds go to a scratch row per head.
+// bound_kernel_mf: the same on the matrix cores, for a query of the metadata's dtype over aligned rows.
 //
-// Selection: one 1024-thread workgroup per KV head, by range-adaptive radix select: each pass
-// histograms the keys of the current range into at most 2048 bins scaled to that range (so the
-// first pass spreads the clustered bounds instead of piling them into a few exponent bins) and
-// keeps the bin holding the K-th key; once that bin holds few keys they are ranked directly.
+// Selection, by range-adaptive radix select: each pass histograms the keys of the current range into
+// at most 2048 bins scaled to that range (so the first pass spreads the clustered bounds instead of
+// piling them into a few exponent bins) and keeps the bin holding the K-th key; once that bin holds
+// few keys they are ranked directly. One 1024-thread workgroup per KV head, with the row in registers
+// up to 12,288 candidates (select_block_kernel) and reading it three times beyond
+// (select_stream_kernel, select_kernel); beyond 16,384 in parts of 8,192, a workgroup each, and then
+// the parts' picks (select_part_kernel, select_block_kernel) where the caller's workspace has room for
+// them. The decode and residency launches of a one-call step select inside themselves up to 8,192.
 // Scoring and selection are separate launches so that no workgroup has to publish its bounds across
 // XCDs inside one launch (a device-scope release writes back the L2); the kernel boundary does that
 // once.
