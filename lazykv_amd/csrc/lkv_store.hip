@@ -516,7 +516,7 @@ void launch_one(hipStream_t s, const StoreArgs& a, int64_t max_wgs) {
 
 // The instance for blocks of a.bs tokens: as many loads of RG rows as they fill, up to a 16-row chunk's, and two 4-token blocks in a
 // load of 8 rows. (A whole chunk's loads for all: 65,536 pairs of 4 x 64 float16 packed with their metadata in 98 us, of 4 x 128 in 157;
-// here in 45 and 85.)
+// here in 43 and 82.)
 template <int D, int MT, int MODE, bool META>
 void launch_rows(hipStream_t s, const StoreArgs& a, int64_t max_wgs) {
   constexpr int RG = Rows<D, MT>::RG;
