@@ -728,3 +728,71 @@ def test_pack_at_and_beside_halves(bs: int, d: int) -> None:
         scale = np.maximum((mx - lo) / np.float32(255), np.finfo(np.float32).tiny)
         want.append((np.clip(np.rint((part - lo) / scale), 0, 255) - 128).astype(np.int8).reshape(m, -1))
     assert np.array_equal(got[:, : 2 * bs * d].view(np.int8), np.concatenate(want, axis=1))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("bs", [4, 8, 12, 16, 20])
+@pytest.mark.parametrize(("h", "n"), [(1, 1), (3, 1), (1, 9), (5, 3)])
+def test_stores_of_every_row_count_and_an_odd_number_of_pairs(h: int, n: int, bs: int, d: int) -> None:
+    """Blocks that fill one, two or four of a chunk's loads, two of them a wave at 4 tokens and d 64, the last wave half empty: pairs, records
+    and metadata match the oracle's, and nothing past the range is written."""
+    from lazykv_amd import kernels
+    from lazykv_amd.quant import packed_pair_bytes
+
+    gen = torch.Generator().manual_seed(100 * bs + 10 * h + n)
+    pool = torch.randn((n + 2, h, 2, bs, d), generator=gen).to(torch.bfloat16)
+    recs = R.pack(_bits(pool), "bf16")
+    src = kernels.pool_source(pool.cuda())
+    for what in ("copy", "records", "metadata"):
+        kmin = torch.full((1, h, n + 2, d), 7.0, dtype=torch.bfloat16, device="cuda")
+        kmax = torch.full_like(kmin, 7.0)
+        keys = pool[:, :, 0].float()
+        dst = None
+        if what == "copy":
+            store = torch.full(tuple(pool.shape), 7.0, dtype=torch.bfloat16, device="cuda")
+            dst = kernels.pool_source(store)
+        elif what == "records":
+            store = torch.full((n + 2, h, packed_pair_bytes(bs, d)), 7, dtype=torch.uint8, device="cuda")
+            dst = kernels.record_source(store, torch.bfloat16)
+            keys = torch.from_numpy(R.to_f32(R.unpack(recs.reshape((n + 2) * h, -1), bs, d, "bf16"), "bf16")).view(n + 2, h, 2, bs, d)[:, :, 0]
+        kernels.store_blocks(src, dst=dst, n_kv=h, head_dim=d, block_size=bs, first_block=1, n_blocks=n, kmin=kmin, kmax=kmax)
+        if dst is not None:
+            want = pool if what == "copy" else torch.from_numpy(recs)
+            got = store.cpu()
+            assert torch.equal(got[1 : n + 1], want[1 : n + 1]), what
+            assert (got[0] == 7).all() and (got[n + 1] == 7).all(), what
+        for meta, ref in ((kmin, keys.amin(2)), (kmax, keys.amax(2))):
+            got = meta[0].float().cpu().transpose(0, 1)  # [n + 2, h, d]
+            assert torch.equal(got[1 : n + 1], ref[1 : n + 1]), what
+            assert (got[0] == 7).all() and (got[n + 1] == 7).all(), what
+
+
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize(("g", "d", "bs", "n", "first", "k"), [
+    (4, 64, 4, 700, 3, 60), (1, 64, 4, 333, 0, 5), (4, 128, 16, 1, 0, 0), (2, 64, 16, 9, 0, 1), (8, 64, 16, 300, 7, 299), (1, 128, 20, 130, 1, 40),
+    (4, 64, 36, 77, 0, 10), (2, 128, 64, 65, 2, 20), (4, 128, 256, 17, 0, 3), (1, 64, 256, 40, 5, 0),
+])
+def test_remainder_runs_of_every_block_size(g: int, d: int, bs: int, n: int, first: int, k: int, int8: bool) -> None:
+    """The blocks a selection leaves, as chunks over the waves of their runs: blocks of one partial chunk to sixteen, runs shorter than a
+    workgroup, runs of which nearly all or none are excluded. The selection and its remainder are the whole range: full attention."""
+    from lazykv_amd import kernels
+
+    h, scale, dt = 2, d**-0.5, torch.bfloat16
+    gen = torch.Generator().manual_seed(n + bs)
+    pool = torch.randn((n, h, 2, bs, d), generator=gen).to(dt)
+    if int8:
+        recs = R.pack(_bits(pool), "bf16")
+        src = kernels.record_source(torch.from_numpy(recs).cuda(), dt)
+        values = torch.from_numpy(R.to_f32(R.unpack(recs.reshape(n * h, -1), bs, d, "bf16"), "bf16")).view(n, h, 2, bs, d).double()
+    else:
+        src = kernels.pool_source(pool.cuda())
+        values = pool.double()
+    q = torch.randn((h * g, d), generator=gen).to(dt)
+    idx = torch.stack([first + torch.randperm(n - first, generator=gen)[:k].sort().values for _ in range(h)]).to(torch.int32).cuda() if k else None
+    out, lse = kernels.sparse_decode(q.cuda(), n_kv=h, block_size=bs, scale=scale, sel=src if k else None, idx=idx, rem=src, rem_range=(first, n), out_dtype=torch.float32)
+    # float32 scores of up to 30 are off by 2^-22 of that each: the weights, and their sums, by some 1e-5.
+    for j in range(h):
+        keys, vals = (values[first:, j, i].reshape(-1, d) for i in (0, 1))
+        s = (q[j * g : (j + 1) * g].double() @ keys.T.contiguous()) * scale
+        assert torch.allclose(out[j * g : (j + 1) * g].double().cpu(), torch.softmax(s, 1) @ vals, atol=1e-4, rtol=0)
+        assert torch.allclose(lse[j * g : (j + 1) * g].double().cpu(), torch.logsumexp(s, 1), atol=1e-4, rtol=0)
